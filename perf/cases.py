@@ -152,10 +152,10 @@ def work(case):
 def tolerance(case):
     """Relative errors of another correct implementation at the same precision (see `exact`)."""
     if case["path"] == "solve":
-        return {"rel": 1e-9, "max": 1e-7}  # the same iterates: rounding times the condition of the basis
+        return {"rel": 1e-10, "max": 1e-8}  # the same iterates: rounding times the condition of the basis
     if case["precision"] == "double":
-        return {"rel": 2e-12, "max": 1e-9} if case["path"] == "gradient" else {"rel": 1e-13, "max": 1e-10}
-    return {"rel": 1e-6, "max": 1e-3}
+        return {"rel": 2e-12, "max": 1e-10} if case["path"] == "gradient" else {"rel": 1e-13, "max": 1e-11}
+    return {"rel": 1e-6, "max": 1e-4}
 
 
 # ------------------------------------------------------------------ meshes and inputs
