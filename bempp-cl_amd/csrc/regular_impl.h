@@ -853,10 +853,10 @@ __global__ __launch_bounds__(kRegThreads, (regular_waves<OP, MIXED, DUAL, SYM>()
     s1 = min(s1, s0 + kRegThreads);
     const int jf = s0 + tid;
     const bool valid = jf < s1;
-    // UPPER: a trial block that ends at or before the test tile holds no pair of the upper
-    // triangle (uniform per workgroup, before any barrier)
+    // UPPER: a trial block that ends before the test tile holds no pair of the upper triangle and
+    // no diagonal entry (uniform per workgroup, before any barrier)
     if constexpr (UPPER) {
-        if (s1 <= (int)blockIdx.y * TM + 1) return;
+        if (s1 <= (int)blockIdx.y * TM) return;
     }
 
     // stage the test elements at list positions [pos0, pos0 + n) into T_[0, n): all lanes share

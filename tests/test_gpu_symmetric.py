@@ -326,3 +326,32 @@ def test_dp0_upper_triangle_strided_output(level, precision_name, hip_available)
     assert bool((big[:, n:] == 7.0 + 3.0j).all())
     assert bool((ref == ref.T).all())
     assert bool((torch.diagonal(ref) == 0).all())
+
+
+@pytest.mark.parametrize("n", [1, 5, 17, 257, 5105])
+@pytest.mark.parametrize("precision", ["double", "single"])
+def test_dp0_upper_triangle_writes_every_entry(n, precision, default_parameters, hip_available):
+    """The upper-triangle pass overwrites its output: a matrix full of NaN becomes the ordered pass's
+    matrix, also where the last test tile holds only the last element (n = 1 modulo the tile's 4 or
+    16 elements), whose one entry on the diagonal no pair of the upper triangle stores."""
+    import torch
+
+    from bempp_amd.api import function_space
+    from bempp_amd.api.grid.shapes import icosphere
+    from bempp_amd.api.operators.boundary.laplace import single_layer
+    from bempp_amd.core import hip_backend as hb
+    from bempp_amd.core.dense_assembler import hip_dense_assemble, use_upper_triangle
+
+    space = function_space(icosphere(4 if n > 1280 else 3), "DP", 0, support_elements=np.arange(n))
+    assert use_upper_triangle(space, space, "laplace_single_layer")
+    descriptor = single_layer(space, space, space, parameters=default_parameters, precision=precision).descriptor
+    out = torch.full((n, n), float("nan"), dtype=torch.float64 if precision == "double" else torch.float32,
+                     device=hb.device())
+    hip_dense_assemble(space, space, default_parameters, descriptor, out=out, accumulate=False)
+    default_parameters.hip.symmetric = False
+    try:
+        ref = hip_dense_assemble(space, space, default_parameters, descriptor)
+    finally:
+        default_parameters.hip.symmetric = True
+    # the same sums in another order: rounding of the FP64 (FP32) values
+    assert rel(out, ref) < (1e-13 if precision == "double" else 1e-6)
