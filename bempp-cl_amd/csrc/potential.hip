@@ -553,23 +553,32 @@ __global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_efie(const P
 }
 
 // MIXED scalar potentials (Laplace and Helmholtz single and double layer). The sources of a tile
-// of 256 are staged once as FP32 records relative to the tile's reference source c:
+// of 256 are staged once as FP32 records relative to the reference source c (the middle one) of
+// their group of GS:
 //   u = c - y, |u|^2, the weights c_j / (4 pi) and, for the double layer, n_y and u.n_y,
-// read by every lane as LDS broadcasts. Per (target, tile) the FP64 part forms v = x - c,
+// read by every lane as LDS broadcasts. Per (target, group) the FP64 part forms v = x - c,
 // r0^2 = |v|^2, r0 and e^{i k r0}; per source only
 //   t = r^2 - r0^2 = 2 v.u + |u|^2,  r = sqrt(r0^2 + t),  k (r - r0) / 2 pi = t / ((r + r0) K)
 // (K = 2 pi / k) are needed in FP32, with the hardware rsq, rcp, sin and cos (revolutions). DAMP:
-// complex wavenumber, e^{-Im(k) (r - r0)} per source (exp2), e^{-Im(k) r0} per tile.
+// complex wavenumber, e^{-Im(k) (r - r0)} per source (exp2), e^{-Im(k) r0} per group.
+// GS: the radius of a group decides how many (target, group) pairs take the FP64 path and how large
+// k (r - r0) gets; the FP64 part costs about 70 instructions a group and target. 20,480 triangles,
+// 16,384 targets 0.5 to 2 off the surface (whole pass): one reference per tile of 256 7.3 ms
+// (4.5 ms by rsqrt_t alone), groups of 64 2.31, of 32 1.62 ms; with the elements along a space-filling
+// curve (hip_backend.potential_space) 1.63, 1.34 and 1.28 ms, errors 2.5e-7, 1.2e-7 and 8.4e-8. The
+// inner loop is bound by its 17.5 instructions, 4 of them transcendental.
 template <int OP, bool DAMP>
 __global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_scalar(const PotArgs a) {
+    constexpr int GS = 32;
+    constexpr int NG = kPotTile / GS;
     constexpr bool HELM = OP == kHelmholtzSL || OP == kHelmholtzDL;
     constexpr bool DL = OP == kLaplaceDL || OP == kHelmholtzDL;
     static_assert(!DAMP || HELM, "only Helmholtz wavenumbers are complex");
     __shared__ float4 shu[kPotTile];           // u, |u|^2
     __shared__ float4 shw[kPotTile];           // Re c / 4 pi, Im c / 4 pi, u.n_y, -
     __shared__ float4 shn[DL ? kPotTile : 1];  // n_y, -
-    __shared__ double sc[3];
-    __shared__ float srad2[kPotThreads / 64];  // per wave: max |u|^2 of its staged sources
+    __shared__ double sc[NG][3];
+    __shared__ float srad2[NG];  // max |u|^2 of the group's sources
     const int m = blockIdx.x * kPotThreads + threadIdx.x;
     const int chunk = blockIdx.y;
     const int s0 = chunk * a.chunk_len;
@@ -590,12 +599,12 @@ __global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_scalar(const
         const int nt = min(kPotTile, s1 - t0);
         __syncthreads();
         {
-            const int cidx = t0 + min(kPotTile / 2, nt - 1);  // reference: the tile's middle source
+            const int j = threadIdx.x, g = j / GS, s = t0 + j;
+            const int cidx = t0 + min(g * GS + GS / 2, nt - 1);
             double c[3];
             for (int d = 0; d < 3; ++d) c[d] = a.src[(int64_t)d * P + cidx];
-            if (threadIdx.x == 0)
-                for (int d = 0; d < 3; ++d) sc[d] = c[d];
-            const int j = threadIdx.x, s = t0 + j;
+            if (j % GS == 0)
+                for (int d = 0; d < 3; ++d) sc[g][d] = c[d];
             float4 U = make_float4(0.f, 0.f, 0.f, 0.f), W = make_float4(0.f, 0.f, 0.f, 0.f);
             float4 N = make_float4(0.f, 0.f, 0.f, 0.f);
             if (j < nt) {
@@ -615,91 +624,89 @@ __global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_scalar(const
             if constexpr (DL) shn[j] = N;
             float w2 = U.w;
 #pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) w2 = fmaxf(w2, __shfl_xor(w2, off, 64));
-            if ((j & 63) == 0) srad2[j >> 6] = w2;
+            for (int off = GS / 2; off >= 1; off >>= 1) w2 = fmaxf(w2, __shfl_xor(w2, off, 64));
+            if (j % GS == 0) srad2[g] = w2;
         }
         __syncthreads();
-        // per (target, tile): FP64 reference distance and phase
-        const double v0d = x0 - sc[0], v1d = x1 - sc[1], v2d = x2 - sc[2];
-        const double r0sq_d = v0d * v0d + v1d * v1d + v2d * v2d;
-        {
-            // targets close to the tile's sources: this tile in FP64 for the whole wave
-            float R2 = srad2[0];
-#pragma unroll
-            for (int w = 1; w < kPotThreads / 64; ++w) R2 = fmaxf(R2, srad2[w]);
-            if (__any(m < a.npts && r0sq_d < kNearTileFactor * kNearTileFactor * (double)R2 * (1.0 + 1e-6))) {
-                sources_fp64_near<OP, 1>(a, t0, t0 + nt, x0, x1, x2, 0.0, 0.0, &accr, &acci);
+        for (int g = 0; g < NG && g * GS < nt; ++g) {
+            const int j0 = g * GS, j1 = min(j0 + GS, nt);
+            // per (target, group): FP64 reference distance and phase
+            const double v0d = x0 - sc[g][0], v1d = x1 - sc[g][1], v2d = x2 - sc[g][2];
+            const double r0sq_d = v0d * v0d + v1d * v1d + v2d * v2d;
+            // targets close to the group's sources: the group in FP64 for the whole wave
+            if (__any(m < a.npts && r0sq_d < kNearTileFactor * kNearTileFactor * (double)srad2[g] * (1.0 + 1e-6))) {
+                sources_fp64_near<OP, 1>(a, t0 + j0, t0 + j1, x0, x1, x2, 0.0, 0.0, &accr, &acci);
                 continue;
             }
-        }
-        const double r0d = sqrt(r0sq_d);
-        const float tv0 = (float)(2.0 * v0d), tv1 = (float)(2.0 * v1d), tv2 = (float)(2.0 * v2d);
-        const float v0 = (float)v0d, v1 = (float)v1d, v2 = (float)v2d;
-        const float r0sq = (float)r0sq_d, r0 = (float)r0d;
-        const float r0k = r0 * kinv;
-        float Ar = 0.f, Ai = 0.f;
+            const double r0d = r0sq_d * rsqrt_t(r0sq_d);
+            const float tv0 = (float)(2.0 * v0d), tv1 = (float)(2.0 * v1d), tv2 = (float)(2.0 * v2d);
+            const float v0 = (float)v0d, v1 = (float)v1d, v2 = (float)v2d;
+            const float r0sq = (float)r0sq_d, r0 = (float)r0d;
+            const float r0k = r0 * kinv;
+            float Ar = 0.f, Ai = 0.f;
 #pragma unroll 4
-        for (int j = 0; j < nt; ++j) {
-            const float4 U = shu[j];
-            const float4 W = shw[j];
-            const float tt = tv0 * U.x + (tv1 * U.y + (tv2 * U.z + U.w));  // r^2 - r0^2
-            const float r2 = r0sq + tt;
-            const float rinv = __builtin_amdgcn_rsqf(r2);
-            float er = rinv, ei = 0.f;  // e^{ik(r - r0)} / r (Laplace: 1 / r)
-            float r = 0.f;
-            if constexpr (HELM) {
-                r = r2 * rinv;
-                float ph, amp = rinv;
-                if constexpr (DAMP) {
-                    const float delta = tt * __builtin_amdgcn_rcpf(r + r0);
-                    ph = kr_rev * delta;
-                    amp *= __builtin_amdgcn_exp2f(-ki_log2e * delta);
-                } else {
-                    ph = tt * __builtin_amdgcn_rcpf(r * kinv + r0k);
-                }
-                const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
-                if constexpr (!DL) {
-                    // single layer: the weight times e^{ik(r - r0)} first, then one FMA by the amplitude
-                    Ar += amp * (cs * W.x - sn * W.y);
-                    Ai += amp * (cs * W.y + sn * W.x);
-                    continue;
-                }
-                er = cs * amp;
-                ei = sn * amp;
-            }
-            if constexpr (DL) {
-                // (i k r - 1) (y - x).n_y / r^2 with y - x = -(v + u)
-                const float4 N = shn[j];
-                const float dot = -(v0 * N.x + (v1 * N.y + (v2 * N.z + W.z)));
-                const float f = dot * rinv * rinv;
+            for (int j = j0; j < j1; ++j) {
+                const float4 U = shu[j];
+                const float4 W = shw[j];
+                const float tt = tv0 * U.x + (tv1 * U.y + (tv2 * U.z + U.w));  // r^2 - r0^2
+                const float r2 = r0sq + tt;
+                const float rinv = __builtin_amdgcn_rsqf(r2);
+                float er = rinv, ei = 0.f;  // e^{ik(r - r0)} / r (Laplace: 1 / r)
+                float r = 0.f;
                 if constexpr (HELM) {
-                    const float ar = DAMP ? -1.f - ki_f * r : -1.f, ai = kr_f * r;
-                    const float pr = (ar * er - ai * ei) * f, pi = (ar * ei + ai * er) * f;
-                    er = pr;
-                    ei = pi;
+                    r = r2 * rinv;
+                    float ph, amp = rinv;
+                    if constexpr (DAMP) {
+                        const float delta = tt * __builtin_amdgcn_rcpf(r + r0);
+                        ph = kr_rev * delta;
+                        amp *= __builtin_amdgcn_exp2f(-ki_log2e * delta);
+                    } else {
+                        ph = tt * __builtin_amdgcn_rcpf(r * kinv + r0k);
+                    }
+                    const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
+                    if constexpr (!DL) {
+                        // single layer: the weight times e^{ik(r - r0)} first, then one FMA by the amplitude
+                        Ar += amp * (cs * W.x - sn * W.y);
+                        Ai += amp * (cs * W.y + sn * W.x);
+                        continue;
+                    }
+                    er = cs * amp;
+                    ei = sn * amp;
+                }
+                if constexpr (DL) {
+                    // (i k r - 1) (y - x).n_y / r^2 with y - x = -(v + u)
+                    const float4 N = shn[j];
+                    const float dot = -(v0 * N.x + (v1 * N.y + (v2 * N.z + W.z)));
+                    const float f = dot * rinv * rinv;
+                    if constexpr (HELM) {
+                        const float ar = DAMP ? -1.f - ki_f * r : -1.f, ai = kr_f * r;
+                        const float pr = (ar * er - ai * ei) * f, pi = (ar * ei + ai * er) * f;
+                        er = pr;
+                        ei = pi;
+                    } else {
+                        er = -er * f;
+                    }
+                }
+                if constexpr (HELM) {
+                    Ar += er * W.x - ei * W.y;
+                    Ai += er * W.y + ei * W.x;
                 } else {
-                    er = -er * f;
+                    Ar += er * W.x;
+                    Ai += er * W.y;
                 }
             }
+            // multiply the group's sum by e^{i k r0} (e^{-Im(k) r0}) in FP64
+            double pr = 1.0, pi = 0.0;
             if constexpr (HELM) {
-                Ar += er * W.x - ei * W.y;
-                Ai += er * W.y + ei * W.x;
-            } else {
-                Ar += er * W.x;
-                Ai += er * W.y;
+                double sn, cs;
+                sincos_fast(a.kr * r0d, &sn, &cs);
+                const double damp0 = DAMP ? exp(-a.ki * r0d) : 1.0;
+                pr = cs * damp0;
+                pi = sn * damp0;
             }
+            accr += pr * Ar - pi * Ai;
+            acci += pr * Ai + pi * Ar;
         }
-        // multiply the tile sum by e^{i k r0} (e^{-Im(k) r0}) in FP64
-        double pr = 1.0, pi = 0.0;
-        if constexpr (HELM) {
-            double sn, cs;
-            sincos_fast(a.kr * r0d, &sn, &cs);
-            const double damp0 = DAMP ? exp(-a.ki * r0d) : 1.0;
-            pr = cs * damp0;
-            pi = sn * damp0;
-        }
-        accr += pr * Ar - pi * Ai;
-        acci += pr * Ai + pi * Ar;
     }
     if (m < a.npts) {
         double *p = a.partial + 2 * ((int64_t)chunk * a.npts + m);
@@ -1048,15 +1055,36 @@ __global__ __launch_bounds__(kPotThreads) void far_field_eval_mixed(const PotArg
     }
 }
 
+// out[i] = sum of the chunk partials. A workgroup takes kRedOutputs consecutive outputs; 256 /
+// kRedOutputs lanes share one and add every (256 / kRedOutputs)-th chunk, so that few targets with
+// many chunks (1,024 targets, 120 chunks: a serial chain of 120 loads in four workgroups before,
+// 36 us) still keep the memory system busy. The order of the sums is fixed.
+constexpr int kRedOutputs = 32;
+
 template <typename OutT>
-__global__ void potential_reduce_kernel(const PotArgs a, int kd) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= kd * a.npts) return;
+__global__ __launch_bounds__(256) void potential_reduce_kernel(const PotArgs a, int kd) {
+    constexpr int NG = 256 / kRedOutputs;
+    __shared__ double2 part[NG][kRedOutputs];
+    const int c = threadIdx.x % kRedOutputs, g = threadIdx.x / kRedOutputs;
+    const int i = blockIdx.x * kRedOutputs + c;
+    const int64_t n = (int64_t)kd * a.npts;
     double sr = 0, si = 0;
-    for (int c = 0; c < a.nchunk; ++c) {
-        const double *p = a.partial + 2 * ((int64_t)c * kd * a.npts + i);
-        sr += p[0];
-        si += p[1];
+    if (i < n) {
+        const double2 *p = reinterpret_cast<const double2 *>(a.partial) + i;
+#pragma unroll 4
+        for (int ch = g; ch < a.nchunk; ch += NG) {
+            const double2 v = p[ch * n];
+            sr += v.x;
+            si += v.y;
+        }
+    }
+    part[g][c] = make_double2(sr, si);
+    __syncthreads();
+    if (g != 0 || i >= n) return;
+#pragma unroll
+    for (int k = 1; k < NG; ++k) {
+        sr += part[k][c].x;
+        si += part[k][c].y;
     }
     OutT *o = reinterpret_cast<OutT *>(a.out);
     o[2 * (int64_t)i] = (OutT)sr;
@@ -1132,9 +1160,9 @@ static int run_potential(PotArgs &a, int precision, int out_dtype, hipStream_t s
     }
     int n = kd * a.npts;
     if (out_dtype == BEM_C128)
-        hipLaunchKernelGGL((potential_reduce_kernel<double>), dim3((n + 255) / 256), dim3(256), 0, s, a, kd);
+        hipLaunchKernelGGL((potential_reduce_kernel<double>), dim3((n + kRedOutputs - 1) / kRedOutputs), dim3(256), 0, s, a, kd);
     else
-        hipLaunchKernelGGL((potential_reduce_kernel<float>), dim3((n + 255) / 256), dim3(256), 0, s, a, kd);
+        hipLaunchKernelGGL((potential_reduce_kernel<float>), dim3((n + kRedOutputs - 1) / kRedOutputs), dim3(256), 0, s, a, kd);
     return check_launch("potential_reduce_kernel");
 }
 
