@@ -74,7 +74,12 @@ class SingularRule(object):
         pairs[i1:, 3] = vertex_offsets[va[3]]
         pairs[i1:, 4] = nco + ned
         pairs[i1:, 5] = nve
-        self.pairs = pairs
+        # pairs of one rule (kind and local vertices) together, the kinds in order: the device kernel
+        # reads a rule's points once for 64 consecutive pairs
+        rules = _np.zeros(n, dtype=_np.int16)
+        rules[i0:i1] = 1 + 6 * _EDGE_OFFSET_INDEX[ea[2], ea[3]] + _EDGE_OFFSET_INDEX[ea[4], ea[5]]
+        rules[i1:] = 37 + 3 * va[2] + va[3]
+        self.pairs = pairs[_np.argsort(rules, kind="stable")]
         self.counts = {"coincident": i0, "edge_adjacent": i1 - i0, "vertex_adjacent": n - i1}
 
     @property

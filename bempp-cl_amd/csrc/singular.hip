@@ -1,16 +1,19 @@
-// Singular (Sauter-Schwab) pairs, FP64, for gfx950.
+// Singular (Sauter-Schwab) pairs, FP64, for gfx950: (test element, trial element) pairs that share a
+// vertex, an edge or the whole triangle (bempp_cl/core/numba_kernels.py:1471-1526 scalar, 1973-2061
+// EFIE), with 512 (vertex), 1280 (edge) or 1536 (coincident) Duffy points per pair at order 4.
 //
-// A group of G lanes (8, or 32 for small launches) per (test element, trial element) pair that
-// shares a vertex, an edge or the whole triangle (bempp_cl/core/numba_kernels.py:1471-1526 scalar,
-// 1973-2061 EFIE); a wavefront takes 64 / G consecutive pairs, which are mostly of one kind (the
-// pair table lists coincident, then edge, then vertex pairs). The pair's 512..1536 Duffy
-// points are strided over the group's lanes; each lane accumulates the 3x3 moment block
-// S[a][b] = sum_k G_k w_k u_a(xi_k) u_b(eta_k) with u = (1, xi_0, xi_1), the block is summed
-// over the group with log2(G) shuffle steps (a reduction over the whole wavefront would cost 6
-// steps for one pair), scaled by J_test J_trial and turned into the local matrix block exactly as
-// for regular pairs. The group's lanes add the multiplied entries to the dense output with
-// hardware atomics, which replaces the reference's host-side np.add.at scatter
+// A workgroup of W waves takes 64 / G consecutive pairs; in every wave G lanes share a pair and the
+// pair's points are split over the W G lanes. The pair table lists the pairs of one rule (kind and
+// local vertices) together, so a wave's pairs share the points: the wave stages its part of them in LDS
+// with coalesced loads and reads them as broadcasts (a wave whose pairs have several rules runs them one
+// after the other). Each lane accumulates the moment block S[a][b] = sum_k G_k w_k u_a(xi_k) u_b(eta_k),
+// u = (1, xi_0, xi_1), of its points; the partial blocks are summed by shuffles and through LDS, scaled
+// by J_test J_trial and turned into the local matrix block exactly as for regular pairs. The entries are
+// added to the dense output with hardware atomics, real and imaginary part on neighbouring lanes (one
+// memory-side request), which replaces the reference's host-side np.add.at scatter
 // (bempp_cl/core/dense_assembler.py:78-98).
+// Bound by FP64 arithmetic: 68 instructions a point for a complex single layer on P1, 23 for the
+// Laplace one on DP0.
 #include "bem_device.h"
 #include "bem_internal.h"
 
@@ -27,152 +30,245 @@ struct SingularArgs {
     int64_t ld;
 };
 
-// lanes per pair: 8, or 32 for launches of fewer than kSingSmallPairs pairs, whose 8-lane groups
-// would give fewer than four waves per SIMD on 256 CUs (1,280 triangles: 16,580 pairs, 2,073 waves;
-// there 32 lanes per pair take 0.033 instead of 0.048 ms, while at 66,500 EFIE pairs they are 25 %
-// slower than 8)
-constexpr int kSingGroup = 8;
-constexpr int kSingGroupSmall = 32;
-constexpr int kSingSmallPairs = 32768;
-
-template <int G, typename T>
-__device__ __forceinline__ T group_sum(T v) {
-#pragma unroll
-    for (int off = G / 2; off >= 1; off >>= 1) v += __shfl_xor(v, off, G);
-    return v;
-}
+// LDS of one workgroup: the staged points, then the partial moments and the local blocks
+template <int NV, int W, int G>
+union SingularShared {
+    static constexpr int kChunk = G == 1 ? 64 : 96;  // points a wave stages at a time
+    double2 points[W][kChunk][3];                     // (xi_0, xi_1), (eta_0, eta_1), (w, -)
+    double moments[W][NV][64 / G];
+};
 
 // DUAL: OP is a single layer; the double layer of the same family (sharing r and e^{ikr} at
 // every point) goes to a.out2.
-template <int OP, int NTS, int NSS, typename OutT, bool DUAL = false, int G = kSingGroup>
-__global__ __launch_bounds__(256) void singular_kernel(const SingularArgs a) {
+template <int OP, int NTS, int NSS, typename OutT, bool DUAL, int W, int G>
+__global__ __launch_bounds__(64 * W, W == 4 && !(DUAL && NTS * NSS == 9) ? 3 : 2) void singular_kernel(const SingularArgs a) {
     constexpr bool CPLX = OpTraits<OP>::is_complex;
-    const int lane = threadIdx.x & (G - 1);  // lane within the pair's group
-    const int pair = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G);
-    // the group's lanes share the pair, so whole groups leave together and the group shuffles
-    // below only read lanes of groups that stay
-    if (pair >= a.n_pairs) return;
-    const int32_t *pd = a.pairs + 6 * (int64_t)pair;
+    constexpr int NC = CPLX ? 2 : 1, NB = NTS * NSS, NV = NB * NC, NOPS = DUAL ? 2 : 1;
+    constexpr int PP = 64 / G;  // pairs per workgroup
+    using Shared = SingularShared<NV, W, G>;
+    __shared__ Shared sh;
+    __shared__ int32_t rows[NTS][PP], cols[NSS][PP];
+    __shared__ double mult[NTS + NSS][PP];
+    const int lane = threadIdx.x & 63, p = lane % PP, sub = lane / PP;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int first = blockIdx.x * PP;
+    const bool active = first + p < a.n_pairs;
+    const int32_t *pd = a.pairs + 6 * (int64_t)(active ? first + p : first);
     const int e = pd[0], f = pd[1], toff = pd[2], soff = pd[3], woff = pd[4], np = pd[5];
-    const double *gt = a.test.geom + (int64_t)e * BEM_GEOM_STRIDE;
-    const double *gf = a.trial.geom + (int64_t)f * BEM_GEOM_STRIDE;
-    double tnm = a.test.nmult ? (double)a.test.nmult[e] : 1.0;
-    double snm = a.trial.nmult ? (double)a.trial.nmult[f] : 1.0;
-    double nx[3] = {gt[9] * tnm, gt[10] * tnm, gt[11] * tnm};
-    double ny[3] = {gf[9] * snm, gf[10] * snm, gf[11] * snm};
-
-    double Sr[NTS][NSS], Si[NTS][NSS], Sr2[DUAL ? NTS : 1][DUAL ? NSS : 1], Si2[DUAL ? NTS : 1][DUAL ? NSS : 1];
+    const double tnm = a.test.nmult ? (double)a.test.nmult[e] : 1.0;
+    const double snm = a.trial.nmult ? (double)a.trial.nmult[f] : 1.0;
+    // dofs and multipliers of the scatter, loaded together with the geometry
+    if (wave == 0 && sub == 0) {
 #pragma unroll
-    for (int i = 0; i < NTS; ++i)
+        for (int i = 0; i < NTS; ++i) {
+            rows[i][p] = a.test.l2g[(int64_t)e * NTS + i];
+            mult[i][p] = a.test.mult[(int64_t)e * NTS + i];
+        }
 #pragma unroll
         for (int j = 0; j < NSS; ++j) {
-            Sr[i][j] = Si[i][j] = 0.0;
-            if constexpr (DUAL) Sr2[i][j] = Si2[i][j] = 0.0;
+            cols[j][p] = a.trial.l2g[(int64_t)f * NSS + j];
+            mult[NTS + j][p] = a.trial.mult[(int64_t)f * NSS + j];
         }
+    }
+    // the geometry rows in registers; y - x = c + e1_f eta_0 + e2_f eta_1 - e1_t xi_0 - e2_t xi_1
+    double gt[14], gf[14], c[3], nx[3], ny[3];
+#pragma unroll
+    for (int k = 0; k < 14; ++k) {
+        gt[k] = a.test.geom[(int64_t)e * BEM_GEOM_STRIDE + k];
+        gf[k] = a.trial.geom[(int64_t)f * BEM_GEOM_STRIDE + k];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        c[d] = gf[d] - gt[d];
+        nx[d] = gt[9 + d] * tnm;
+        ny[d] = gf[9 + d] * snm;
+    }
 
-    // every distance within the pair is at most diam_t + diam_f (triangles sharing a vertex), so a
-    // wave-uniform bound selects the phase mode: the series sin/cos without range reduction when
-    // k r <= 1, else (real wavenumbers) the branch-free reduction
-    auto points = [&](auto phase_tag) {
-        constexpr int PH = decltype(phase_tag)::value;
-        for (int k = lane; k < np; k += G) {
-            double xi0 = a.tpts[2 * (int64_t)(toff + k)], xi1 = a.tpts[2 * (int64_t)(toff + k) + 1];
-            double et0 = a.spts[2 * (int64_t)(soff + k)], et1 = a.spts[2 * (int64_t)(soff + k) + 1];
-            double w = a.wts[woff + k];
-            double dx = (gf[0] + gf[3] * et0 + gf[6] * et1) - (gt[0] + gt[3] * xi0 + gt[6] * xi1);
-            double dy = (gf[1] + gf[4] * et0 + gf[7] * et1) - (gt[1] + gt[4] * xi0 + gt[7] * xi1);
-            double dz = (gf[2] + gf[5] * et0 + gf[8] * et1) - (gt[2] + gt[5] * xi0 + gt[8] * xi1);
-            double r2 = dx * dx + dy * dy + dz * dz;
-            double gre, gim, g2re, g2im;
-            green2<green_op<OP>(), DUAL, double, PH>(dx, dy, dz, r2, nx, ny, a.kr, a.ki, gre, gim, g2re, g2im);
-            gre *= w;
-            gim *= w;
-            g2re *= w;
-            g2im *= w;
-            double ut[3] = {1.0, xi0, xi1}, us[3] = {1.0, et0, et1};
+    double S[NOPS][NC][NTS][NSS];
+#pragma unroll
+    for (int o = 0; o < NOPS; ++o)
+#pragma unroll
+        for (int z = 0; z < NC; ++z)
 #pragma unroll
             for (int i = 0; i < NTS; ++i)
 #pragma unroll
-                for (int j = 0; j < NSS; ++j) {
-                    double u = ut[i] * us[j];
-                    Sr[i][j] += gre * u;
-                    Si[i][j] += gim * u;
-                    if constexpr (DUAL) {
-                        Sr2[i][j] += g2re * u;
-                        Si2[i][j] += g2im * u;
-                    }
+                for (int j = 0; j < NSS; ++j) S[o][z][i][j] = 0.0;
+
+    auto points = [&](auto phase_tag) {
+        constexpr int PH = decltype(phase_tag)::value;
+        unsigned long long todo = __ballot(active);
+        while (todo) {
+            // the rule of the first pair left, and the lanes that share it
+            const int lead = __ffsll(todo) - 1;
+            const int to = __builtin_amdgcn_readlane(toff, lead), so = __builtin_amdgcn_readlane(soff, lead);
+            const int wo = __builtin_amdgcn_readlane(woff, lead), n = __builtin_amdgcn_readlane(np, lead);
+            const bool mine = active && toff == to && soff == so && woff == wo && np == n;
+            todo &= ~__ballot(mine);
+            const int per = (n + W - 1) / W, k0 = min(wave * per, n), k1 = min(k0 + per, n);
+            for (int kb = k0; kb < k1; kb += Shared::kChunk) {
+                const int count = min(Shared::kChunk, k1 - kb);
+                // the wave's own part of LDS: its accesses complete in order, no barrier
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                for (int k = lane; k < count; k += 64) {
+                    const int64_t kk = kb + k;
+                    sh.points[wave][k][0] = *reinterpret_cast<const double2 *>(a.tpts + 2 * (to + kk));
+                    sh.points[wave][k][1] = *reinterpret_cast<const double2 *>(a.spts + 2 * (so + kk));
+                    sh.points[wave][k][2].x = a.wts[wo + kk];
                 }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (!mine) continue;
+#pragma unroll 2
+                for (int k = sub; k < count; k += G) {
+                    const double2 px = sh.points[wave][k][0], py = sh.points[wave][k][1];
+                    const double xi0 = px.x, xi1 = px.y, et0 = py.x, et1 = py.y, w = sh.points[wave][k][2].x;
+                    double d[3];
+#pragma unroll
+                    for (int m = 0; m < 3; ++m)
+                        d[m] = fma(-gt[6 + m], xi1, fma(-gt[3 + m], xi0, fma(gf[6 + m], et1, fma(gf[3 + m], et0, c[m]))));
+                    const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+                    double g[2][2];
+                    green2<green_op<OP>(), DUAL, double, PH>(d[0], d[1], d[2], r2, nx, ny, a.kr, a.ki, g[0][0], g[0][1],
+                                                             g[1][0], g[1][1]);
+#pragma unroll
+                    for (int o = 0; o < NOPS; ++o)
+#pragma unroll
+                        for (int z = 0; z < NC; ++z) {
+                            const double t0 = g[o][z] * w;
+                            const double t[3] = {t0, t0 * et0, t0 * et1};
+#pragma unroll
+                            for (int j = 0; j < NSS; ++j) {
+                                S[o][z][0][j] += t[j];
+                                if constexpr (NTS == 3) {
+                                    S[o][z][1][j] = fma(t[j], xi0, S[o][z][1][j]);
+                                    S[o][z][2][j] = fma(t[j], xi1, S[o][z][2][j]);
+                                }
+                            }
+                        }
+                }
+            }
         }
     };
-    const double kd = fabs(a.kr) * (gt[13] + gf[13]);
-    if (kd <= 1.0 && a.ki == 0.0) points(std::integral_constant<int, kPhSmall | kPhReal>{});
-    else if (kd <= 1.0) points(std::integral_constant<int, kPhSmall>{});
-    else if (kd < 0x1p25 && a.ki == 0.0) points(std::integral_constant<int, kPhReduced | kPhReal>{});
-    else points(std::integral_constant<int, 0>{});
+    // every distance within a pair is at most diam_t + diam_f (triangles sharing a vertex), so a
+    // wave-uniform bound selects the phase mode: the series sin/cos without range reduction when
+    // k r <= 1, else the branch-free reduction
+    if constexpr (OpTraits<green_op<OP>()>::is_complex) {
+        const double kd = fabs(a.kr) * (gt[13] + gf[13]);
+        const bool small = __all(kd <= 1.0), reduced = __all(kd < 0x1p25), real = a.ki == 0.0;
+        if (small && real) points(std::integral_constant<int, kPhSmall | kPhReal>{});
+        else if (small) points(std::integral_constant<int, kPhSmall>{});
+        else if (reduced && real) points(std::integral_constant<int, kPhReduced | kPhReal>{});
+        else if (reduced) points(std::integral_constant<int, kPhReduced>{});
+        else points(std::integral_constant<int, 0>{});
+    } else {
+        points(std::integral_constant<int, 0>{});
+    }
+
+    // sums over the lanes of a pair
+#pragma unroll
+    for (int o = 0; o < NOPS; ++o)
+#pragma unroll
+        for (int z = 0; z < NC; ++z)
+#pragma unroll
+            for (int i = 0; i < NTS; ++i)
+#pragma unroll
+                for (int j = 0; j < NSS; ++j)
+#pragma unroll
+                    for (int off = 32; off >= PP; off >>= 1) S[o][z][i][j] += __shfl_xor(S[o][z][i][j], off, 64);
     const double jj = gt[12] * gf[12];
-    C2d S[NTS][NSS], S2[NTS][NSS];
 #pragma unroll
-    for (int i = 0; i < NTS; ++i)
+    for (int o = 0; o < NOPS; ++o) {
+        __syncthreads();  // the points (the previous operator's blocks) have been read
+        if (sub == 0) {
 #pragma unroll
-        for (int j = 0; j < NSS; ++j) {
-            S[i][j].re = group_sum<G>(Sr[i][j]) * jj;
-            S[i][j].im = CPLX ? group_sum<G>(Si[i][j]) * jj : 0.0;
-            if constexpr (DUAL) {
-                S2[i][j].re = group_sum<G>(Sr2[i][j]) * jj;
-                S2[i][j].im = CPLX ? group_sum<G>(Si2[i][j]) * jj : 0.0;
-            }
+            for (int z = 0; z < NC; ++z)
+#pragma unroll
+                for (int i = 0; i < NTS; ++i)
+#pragma unroll
+                    for (int j = 0; j < NSS; ++j) sh.moments[wave][(i * NSS + j) * NC + z][p] = S[o][z][i][j] * jj;
         }
-    // the group's lanes add entries l = lane, lane + G, ... (DUAL: l >= NTS*NSS are the double
-    // layer's)
-    const int nb = NTS * NSS;
-    for (int ll = lane; ll < (DUAL ? 2 * nb : nb); ll += G) {
-        const bool second = DUAL && ll >= nb;
-        const int l = second ? ll - nb : ll;
-        int i = l / NSS, j = l % NSS;
-        double m = a.test.mult[(int64_t)e * NTS + i] * a.trial.mult[(int64_t)f * NSS + j];
-        if (m != 0.0) {
-            C2d v;
-            if constexpr (DUAL) {
-                v = second ? local_value<OP + 1, NTS, NSS>(S2, i, j, gt, gf, a.kr, a.ki)
-                           : local_value<OP, NTS, NSS>(S, i, j, gt, gf, a.kr, a.ki);
-            } else {
-                v = local_value<OP, NTS, NSS>(S, i, j, gt, gf, a.kr, a.ki, tnm * snm);
+        __syncthreads();
+        // the sums over the waves: each thread its own values
+        for (int idx = threadIdx.x; idx < NV * PP; idx += 64 * W) {
+            double *m = &sh.moments[0][0][0] + idx;
+            double sum = m[0];
+#pragma unroll
+            for (int k = 1; k < W; ++k) sum += m[k * NV * PP];
+            m[0] = sum;
+        }
+        __syncthreads();
+        // the local blocks [pair][entry][re, im], in the memory of the second wave's partial sums
+        OutT *block = reinterpret_cast<OutT *>(&sh.moments[1][0][0]);
+        C2d M[NTS][NSS];
+#pragma unroll
+        for (int i = 0; i < NTS; ++i)
+#pragma unroll
+            for (int j = 0; j < NSS; ++j) {
+                M[i][j].re = sh.moments[0][(i * NSS + j) * NC][p];
+                M[i][j].im = CPLX ? sh.moments[0][(i * NSS + j) * NC + NC - 1][p] : 0.0;
             }
-            int row = a.test.l2g[(int64_t)e * NTS + i];
-            int col = a.trial.l2g[(int64_t)f * NSS + j];
-            OutT *o = reinterpret_cast<OutT *>(second ? a.out2 : a.out);
-            int64_t idx = (int64_t)row * a.ld + col;
-            if constexpr (CPLX) {
-                atomic_add(o + 2 * idx, (OutT)(v.re * m));
-                atomic_add(o + 2 * idx + 1, (OutT)(v.im * m));
-            } else {
-                atomic_add(o + idx, (OutT)(v.re * m));
+        // entry l is formed by wave l % W (lanes of sub 0)
+#pragma unroll
+        for (int l = 0; l < NB; ++l) {
+            if (l % W != wave || sub != 0) continue;
+            const int i = l / NSS, j = l % NSS;
+            const double m = mult[i][p] * mult[NTS + j][p];
+            C2d v = {0.0, 0.0};
+            if (m != 0.0) {
+                if constexpr (DUAL)
+                    v = o ? local_value<OP + 1, NTS, NSS>(M, i, j, gt, gf, a.kr, a.ki)
+                          : local_value<OP, NTS, NSS>(M, i, j, gt, gf, a.kr, a.ki);
+                else
+                    v = local_value<OP, NTS, NSS>(M, i, j, gt, gf, a.kr, a.ki, tnm * snm);
             }
+            OutT *dst = block + (p * NB + l) * NC;
+            dst[0] = (OutT)(v.re * m);
+            if constexpr (CPLX) dst[1] = (OutT)(v.im * m);
+        }
+        __syncthreads();
+        OutT *out = reinterpret_cast<OutT *>(o ? a.out2 : a.out);
+        const int count = min(PP, a.n_pairs - first) * NV;
+        for (int idx = threadIdx.x; idx < count; idx += 64 * W) {
+            const int q = idx / NV, l = (idx - q * NV) / NC;
+            const OutT v = block[idx];
+            const int64_t at = (int64_t)rows[l / NSS][q] * a.ld + cols[l % NSS][q];
+            if (v != (OutT)0) atomic_add(out + NC * at + idx % NC, v);
         }
     }
 }
 
-template <int OP, typename OutT, bool DUAL, int G>
-static int launch_sing_g(const SingularArgs &a, hipStream_t s) {
-    dim3 grid((unsigned)(((int64_t)a.n_pairs * G + 255) / 256));
+// Lanes of a wave per pair (G) and waves (W): the points of a pair are split W G ways. The coincident
+// pairs' lanes form the longest chain (1536 / (W G) points), a split costs the set-up of more workgroups.
+// Kernel times with (W, G) = (4, 1) / (4, 4) / (8, 2) / (8, 16), against lanes striding over a pair's
+// points with loads of their own before:
+//   266,000 pairs, Helmholtz single + double layer P1:   737 / 866 / 1006 us   (before 1117)
+//    66,500 pairs, electric field operator:              179 / 160 /  203 us   (305)
+//    43,900 pairs, Helmholtz double layer P1, FP64:      163 / 126 /  164 us   (207)
+//    16,600 pairs, Laplace DP0, FP64:                     62 /  27 /   31 us   (29)
+//     1,000 pairs, Laplace P1, FP64:                       - /  - /    - / 9 us (14)
+constexpr int kSingLargePairs = 131072, kSingSmallPairs = 4096;
+
+template <int OP, typename OutT, bool DUAL, int W, int G>
+static int launch_sing_split(const SingularArgs &a, hipStream_t s) {
+    constexpr int PP = 64 / G;
+    const dim3 grid((unsigned)(((int64_t)a.n_pairs + PP - 1) / PP)), threads(64 * W);
     if constexpr (OP == kMaxwellEFIE) {
-        hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, false, G>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, false, W, G>), grid, threads, 0, s, a);
     } else if constexpr (is_hypersingular<OP>()) {
         if (nshape_of(a.test.shape) != 3 || nshape_of(a.trial.shape) != 3) {
             set_error("hypersingular operators need P1 shape functions on both sides");
             return BEM_ERR_INVALID_ARGUMENT;
         }
-        hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, false, G>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, false, W, G>), grid, threads, 0, s, a);
     } else {
         int nt = nshape_of(a.test.shape), ns = nshape_of(a.trial.shape);
         if (nt == 1 && ns == 1)
-            hipLaunchKernelGGL((singular_kernel<OP, 1, 1, OutT, DUAL, G>), grid, dim3(256), 0, s, a);
+            hipLaunchKernelGGL((singular_kernel<OP, 1, 1, OutT, DUAL, W, G>), grid, threads, 0, s, a);
         else if (nt == 1 && ns == 3)
-            hipLaunchKernelGGL((singular_kernel<OP, 1, 3, OutT, DUAL, G>), grid, dim3(256), 0, s, a);
+            hipLaunchKernelGGL((singular_kernel<OP, 1, 3, OutT, DUAL, W, G>), grid, threads, 0, s, a);
         else if (nt == 3 && ns == 1)
-            hipLaunchKernelGGL((singular_kernel<OP, 3, 1, OutT, DUAL, G>), grid, dim3(256), 0, s, a);
+            hipLaunchKernelGGL((singular_kernel<OP, 3, 1, OutT, DUAL, W, G>), grid, threads, 0, s, a);
         else
-            hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, DUAL, G>), grid, dim3(256), 0, s, a);
+            hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, DUAL, W, G>), grid, threads, 0, s, a);
     }
     return check_launch("singular_kernel");
 }
@@ -180,8 +276,9 @@ static int launch_sing_g(const SingularArgs &a, hipStream_t s) {
 template <int OP, typename OutT, bool DUAL>
 static int launch_sing(const SingularArgs &a, hipStream_t s) {
     if (a.n_pairs == 0) return BEM_OK;
-    if (a.n_pairs < kSingSmallPairs) return launch_sing_g<OP, OutT, DUAL, kSingGroupSmall>(a, s);
-    return launch_sing_g<OP, OutT, DUAL, kSingGroup>(a, s);
+    if (a.n_pairs >= kSingLargePairs) return launch_sing_split<OP, OutT, DUAL, 4, 1>(a, s);
+    if (a.n_pairs >= kSingSmallPairs) return launch_sing_split<OP, OutT, DUAL, 4, 4>(a, s);
+    return launch_sing_split<OP, OutT, DUAL, 8, 16>(a, s);
 }
 
 template <int OP, bool DUAL = false>

@@ -1,0 +1,42 @@
+"""The singular kernel's grouping of pairs: workgroups take consecutive pairs of the table, a wave's pairs
+may follow several rules, and the split of a pair's points depends on the number of pairs."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# 3, 63 and 4,095 pairs: the smallest launches and their last workgroup; 4,096 to 15,777: the split of
+# medium launches (16 pairs per workgroup, remainder 1); 131,073: one lane per pair (64 pairs, remainder 1)
+@pytest.mark.parametrize("op,space,k", [("laplace_single_layer", "P1", 0.0), ("helmholtz_double_layer", "DP0", 2.0),
+                                        ("helmholtz_hypersingular", "P1", 2.0 + 0.3j),
+                                        ("maxwell_electric_field", "RWG", 3.0)])
+@pytest.mark.parametrize("count", [3, 63, 4095, 4096, 15777, 131073])
+def test_singular_pairs_in_any_order(op, space, k, count, hip_available):
+    """A table of `count` pairs gives the same sum whether the pairs of one rule stand together (every
+    wave reads one set of points) or the table is shuffled (every wave runs many rules)."""
+    import torch
+
+    from bempp_amd.api import function_space
+    from bempp_amd.api.grid.shapes import icosphere
+    from bempp_amd.core import hip_backend as hb
+    from bempp_amd.core.singular_assembler import singular_rule
+
+    grid = icosphere(3 if count <= 15777 else 5)
+    sp = function_space(grid, *{"P1": ("P", 1), "DP0": ("DP", 0), "RWG": ("RWG", 0)}[space])
+    rule = singular_rule(grid, 2, sp.support, sp.support)
+    rng = np.random.default_rng(count)
+    chosen = np.sort(rng.permutation(len(rule.host.pairs))[:count])
+    complex_op = not op.startswith("laplace")
+    results = []
+    for order in (chosen, rng.permutation(chosen)):
+        pairs = torch.from_numpy(np.ascontiguousarray(rule.host.pairs[order])).to(hb.device())
+        out = torch.zeros((sp.global_dof_count,) * 2, dtype=torch.complex128 if complex_op else torch.float64,
+                          device=hb.device())
+        hb.singular_assemble(op, hb.device_space(sp), hb.device_space(sp), pairs, rule.test_points, rule.trial_points,
+                             rule.weights, k, out)
+        results.append(out)
+    assert torch.linalg.norm(results[0]) > 0
+    # the same FP64 terms in another order of the atomics: a few roundings per entry
+    assert torch.linalg.norm(results[0] - results[1]) < 1e-14 * torch.linalg.norm(results[0])
