@@ -94,6 +94,30 @@ __device__ __forceinline__ void sincos_small(double x, double *s, double *c) {
     *c = 1.0 - x2 * pc;
 }
 
+// e^x of |x| <= 1 from its Taylor series through x^18 (remainder below e / 19! = 2.3e-17), with no
+// range reduction.
+__device__ __forceinline__ double exp_small(double x) {
+    double p = 1.0 / 6402373705728000.0;  // 1/18!
+    p = fma(p, x, 1.0 / 355687428096000.0);
+    p = fma(p, x, 1.0 / 20922789888000.0);
+    p = fma(p, x, 1.0 / 1307674368000.0);
+    p = fma(p, x, 1.0 / 87178291200.0);
+    p = fma(p, x, 1.0 / 6227020800.0);
+    p = fma(p, x, 1.0 / 479001600.0);
+    p = fma(p, x, 1.0 / 39916800.0);
+    p = fma(p, x, 1.0 / 3628800.0);
+    p = fma(p, x, 1.0 / 362880.0);
+    p = fma(p, x, 1.0 / 40320.0);
+    p = fma(p, x, 1.0 / 5040.0);
+    p = fma(p, x, 1.0 / 720.0);
+    p = fma(p, x, 1.0 / 120.0);
+    p = fma(p, x, 1.0 / 24.0);
+    p = fma(p, x, 1.0 / 6.0);
+    p = fma(p, x, 0.5);
+    p = fma(p, x, 1.0);
+    return fma(p, x, 1.0);
+}
+
 // sin and cos of x (radians), |x| < 2^26: x = n pi / 2 + y with n = rint(2 x / pi) and |y| <= pi / 4
 // from a three-part Cody-Waite subtraction (pi / 2 split into three doubles; FMA keeps each step to
 // one rounding), the Taylor polynomials of sin y through y^15 and of cos y through y^16 (remainders
@@ -146,8 +170,9 @@ __device__ __forceinline__ void sincos_fast(double x, double *sp, double *cp) {
 // guarantees |k r| <= 1 (Taylor series, sincos_small); kPhReduced, the caller guarantees
 // |k r| < 2^26 (sincos_reduced, no large-argument branch); otherwise sincos_fast. kPhReal may be
 // or-ed in when the wavenumber is real: the e^{-Im(k) r} factor and its branch are left out.
-// kPhShift: the Green's functions return e^{-i ph0} times their value, with the phase k r - ph0
-// (|k r - ph0| <= 1 guaranteed by the caller) from sincos_small; the caller multiplies by e^{i ph0}.
+// kPhShift: the Green's functions return e^{-i ph0} e^{dm0} times their value, with the phase
+// Re(k) r - ph0 and the damping exponent dm0 - Im(k) r (both at most 1 in modulus, guaranteed by the
+// caller) from sincos_small and exp_small; the caller multiplies by e^{i ph0} e^{-dm0}.
 constexpr int kPhSmall = 1, kPhReduced = 2, kPhReal = 4, kPhShift = 8;
 
 // Wave-uniform: the wavenumber is real and |k r| < 2^25 on every point pair of every active lane's
@@ -174,11 +199,19 @@ __device__ __forceinline__ void phase_t(T kr, T r, T ph0, T *s, T *c) {
 __device__ __forceinline__ double exp_t(double x) { return exp(x); }
 __device__ __forceinline__ float exp_t(float x) { return __expf(x); }
 
+// the damping factor e^{-Im(k) r} (e^{dm0 - Im(k) r} with kPhShift); 1 for a real wavenumber
+template <int PH, typename T>
+__device__ __forceinline__ void damp_t(T ki, T r, T dm0, T &g) {
+    if constexpr (PH & kPhReal) return;
+    else if constexpr ((PH & kPhShift) && sizeof(T) == 8) g *= exp_small(fma(-ki, r, dm0));
+    else if (ki != T(0)) g *= exp_t(-ki * r);
+}
+
 // Green's function of operator OP for d = y - x, r2 = |d|^2.
 // nx: test normal (ADL), ny: trial normal (DL). Returns (re, im).
 template <int OP, typename T, int PH = 0>
 __device__ __forceinline__ void green(T dx, T dy, T dz, T r2, const T *nx, const T *ny, T kr, T ki, T &gre, T &gim,
-                                      T ph0 = T(0)) {
+                                      T ph0 = T(0), T dm0 = T(0)) {
     T rinv = rsqrt_t(r2);
     if constexpr (OP == kLaplaceSL) {
         gre = T(kInv4Pi) * rinv;
@@ -196,7 +229,7 @@ __device__ __forceinline__ void green(T dx, T dy, T dz, T r2, const T *nx, const
         T s, c;
         phase_t<PH>(kr, r, ph0, &s, &c);
         T g = T(kInv4Pi) * rinv;
-        if constexpr (!(PH & kPhReal)) { if (ki != T(0)) g *= exp_t(-ki * r); }
+        damp_t<PH>(ki, r, dm0, g);
         gre = c * g;
         gim = s * g;
     } else {  // Helmholtz DL / ADL
@@ -207,7 +240,7 @@ __device__ __forceinline__ void green(T dx, T dy, T dz, T r2, const T *nx, const
         T s, c;
         phase_t<PH>(kr, r, ph0, &s, &c);
         T g = T(kInv4Pi) * dot * rinv * rinv * rinv;
-        if constexpr (!(PH & kPhReal)) { if (ki != T(0)) g *= exp_t(-ki * r); }
+        damp_t<PH>(ki, r, dm0, g);
         T fr = c * g, fi = s * g;
         T a = T(-1) - ki * r, b = kr * r;  // i k r - 1 = a + i b
         gre = a * fr - b * fi;
@@ -219,7 +252,7 @@ __device__ __forceinline__ void green(T dx, T dy, T dz, T r2, const T *nx, const
 // (g1re, g1im) = SL, (g2re, g2im) = DL with the trial normal ny.
 template <bool HELM, typename T, int PH = 0>
 __device__ __forceinline__ void green_sl_dl(T dx, T dy, T dz, T r2, const T *ny, T kr, T ki, T &g1re, T &g1im,
-                                            T &g2re, T &g2im, T ph0 = T(0)) {
+                                            T &g2re, T &g2im, T ph0 = T(0), T dm0 = T(0)) {
     const T rinv = rsqrt_t(r2);
     const T dot = dx * ny[0] + dy * ny[1] + dz * ny[2];
     if constexpr (!HELM) {
@@ -232,7 +265,7 @@ __device__ __forceinline__ void green_sl_dl(T dx, T dy, T dz, T r2, const T *ny,
         T s, c;
         phase_t<PH>(kr, r, ph0, &s, &c);
         T g = T(kInv4Pi) * rinv;
-        if constexpr (!(PH & kPhReal)) { if (ki != T(0)) g *= exp_t(-ki * r); }
+        damp_t<PH>(ki, r, dm0, g);
         g1re = c * g;
         g1im = s * g;
         const T gd = g * dot * rinv * rinv;
@@ -249,7 +282,7 @@ __device__ __forceinline__ void green_sl_dl(T dx, T dy, T dz, T r2, const T *ny,
 // symmetric pass computes together with the (e, f) entries.
 template <bool HELM, typename T, int PH = 0>
 __device__ __forceinline__ void green_sl_dl_rev(T dx, T dy, T dz, T r2, const T *nx, const T *ny, T kr, T ki, T &g1re,
-                                                T &g1im, T &g2re, T &g2im, T &g3re, T &g3im, T ph0 = T(0)) {
+                                                T &g1im, T &g2re, T &g2im, T &g3re, T &g3im, T ph0 = T(0), T dm0 = T(0)) {
     const T rinv = rsqrt_t(r2);
     const T dot2 = dx * ny[0] + dy * ny[1] + dz * ny[2];
     const T dot3 = -(dx * nx[0] + dy * nx[1] + dz * nx[2]);
@@ -265,7 +298,7 @@ __device__ __forceinline__ void green_sl_dl_rev(T dx, T dy, T dz, T r2, const T 
         T s, c;
         phase_t<PH>(kr, r, ph0, &s, &c);
         T g = T(kInv4Pi) * rinv;
-        if constexpr (!(PH & kPhReal)) { if (ki != T(0)) g *= exp_t(-ki * r); }
+        damp_t<PH>(ki, r, dm0, g);
         g1re = c * g;
         g1im = s * g;
         const T gd = g * rinv * rinv;
@@ -283,11 +316,11 @@ __device__ __forceinline__ void green_sl_dl_rev(T dx, T dy, T dz, T r2, const T 
 // family at the same point pair (shared r and e^{ikr}).
 template <int OP, bool DUAL, typename T, int PH = 0>
 __device__ __forceinline__ void green2(T dx, T dy, T dz, T r2, const T *nx, const T *ny, T kr, T ki, T &g1re, T &g1im,
-                                       T &g2re, T &g2im, T ph0 = T(0)) {
+                                       T &g2re, T &g2im, T ph0 = T(0), T dm0 = T(0)) {
     if constexpr (DUAL) {
-        green_sl_dl<OpTraits<OP>::is_complex, T, PH>(dx, dy, dz, r2, ny, kr, ki, g1re, g1im, g2re, g2im, ph0);
+        green_sl_dl<OpTraits<OP>::is_complex, T, PH>(dx, dy, dz, r2, ny, kr, ki, g1re, g1im, g2re, g2im, ph0, dm0);
     } else {
-        green<OP, T, PH>(dx, dy, dz, r2, nx, ny, kr, ki, g1re, g1im, ph0);
+        green<OP, T, PH>(dx, dy, dz, r2, nx, ny, kr, ki, g1re, g1im, ph0, dm0);
         g2re = g2im = T(0);
     }
 }
@@ -427,7 +460,9 @@ __device__ __forceinline__ C2d local_value(const C2d (&S)[NTS][NSS], int i, int 
         for (int a = 0; a < NTS; ++a)
 #pragma unroll
             for (int b = 0; b < NSS; ++b) {
-                double c = (NTS == 1 ? 1.0 : coef(a, i)) * (NSS == 1 ? 1.0 : coef(b, j));
+                const double c = (NTS == 1 ? 1.0 : coef(a, i)) * (NSS == 1 ? 1.0 : coef(b, j));
+                // the compiler keeps additions of 0 times a value: leave them out where i and j are constants
+                if (__builtin_constant_p(c) && c == 0.0) continue;
                 v.re += c * S[a][b].re;
                 v.im += c * S[a][b].im;
             }
