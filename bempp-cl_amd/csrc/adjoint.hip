@@ -16,8 +16,8 @@
 // trial-side derivative, and no cross-lane reductions are needed. MIXED mode: far pairs in
 // FP32 with the reference-distance split (far_split.h), each unordered pair once, both sides'
 // derivatives from one evaluation (adjoint_far_kernel<TM, true>); near pairs (the ones the
-// mixed forward kernels compute in FP64) in FP64, all ordered pairs. Singular pairs (one
-// wavefront per pair, FP64) differentiate both elements with the weight conj(x_e) y_f, since
+// mixed forward kernels compute in FP64) in FP64, all ordered pairs. Singular pairs (several
+// lanes per pair, FP64) differentiate both elements with the weight conj(x_e) y_f, since
 // their quadrature is not symmetric.
 //
 // Potential. For u_p = sum_e m_e c_e sum_q w_q J_e G(|x_p - y_q|) (bempp_cl/core/numba_kernels.py:
@@ -452,98 +452,154 @@ __global__ __launch_bounds__(256) void adjoint_near_kernel(const Args a, int n_p
 }
 
 // ------------------------------------------------------------------ singular pairs, FP64, both elements
-// kSingLanes lanes per pair (8 pairs per wavefront): the 512..1536 Duffy points are strided over
-// them and the 19 sums reduced in 3 shuffle steps (a wavefront per pair left most lanes of the
-// vertex pairs with 8 points and spent 6 steps per sum)
-constexpr int kSingLanes = 8;
+// The layout of the forward singular kernel: a workgroup takes kSingPairs pairs, kSingSub lanes of every
+// wave share a pair, the pair's points are split over the kSingWaves * kSingSub lanes, the wave stages its
+// points in LDS for all its pairs (the pairs of one rule stand together in the table; a wave with several
+// rules runs them one after the other), and the 19 sums go through shuffles and LDS. 66,500 pairs
+// (5,120 triangles, k = 8): 259 us with 8 lanes per pair loading their own points -> 185 us.
+constexpr int kSingWaves = 4, kSingSub = 4, kSingPairs = 64 / kSingSub, kSingChunk = 96, kSingSums = 19;
 
-template <typename T>
-__device__ __forceinline__ T sing_group_sum(T v) {
+union SingularShared {
+    double2 points[kSingWaves][kSingChunk][3];  // (xi_0, xi_1), (eta_0, eta_1), (w, -)
+    double sums[kSingWaves][kSingSums][kSingPairs];
+};
+
+__global__ __launch_bounds__(64 * kSingWaves, 3) void adjoint_singular_kernel(const Args a, int n_pairs,
+                                                                              const int32_t *pd_all, const double *tpts,
+                                                                              const double *spts, const double *wts) {
+    __shared__ SingularShared sh;
+    __shared__ int32_t vertex[kSingPairs][6];
+    const int lane = threadIdx.x & 63, p = lane % kSingPairs, sub = lane / kSingPairs;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int first = blockIdx.x * kSingPairs;
+    const bool active = first + p < n_pairs;
+    const int32_t *pd = pd_all + 6 * (int64_t)(active ? first + p : first);
+    const int e = pd[0], f = pd[1], toff = pd[2], soff = pd[3], woff = pd[4], np = pd[5];
+    if (threadIdx.x < kSingPairs) {
 #pragma unroll
-    for (int off = kSingLanes / 2; off >= 1; off >>= 1) v += __shfl_xor(v, off, kSingLanes);
-    return v;
-}
-
-__global__ __launch_bounds__(256) void adjoint_singular_kernel(const Args a, int n_pairs, const int32_t *pd_all,
-                                                               const double *tpts, const double *spts,
-                                                               const double *wts) {
-    const int lane = threadIdx.x & (kSingLanes - 1);
-    const int pair = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kSingLanes);
-    // the group's lanes share the pair, so whole groups leave together and the group shuffles
-    // below only read lanes of groups that stay
-    if (pair >= n_pairs) return;
-    const int32_t *pd = pd_all + 6 * (int64_t)pair;
-    const int e = pd[0], f = pd[1], np = pd[5];
-    const double *tp = tpts + 2 * (int64_t)pd[2], *sp = spts + 2 * (int64_t)pd[3], *w = wts + pd[4];
-    const double *gt = a.sp.geom + (int64_t)e * BEM_GEOM_STRIDE;
-    const double *gf = a.sp.geom + (int64_t)f * BEM_GEOM_STRIDE;
+        for (int j = 0; j < 3; ++j) {
+            vertex[p][j] = a.sp.vids[4 * f + j];
+            vertex[p][3 + j] = a.sp.vids[4 * e + j];
+        }
+    }
+    double gt[14], gf[14], c[3];
+#pragma unroll
+    for (int k = 0; k < 14; ++k) {
+        gt[k] = a.sp.geom[(int64_t)e * BEM_GEOM_STRIDE + k];
+        gf[k] = a.sp.geom[(int64_t)f * BEM_GEOM_STRIDE + k];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) c[d] = gf[d] - gt[d];
     double Wr, Wi;
     cmul_conj(a.x, a.sp.l2g[e], a.y, a.sp.l2g[f], Wr, Wi);
     const double m = a.sp.mult[e] * a.sp.mult[f];
     Wr *= m;
     Wi *= m;
-    // Ay[j]: trial vertex j, Ax[j]: test vertex j (both without the J_e J_f factor); S: sum w Re(W G)
-    double Ay[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, Ax[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, S = 0.0;
+    // R[0..8]: trial vertices, R[9..17]: test vertices (both without the J_e J_f factor); R[18]: sum w Re(W G)
+    double R[kSingSums];
+#pragma unroll
+    for (int v = 0; v < kSingSums; ++v) R[v] = 0.0;
     auto points = [&](auto phase_tag) {
         constexpr int PH = decltype(phase_tag)::value;
-        for (int kk = lane; kk < np; kk += kSingLanes) {
-            const double xi0 = tp[2 * kk], xi1 = tp[2 * kk + 1], et0 = sp[2 * kk], et1 = sp[2 * kk + 1];
-            double dv[3];
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                dv[d] = (gf[d] + gf[3 + d] * et0 + gf[6 + d] * et1) - (gt[d] + gt[3 + d] * xi0 + gt[6 + d] * xi1);
-            const double r2 = dv[0] * dv[0] + dv[1] * dv[1] + dv[2] * dv[2];
-            const double rinv = rsqrt_t(r2), r = r2 * rinv;
-            double s, c;
-            sincos_t<PH>(a.k * r, &s, &c);
-            const double Zr = Wr * c - Wi * s, Zi = Wr * s + Wi * c;
-            const double amp = w[kk] * kInv4Pi * rinv;
-            S += amp * Zr;
-            const double t = amp * (-Zr - a.k * r * Zi) * (rinv * rinv);
-            const double py[3] = {1.0 - et0 - et1, et0, et1}, px[3] = {1.0 - xi0 - xi1, xi0, xi1};
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    Ay[j][d] += py[j] * t * dv[d];
-                    Ax[j][d] -= px[j] * t * dv[d];
+        unsigned long long todo = __ballot(active);
+        while (todo) {
+            // the rule of the first pair left, and the lanes that share it
+            const int lead = __ffsll(todo) - 1;
+            const int to = __builtin_amdgcn_readlane(toff, lead), so = __builtin_amdgcn_readlane(soff, lead);
+            const int wo = __builtin_amdgcn_readlane(woff, lead), n = __builtin_amdgcn_readlane(np, lead);
+            const bool mine = active && toff == to && soff == so && woff == wo && np == n;
+            todo &= ~__ballot(mine);
+            const int per = (n + kSingWaves - 1) / kSingWaves, k0 = min(wave * per, n), k1 = min(k0 + per, n);
+            for (int kb = k0; kb < k1; kb += kSingChunk) {
+                const int count = min(kSingChunk, k1 - kb);
+                // the wave's own part of LDS: its accesses complete in order, no barrier
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                for (int k = lane; k < count; k += 64) {
+                    const int64_t kk = kb + k;
+                    sh.points[wave][k][0] = *reinterpret_cast<const double2 *>(tpts + 2 * (to + kk));
+                    sh.points[wave][k][1] = *reinterpret_cast<const double2 *>(spts + 2 * (so + kk));
+                    sh.points[wave][k][2].x = wts[wo + kk];
                 }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (!mine) continue;
+#pragma unroll 2
+                for (int k = sub; k < count; k += kSingSub) {
+                    const double2 px = sh.points[wave][k][0], py = sh.points[wave][k][1];
+                    const double w = sh.points[wave][k][2].x;
+                    double dv[3];
+#pragma unroll
+                    for (int d = 0; d < 3; ++d)
+                        dv[d] = fma(-gt[6 + d], px.y, fma(-gt[3 + d], px.x, fma(gf[6 + d], py.y, fma(gf[3 + d], py.x, c[d]))));
+                    const double r2 = dv[0] * dv[0] + dv[1] * dv[1] + dv[2] * dv[2];
+                    const double rinv = rsqrt_t(r2), r = r2 * rinv;
+                    double s, co;
+                    sincos_t<PH>(a.k * r, &s, &co);
+                    const double Zr = Wr * co - Wi * s, Zi = Wr * s + Wi * co;
+                    const double amp = w * kInv4Pi * rinv;
+                    R[18] += amp * Zr;
+                    const double t = amp * (-Zr - a.k * r * Zi) * (rinv * rinv);
+                    // phi_0 = 1 - xi_0 - xi_1: vertex 0 gets the sum less the other two, after the loop
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        const double td = t * dv[d];
+                        R[d] += td;
+                        R[3 + d] = fma(py.x, td, R[3 + d]);
+                        R[6 + d] = fma(py.y, td, R[6 + d]);
+                        R[12 + d] = fma(-px.x, td, R[12 + d]);
+                        R[15 + d] = fma(-px.y, td, R[15 + d]);
+                    }
+                }
+            }
         }
     };
     // every distance within the pair is at most diam_e + diam_f (triangles sharing a vertex): the
-    // series sin/cos without range reduction when |k| r <= 1, else the branch-free reduction
+    // series sin/cos without range reduction when |k| r <= 1, else the branch-free reduction (wave-uniform)
     const double kd = fabs(a.k) * (gt[13] + gf[13]);
-    if (kd <= 1.0) points(std::integral_constant<int, kPhSmall | kPhReal>{});
-    else if (kd < 0x1p25) points(std::integral_constant<int, kPhReduced | kPhReal>{});
+    if (__all(kd <= 1.0)) points(std::integral_constant<int, kPhSmall | kPhReal>{});
+    else if (__all(kd < 0x1p25)) points(std::integral_constant<int, kPhReduced | kPhReal>{});
     else points(std::integral_constant<int, kPhReal>{});
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
+    for (int d = 0; d < 3; ++d) {
+        R[9 + d] = -R[d] - R[12 + d] - R[15 + d];
+        R[d] -= R[3 + d] + R[6 + d];
+    }
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            Ay[j][d] = sing_group_sum(Ay[j][d]);
-            Ax[j][d] = sing_group_sum(Ax[j][d]);
-        }
-    S = sing_group_sum(S);
-    for (int o = lane; o < 18; o += kSingLanes) {
-        const bool trial_side = o < 9;
-        const int j = (o % 9) / 3, d = o % 3;
-        const double *g = trial_side ? gf : gt;
-        const double other_J = trial_side ? gt[12] : gf[12];
-        double dJ[3][3];
+    for (int v = 0; v < kSingSums; ++v)
+#pragma unroll
+        for (int off = 32; off >= kSingPairs; off >>= 1) R[v] += __shfl_xor(R[v], off, 64);
+    __syncthreads();  // the points have been read
+    if (sub == 0) {
+#pragma unroll
+        for (int v = 0; v < kSingSums; ++v) sh.sums[wave][v][p] = R[v];
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < kSingSums * kSingPairs; idx += 64 * kSingWaves) {
+        double *q = &sh.sums[0][0][0] + idx;
+        double sum = q[0];
+#pragma unroll
+        for (int k = 1; k < kSingWaves; ++k) sum += q[k * kSingSums * kSingPairs];
+        q[0] = sum;
+    }
+    __syncthreads();
+    // the first wave forms the trial side's 9 values of every pair, the second the test side's
+    if (wave < 2 && sub == 0) {
+        const bool trial_side = wave == 0;
+        double g[12], dJ[3][3];
+#pragma unroll
+        for (int k = 0; k < 12; ++k) g[k] = trial_side ? gf[k] : gt[k];
         jacobian_gradient(g, dJ);
-        // select entry (j, d) with compile-time indices (keeps the arrays in registers)
-        double acc = 0.0, dj = 0.0;
+        const double S = sh.sums[0][18][p] * (trial_side ? gt[12] : gf[12]), jj = gt[12] * gf[12];
 #pragma unroll
-        for (int jj = 0; jj < 3; ++jj)
-#pragma unroll
-            for (int dd = 0; dd < 3; ++dd)
-                if (jj == j && dd == d) {
-                    acc = trial_side ? Ay[jj][dd] : Ax[jj][dd];
-                    dj = dJ[jj][dd];
-                }
-        const double val = gt[12] * gf[12] * acc + S * other_J * dj;
-        const int v = a.sp.vids[4 * (trial_side ? f : e) + j];
-        atomic_add(a.grad + 3 * (int64_t)v + d, val);
+        for (int v = 0; v < 9; ++v) {
+            const double val = fma(jj, sh.sums[0][(trial_side ? 0 : 9) + v][p], S * dJ[v / 3][v % 3]);
+            sh.sums[1][(trial_side ? 0 : 9) + v][p] = val;
+        }
+    }
+    __syncthreads();
+    const int count = min(kSingPairs, n_pairs - first) * 18;
+    for (int idx = threadIdx.x; idx < count; idx += 64 * kSingWaves) {
+        const int q = idx / 18, v = idx - 18 * q;
+        atomic_add(a.grad + 3 * (int64_t)vertex[q][v / 3] + v % 3, sh.sums[1][v][q]);
     }
 }
 
@@ -710,10 +766,12 @@ extern "C" int bem_adjoint_single_layer(const bem_space_t *space, const bem_quad
     a.grad = grad_vertices;
     hipStream_t s = (hipStream_t)stream;
     if (a.sp.n > 0) {
-        // test ranges sized so that the grid holds >= ~8 workgroups per CU
         const int ntx = (a.sp.n + adj::kThreads - 1) / adj::kThreads;
+        // test ranges of 2048 down to one 32-element tile until the grid holds 4096 workgroups: half of
+        // them lie below the diagonal, and on small meshes long ranges leave a few busy SIMDs to the end
+        // (5,120 triangles, kernel: ranges of 128 1166 us, 64 833, 32 780 us)
         int range = 2048;
-        while (range > 128 && (long)ntx * ((a.sp.n + range - 1) / range) < 2048) range /= 2;
+        while (range > 32 && (long)ntx * ((a.sp.n + range - 1) / range) < 4096) range /= 2;
         a.range = range;
         a.nty = (a.sp.n + range - 1) / range;
         const dim3 grid(ntx, a.nty);
@@ -728,8 +786,9 @@ extern "C" int bem_adjoint_single_layer(const bem_space_t *space, const bem_quad
     }
     if (n_singular > 0) {
         hipLaunchKernelGGL(adj::adjoint_singular_kernel,
-                           dim3((unsigned)(((int64_t)n_singular * adj::kSingLanes + 255) / 256)), dim3(256), 0, s, a,
-                           n_singular, singular_pairs, test_points, trial_points, weights);
+                           dim3((unsigned)(((int64_t)n_singular + adj::kSingPairs - 1) / adj::kSingPairs)),
+                           dim3(64 * adj::kSingWaves), 0, s, a, n_singular, singular_pairs, test_points, trial_points,
+                           weights);
         if ((rc = check_launch("adjoint_singular_kernel"))) return rc;
     }
     return BEM_OK;
@@ -763,7 +822,9 @@ extern "C" int bem_adjoint_potential_single_layer(const bem_space_t *space, cons
     a.grad = grad_vertices;
     const int nbx = (a.sp.n + adj::kThreads - 1) / adj::kThreads;
     int chunk = adj::kPotTile * 8;
-    while (chunk > adj::kPotTile && (long)nbx * ((n_points + chunk - 1) / chunk) < 2048) chunk /= 2;
+    // at least 64 points per workgroup: below that the 11 atomics per element and workgroup cost more than
+    // the idle SIMDs (5,120 triangles, 1,024 points, kernel: chunks of 256 258 us, 128 155, 64 145, 32 159)
+    while (chunk > 64 && (long)nbx * ((n_points + chunk - 1) / chunk) < 2048) chunk /= 2;
     a.chunk = chunk;
     const dim3 grid(nbx, (n_points + chunk - 1) / chunk);
     hipLaunchKernelGGL(adj::potential_adjoint_kernel, grid, dim3(adj::kThreads), 0, (hipStream_t)stream, a);
