@@ -110,14 +110,9 @@ class SingleLayerProblem(object):
         return getattr(hip, "mixed_near_field_factor", DEFAULT_NEAR_FIELD_FACTOR) if hip is not None else DEFAULT_NEAR_FIELD_FACTOR
 
 
-def _full_coefficients(space, c):
-    """Per-element coefficients m_e c_{dof(e)} of a DP0 space (device, complex128)."""
-    import torch
-
-    dev = c.device
-    l2g = torch.from_numpy(_np.ascontiguousarray(space.local2global[:, 0].astype(_np.int64))).to(dev)
-    mult = torch.from_numpy(_np.ascontiguousarray(space.local_multipliers[:, 0])).to(dev)
-    return (c[l2g] * mult).contiguous()
+def _full_coefficients(dspace, c):
+    """Per-element coefficients m_e c_{dof(e)} of a DP0 space (device copy dspace, complex128)."""
+    return (c[dspace.local2global[:, 0].long()] * dspace.multipliers[:, 0]).contiguous()
 
 
 def _device_rule(parameters):
@@ -183,7 +178,6 @@ def _make_functions():
         @staticmethod
         def forward(ctx, vertices, coefficients, points, problem):
             from bempp_amd.core import hip_backend as hb
-            from bempp_amd.core.dense_potential_assembler import hip_potential_assembler
 
             grid = problem.grid(vertices)
             space = problem.space(grid)
@@ -194,10 +188,15 @@ def _make_functions():
             pts = points.detach().to(dev, torch.float64).contiguous()
             if pts.dim() != 2 or pts.shape[1] != 3:
                 raise ValueError("points must have shape (n_points, 3)")
-            points_host = pts.cpu().numpy().T
-            pot = problem.potential(space, points_host)
-            evaluate = hip_potential_assembler(space, pot.descriptor, points_host, problem.parameters)
-            out, _ = evaluate(_full_coefficients(space, c), as_tensor=True)
+            # the points, the density and the dof map stay on the device: a potential operator would copy the
+            # points to the host and map the coefficients there, twice the time of the kernels on small meshes
+            mode = problem.mode()
+            op = "laplace_single_layer" if problem.wavenumber == 0.0 else "helmholtz_single_layer"
+            dspace = hb.potential_space(space, op, mode)
+            out = torch.empty((1, pts.shape[0]), dtype=torch.complex64 if mode == hb.PRECISION_MIXED else torch.complex128,
+                              device=dev)
+            hb.potential_evaluate(op, dspace, _full_coefficients(dspace, c), pts, _device_rule(problem.parameters),
+                                  problem.wavenumber, mode, out)
             ctx.problem, ctx.space, ctx.c, ctx.pts = problem, space, c, pts
             ctx.vdevice, ctx.cdevice = vertices.device, coefficients.device
             return out[0].to(torch.complex128)
