@@ -482,14 +482,12 @@ __global__ __launch_bounds__(64 * kSingWaves, 3) void adjoint_singular_kernel(co
             vertex[p][3 + j] = a.sp.vids[4 * e + j];
         }
     }
-    double gt[14], gf[14], c[3];
+    double gt[14], gf[14];
 #pragma unroll
     for (int k = 0; k < 14; ++k) {
         gt[k] = a.sp.geom[(int64_t)e * BEM_GEOM_STRIDE + k];
         gf[k] = a.sp.geom[(int64_t)f * BEM_GEOM_STRIDE + k];
     }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) c[d] = gf[d] - gt[d];
     double Wr, Wi;
     cmul_conj(a.x, a.sp.l2g[e], a.y, a.sp.l2g[f], Wr, Wi);
     const double m = a.sp.mult[e] * a.sp.mult[f];
@@ -529,7 +527,8 @@ __global__ __launch_bounds__(64 * kSingWaves, 3) void adjoint_singular_kernel(co
                     double dv[3];
 #pragma unroll
                     for (int d = 0; d < 3; ++d)
-                        dv[d] = fma(-gt[6 + d], px.y, fma(-gt[3 + d], px.x, fma(gf[6 + d], py.y, fma(gf[3 + d], py.x, c[d]))));
+                        dv[d] = fma(gf[6 + d], py.y, fma(gf[3 + d], py.x, gf[d])) -
+                                fma(gt[6 + d], px.y, fma(gt[3 + d], px.x, gt[d]));
                     const double r2 = dv[0] * dv[0] + dv[1] * dv[1] + dv[2] * dv[2];
                     const double rinv = rsqrt_t(r2), r = r2 * rinv;
                     double s, co;

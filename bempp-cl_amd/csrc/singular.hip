@@ -12,7 +12,7 @@
 // added to the dense output with hardware atomics, real and imaginary part on neighbouring lanes (one
 // memory-side request), which replaces the reference's host-side np.add.at scatter
 // (bempp_cl/core/dense_assembler.py:78-98).
-// Bound by FP64 arithmetic: 68 instructions a point for a complex single layer on P1, 23 for the
+// Bound by FP64 arithmetic: 71 instructions a point for a complex single layer on P1, 26 for the
 // Laplace one on DP0.
 #include "bem_device.h"
 #include "bem_internal.h"
@@ -70,8 +70,8 @@ __global__ __launch_bounds__(64 * W, W == 4 && !(DUAL && NTS * NSS == 9) ? 3 : 2
             mult[NTS + j][p] = a.trial.mult[(int64_t)f * NSS + j];
         }
     }
-    // the geometry rows in registers; y - x = c + e1_f eta_0 + e2_f eta_1 - e1_t xi_0 - e2_t xi_1
-    double gt[14], gf[14], c[3], nx[3], ny[3];
+    // the geometry rows in registers
+    double gt[14], gf[14], nx[3], ny[3];
 #pragma unroll
     for (int k = 0; k < 14; ++k) {
         gt[k] = a.test.geom[(int64_t)e * BEM_GEOM_STRIDE + k];
@@ -79,7 +79,6 @@ __global__ __launch_bounds__(64 * W, W == 4 && !(DUAL && NTS * NSS == 9) ? 3 : 2
     }
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        c[d] = gf[d] - gt[d];
         nx[d] = gt[9 + d] * tnm;
         ny[d] = gf[9 + d] * snm;
     }
@@ -121,10 +120,13 @@ __global__ __launch_bounds__(64 * W, W == 4 && !(DUAL && NTS * NSS == 9) ? 3 : 2
                 for (int k = sub; k < count; k += G) {
                     const double2 px = sh.points[wave][k][0], py = sh.points[wave][k][1];
                     const double xi0 = px.x, xi1 = px.y, et0 = py.x, et1 = py.y, w = sh.points[wave][k][2].x;
+                    // the two points, then their difference: the swapped points of a coincident pair get exactly
+                    // opposite differences, so that its double layer cancels
                     double d[3];
 #pragma unroll
                     for (int m = 0; m < 3; ++m)
-                        d[m] = fma(-gt[6 + m], xi1, fma(-gt[3 + m], xi0, fma(gf[6 + m], et1, fma(gf[3 + m], et0, c[m]))));
+                        d[m] = fma(gf[6 + m], et1, fma(gf[3 + m], et0, gf[m])) -
+                               fma(gt[6 + m], xi1, fma(gt[3 + m], xi0, gt[m]));
                     const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
                     double g[2][2];
                     green2<green_op<OP>(), DUAL, double, PH>(d[0], d[1], d[2], r2, nx, ny, a.kr, a.ki, g[0][0], g[0][1],
