@@ -75,11 +75,13 @@ def device_gmres(tensor, b, rtol=1e-5, restart=None, maxiter=None, callback=None
 
     if tensor.shape[0] != tensor.shape[1]:
         raise ValueError("GMRES needs a square operator")
-    return krylov_gmres(lambda v: device_matvec(tensor, v), b, tensor.device, rtol, restart, maxiter, callback)
+    return krylov_gmres(lambda v: device_matvec(tensor, v), b, tensor.device, rtol, restart, maxiter, callback,
+                        matrix=tensor if tensor.stride(1) == 1 else None)
 
 
-def krylov_gmres(matvec, b, dev, rtol=1e-5, restart=None, maxiter=None, callback=None):
-    """Restarted GMRES with the operator given as matvec (complex128 tensors on dev)."""
+def krylov_gmres(matvec, b, dev, rtol=1e-5, restart=None, maxiter=None, callback=None, matrix=None):
+    """Restarted GMRES with the operator given as matvec (complex128 tensors on dev). matrix: the operator's
+    row-major device matrix, if it has one: an Arnoldi step is then one library call."""
     import torch
     from scipy.linalg import solve_triangular
 
@@ -112,11 +114,18 @@ def krylov_gmres(matvec, b, dev, rtol=1e-5, restart=None, maxiter=None, callback
         gs_host = [torch.empty(nbuf, dtype=torch.complex128, pin_memory=True) for _ in range(2)]
         gs_event = [torch.cuda.Event() for _ in range(2)]
 
+        step = None
+        if matrix is not None:
+            step = hb.gmres_stepper(matrix, V, torch.empty(n, dtype=torch.complex128, device=dev), gs_out, gs_host, eps)
+
         def issue(c):
-            wv = matvec(V[c]).to(torch.complex128).contiguous()
             b = c % 2
-            hb.gmres_cgs2(V, c + 1, wv, gs_out[b], V[c + 1], eps)
-            gs_host[b][: 2 * c + 4].copy_(gs_out[b][: 2 * c + 4], non_blocking=True)
+            if step is not None:
+                step(c + 1, b)
+            else:
+                wv = matvec(V[c]).to(torch.complex128).contiguous()
+                hb.gmres_cgs2(V, c + 1, wv, gs_out[b], V[c + 1], eps)
+                gs_host[b][: 2 * c + 4].copy_(gs_out[b][: 2 * c + 4], non_blocking=True)
             gs_event[b].record()
 
     h = _np.zeros((restart, restart + 1), dtype=_np.complex128)

@@ -144,6 +144,8 @@ def lib():
         L.bem_dense_matvec.restype = i
         L.bem_gmres_cgs2.argtypes = [P, i64, i, i64, P, P, P, ctypes.c_double, P]
         L.bem_gmres_cgs2.restype = i
+        L.bem_gmres_step.argtypes = [P, i, i64, i64, P, i64, i, P, P, P, ctypes.c_double, P]
+        L.bem_gmres_step.restype = i
         L.bem_regular_assemble_sl_dl.argtypes = [i, SP, SP, BP, BP, i, QP, d, d, i, d, i, P, P, i64, i, i, P]
         L.bem_regular_assemble_sl_dl.restype = i
         L.bem_regular_assemble_sl_dl_symmetric.argtypes = [i, SP, BP, BP, i, P, i64, QP, d, d, i, d, i, P, P, i64, i, P]
@@ -472,6 +474,33 @@ def gmres_cgs2(V, k, w, out, v_next=None, eps=0.0):
         raise ValueError("v_next must be a contiguous complex128 vector of length n")
     check(lib().bem_gmres_cgs2(ptr(V), V.stride(0), int(k), int(n), ptr(w), ptr(out),
                                None if v_next is None else ptr(v_next), float(eps), stream_handle()))
+
+
+def gmres_stepper(A, V, w, out, host, eps):
+    """step(k, b): one Arnoldi step of GMRES on the current stream in one library call (w = A V[k - 1], CGS2 of
+    w against V[:k], next basis vector into V[k], the 2k + 2 coefficients into the page-locked tensor host[b]).
+    The checks are made and the addresses read once per solve; the function keeps the tensors alive."""
+    torch = _torch()
+    n = V.shape[1]
+    if A.shape != (n, n) or A.stride(1) != 1 or V.dtype != torch.complex128 or not V.is_contiguous():
+        raise ValueError("A must be a row-major (n, n) tensor and V a contiguous (m, n) complex128 tensor")
+    for t in (w, *out, *host):
+        if t.dtype != torch.complex128 or not t.is_contiguous():
+            raise ValueError("w, out and host must be contiguous complex128 tensors")
+    m = V.shape[0]
+    if w.shape != (n,) or any(t.numel() < 2 * m for t in (*out, *host)):
+        raise ValueError("w must have length n, out and host 2 * rows of V values")
+    fn, a, dtype, ld, v, wp, s = lib().bem_gmres_step, ptr(A), _dtype_code(A), A.stride(0), ptr(V), ptr(w), stream_handle()
+    outs, hosts = [ptr(t) for t in out], [ptr(t) for t in host]
+
+    keep = (A, V, w, tuple(out), tuple(host))
+
+    def step(k, b, keep=keep):
+        if not 1 <= k < m:
+            raise ValueError("k must leave a row of V for the next basis vector")
+        check(fn(a, dtype, n, ld, v, n, k, wp, outs[b], hosts[b], eps, s))
+
+    return step
 
 
 def regular_assemble_sl_dl(op, test, trial, test_blocks, trial_blocks, grids_identical, rule, wavenumber, precision,

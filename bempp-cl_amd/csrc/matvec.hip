@@ -10,6 +10,7 @@
 //  * op = N, 16-byte aligned rows: workgroups of 32 rows x 1024 columns; the x chunk is staged in
 //    LDS once per workgroup, each wavefront streams 8 rows with 16-byte loads (8 independent loads
 //    in flight per lane), and the column chunks' FP64 sums are combined with FP64 atomics.
+//  * op = N, 16-byte aligned rows, too few such tiles for the chip: one wavefront per one or two rows.
 //  * op = N otherwise: one wavefront per row; lanes read consecutive columns, x from L2.
 //  * op = T/C: each workgroup owns 256 consecutive columns and a band of rows; every lane
 //    walks its column down the band, and the band sums are added to y with FP64 atomics.
@@ -103,6 +104,12 @@ constexpr int kMvRows = 32;          // rows per workgroup
 constexpr int kMvRowsPerWave = 8;    // rows per wavefront
 constexpr int kMvCols = 1024;        // columns per workgroup (x chunk: 16 KB of LDS)
 
+// below this many 32 x 1024 tiles a wavefront takes whole rows instead (kMvSingleRows: one row each up to
+// here, else two): complex64, n = 1,002 12.5 -> 9.8 us (calls back to back), 2,562 14.6 -> 11.9,
+// 4,000 26.6 -> 21.3 us
+constexpr int64_t kMvTiles = 1024;
+constexpr int64_t kMvSingleRows = 2048;
+
 // y_i += sum_{j in the chunk} A_ij x_j (y zeroed beforehand); rows start 16-byte aligned
 template <typename AT>
 __global__ __launch_bounds__(256, sizeof(AT) == 4 ? 3 : 4) void matvec_n_tiled_kernel(const void *A, int64_t rows, int64_t cols, int64_t ld,
@@ -172,6 +179,63 @@ __global__ __launch_bounds__(256, sizeof(AT) == 4 ? 3 : 4) void matvec_n_tiled_k
     }
 }
 
+// y_i = sum_j A_ij x_j, one wavefront per R rows over all columns, 16-byte loads; rows start 16-byte
+// aligned. For matrices whose 32-row tiles would not fill the chip: nothing is shared between workgroups,
+// so y needs no zeroing and no atomics, and x comes from the caches.
+template <typename AT, int R>
+__global__ __launch_bounds__(256) void matvec_n_rows_kernel(const void *A, int64_t rows, int64_t cols, int64_t ld,
+                                                            const double *x, double *y) {
+    using P = Pack16<AT>;
+    constexpr int E = P::E;
+    const int lane = threadIdx.x & 63;
+    const int64_t r0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
+    if (r0 >= rows) return;  // uniform per wavefront
+    const AT *rowp[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) rowp[r] = reinterpret_cast<const AT *>(A) + min(r0 + r, rows - 1) * ld;
+    double sr[R], si[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) sr[r] = si[r] = 0.0;
+    const double2 *xs = reinterpret_cast<const double2 *>(x);
+    const int64_t nfull = cols - cols % E;  // columns covered by whole 16-byte loads
+#pragma unroll 4
+    for (int64_t j = lane * E; j < nfull; j += 64 * E) {
+        double2 xv[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) xv[e] = xs[j + e];
+        typename P::V v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = *reinterpret_cast<const typename P::V *>(rowp[r] + j);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                double ar, ai;
+                P::get(v[r], e, ar, ai);
+                sr[r] += ar * xv[e].x - ai * xv[e].y;
+                si[r] += ar * xv[e].y + ai * xv[e].x;
+            }
+    }
+    for (int64_t j = nfull + lane; j < cols; j += 64) {
+        const double2 xv = xs[j];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            double ar, ai;
+            Elem<AT>::get(rowp[r], j, ar, ai);
+            sr[r] += ar * xv.x - ai * xv.y;
+            si[r] += ar * xv.y + ai * xv.x;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const double a = wsum(sr[r]), b = wsum(si[r]);
+        if (lane == 0 && r0 + r < rows) {
+            y[2 * (r0 + r)] = a;
+            y[2 * (r0 + r) + 1] = b;
+        }
+    }
+}
+
 // y_i = sum_j A_ij x_j, one wavefront per row
 template <typename AT>
 __global__ __launch_bounds__(256) void matvec_n_kernel(const void *A, int64_t rows, int64_t cols, int64_t ld,
@@ -228,6 +292,16 @@ int launch(int trans, const void *A, int64_t rows, int64_t cols, int64_t ld, con
            hipStream_t s) {
     const bool aligned = reinterpret_cast<uintptr_t>(A) % 16 == 0 && (ld * (int64_t)sizeof(AT)) % 16 == 0;
     const int64_t nchunks = (cols + kMvCols - 1) / kMvCols;
+    const int64_t ntiles = (rows + kMvRows - 1) / kMvRows * nchunks;
+    if (trans == 0 && aligned && reinterpret_cast<uintptr_t>(x) % 16 == 0 && ntiles < kMvTiles) {
+        if (rows <= kMvSingleRows)
+            hipLaunchKernelGGL((matvec_n_rows_kernel<AT, 1>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, A, rows,
+                               cols, ld, x, y);
+        else
+            hipLaunchKernelGGL((matvec_n_rows_kernel<AT, 2>), dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, s, A, rows,
+                               cols, ld, x, y);
+        return check_launch("matvec_n_rows_kernel");
+    }
     if (trans == 0 && aligned && nchunks <= 65535) {
         hipLaunchKernelGGL(zero_kernel, dim3((unsigned)((2 * rows + 255) / 256)), dim3(256), 0, s, y, 2 * rows);
         const dim3 grid((unsigned)((rows + kMvRows - 1) / kMvRows), (unsigned)nchunks);
@@ -478,6 +552,95 @@ __global__ __launch_bounds__(kThreads) void cgs2_scale_kernel(const double2 *w, 
     }
 }
 
+// The whole step in one workgroup, for short vectors: w stays in LDS, a wave forms whole dot products, a
+// thread updates its own elements. One launch instead of five with a few blocks each: n = 1,002 (calls back
+// to back) k = 1 / 10 / 20 13.9 / 13.6 / 17.5 us against 21 / 23 / 35; n = 4,096 13.6 / 26 / 43 against
+// 21 / 24 / 35, so the line lies at 2,048.
+constexpr int kSmallThreads = 1024, kSmallN = 2048, kSmallK = 64;
+
+__global__ __launch_bounds__(kSmallThreads) void cgs2_small_kernel(const double2 *V, int64_t ldv, int k, int n,
+                                                                   double2 *w, double2 *out, double eps,
+                                                                   double2 *v_next) {
+    constexpr int NW = kSmallThreads / 64;
+    __shared__ double2 ws[kSmallN];
+    __shared__ double2 c[kSmallK];
+    __shared__ double red[NW][2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // |w|^2 over the workgroup; every thread gets it
+    auto norm2 = [&](double part) {
+        double dummy = 0.0;
+        wave_sum2(part, dummy);
+        if (lane == 0) red[wave][0] = part;
+        __syncthreads();
+        double sum = 0.0;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) sum += red[v][0];
+        __syncthreads();  // red is reused
+        return sum;
+    };
+    // c = conj(V) w
+    auto dots = [&]() {
+        for (int i = wave; i < k; i += NW) {
+            const double2 *row = V + (int64_t)i * ldv;
+            double re = 0.0, im = 0.0;
+#pragma unroll 8
+            for (int j = lane; j < n; j += 64) {
+                const double2 a = row[j], v = ws[j];
+                re += a.x * v.x + a.y * v.y;
+                im += a.x * v.y - a.y * v.x;
+            }
+            wave_sum2(re, im);
+            if (lane == 0) c[i] = make_double2(re, im);
+        }
+        __syncthreads();
+    };
+    // w -= V^T c on the thread's elements; returns their part of |w|^2
+    auto update = [&]() {
+        double part = 0.0;
+        for (int j = tid; j < n; j += kSmallThreads) {
+            double2 v = ws[j];
+#pragma unroll 4
+            for (int i = 0; i < k; ++i) {
+                const double2 a = V[(int64_t)i * ldv + j], ci = c[i];
+                v.x -= a.x * ci.x - a.y * ci.y;
+                v.y -= a.x * ci.y + a.y * ci.x;
+            }
+            ws[j] = v;
+            part += v.x * v.x + v.y * v.y;
+        }
+        return part;
+    };
+    double part = 0.0;
+    for (int j = tid; j < n; j += kSmallThreads) {
+        const double2 v = w[j];
+        ws[j] = v;
+        part += v.x * v.x + v.y * v.y;
+    }
+    const double h0 = norm2(part);  // its barriers publish ws
+    dots();
+    if (tid < k) out[tid] = c[tid];
+    if (tid == 0) out[k] = make_double2(h0, 0.0);
+    update();
+    __syncthreads();  // ws complete, c read
+    dots();
+    if (tid < k) out[k + 1 + tid] = c[tid];
+    const double h1 = norm2(update());
+    if (tid == 0) out[2 * k + 1] = make_double2(h1, 0.0);
+    const double r0 = sqrt(h0), r1 = sqrt(h1);
+    const bool keep = r1 <= eps * r0;
+    for (int j = tid; j < n; j += kSmallThreads) {
+        double2 v = ws[j];
+        w[j] = v;
+        if (v_next) {
+            if (!keep) {
+                v.x /= r1;
+                v.y /= r1;
+            }
+            v_next[j] = v;
+        }
+    }
+}
+
 }  // namespace gs
 
 }  // namespace bem
@@ -497,6 +660,11 @@ extern "C" int bem_gmres_cgs2(const void *V, int64_t ldv, int k, int64_t n, void
         return BEM_ERR_INVALID_ARGUMENT;
     }
     hipStream_t s = (hipStream_t)stream;
+    if (n <= gs::kSmallN && k <= gs::kSmallK && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+        hipLaunchKernelGGL(gs::cgs2_small_kernel, dim3(1), dim3(gs::kSmallThreads), 0, s, (const double2 *)V, ldv, k,
+                           (int)n, (double2 *)w, (double2 *)out, eps, (double2 *)v_next);
+        return check_launch("cgs2_small_kernel");
+    }
     const int64_t nout = 2 * (2 * (int64_t)k + 2);
     hipLaunchKernelGGL(mv::zero_kernel, dim3((unsigned)((nout + 255) / 256)), dim3(256), 0, s, (double *)out, nout);
     int64_t blocks = (n + gs::kThreads - 1) / gs::kThreads;
@@ -561,4 +729,24 @@ extern "C" int bem_dense_matvec(int trans, const void *A, int a_dtype, int64_t r
     case BEM_C128: return mv::launch<double2>(trans, A, rows, cols, ld, xd, yd, s);
     default: set_error("unknown matrix dtype %d", a_dtype); return BEM_ERR_INVALID_ARGUMENT;
     }
+}
+
+extern "C" int bem_gmres_step(const void *A, int a_dtype, int64_t n, int64_t ld, void *V, int64_t ldv, int k, void *w,
+                              void *out, void *out_host, double eps, void *stream) {
+    if (!V || k < 1 || !out_host) {
+        clear_error();
+        set_error("invalid argument");
+        return BEM_ERR_INVALID_ARGUMENT;
+    }
+    double *rows = (double *)V;
+    int rc = bem_dense_matvec(0, A, a_dtype, n, n, ld, rows + 2 * (k - 1) * ldv, w, stream);
+    if (rc == BEM_OK) rc = bem_gmres_cgs2(V, ldv, k, n, w, out, rows + 2 * k * ldv, eps, stream);
+    if (rc != BEM_OK) return rc;
+    const hipError_t e = hipMemcpyAsync(out_host, out, sizeof(double) * 2 * (2 * (size_t)k + 2), hipMemcpyDeviceToHost,
+                                        (hipStream_t)stream);
+    if (e != hipSuccess) {
+        set_error("copy of the coefficients: %s", hipGetErrorString(e));
+        return BEM_ERR_DEVICE;
+    }
+    return BEM_OK;
 }

@@ -383,6 +383,15 @@ int bem_gmres_cgs2(const void *V, int64_t ldv, int k, int64_t n, void *w, void *
                    void *stream);
 
 /*
+ * One Arnoldi step of GMRES in one call (no reference counterpart, as bem_gmres_cgs2): w = A v with v the
+ * row k - 1 of V (A: n x n, leading dimension ld, enum bem_dtype), then bem_gmres_cgs2 of w against the
+ * rows [0, k) with row k of V as the next basis vector, then a copy of the 2k + 2 coefficients to out_host
+ * (page-locked host memory), all enqueued on the stream. V holds at least k + 1 rows.
+ */
+int bem_gmres_step(const void *A, int a_dtype, int64_t n, int64_t ld, void *V, int64_t ldv, int k, void *w, void *out,
+                   void *out_host, double eps, void *stream);
+
+/*
  * y = op(A) x for a dense row-major matrix in HBM (the product of the reference's
  * DenseDiscreteBoundaryOperator, bempp_cl/api/assembly/discrete_boundary_operator.py).
  * trans: 0 = A x, 1 = A^T x, 2 = A^H x. a_dtype: enum bem_dtype. x, y: complex128 device

@@ -240,3 +240,58 @@ def test_gmres_cgs2_entry_point(k, n, hip_available):
     hb.gmres_cgs2(Vt, k, w3, out, Vt[k + 1], 1e300)
     np.testing.assert_array_equal(Vt[k + 1].cpu().numpy(), w3.cpu().numpy())
 
+
+
+@pytest.mark.parametrize("n", [1, 2, 65, 2047, 2048, 2049])
+@pytest.mark.parametrize("dtype", ["float32", "float64", "complex64", "complex128"])
+def test_gmres_step_equals_its_parts(n, dtype, hip_available):
+    """One call per Arnoldi step (product, CGS2, next basis vector, coefficients on the host) against the same
+    step in torch, on both sides of the vector length at which one workgroup does the orthogonalisation."""
+    import torch
+
+    from bempp_amd.core import hip_backend as hb
+
+    dev = hb.device()
+    torch.manual_seed(n)
+    A = torch.randn((n, n), dtype=getattr(torch, dtype), device=dev)
+    m = min(n, 4)
+    Q = torch.linalg.qr(torch.randn((n, m), dtype=torch.complex128, device=dev))[0].T.contiguous()
+    V = torch.zeros((m + 1, n), dtype=torch.complex128, device=dev)
+    V[:m] = Q
+    buf = 2 * (m + 1)
+    out = [torch.empty(buf, dtype=torch.complex128, device=dev) for _ in range(2)]
+    host = [torch.empty(buf, dtype=torch.complex128, pin_memory=True) for _ in range(2)]
+    step = hb.gmres_stepper(A, V, torch.empty(n, dtype=torch.complex128, device=dev), out, host, 0.0)
+    step(m, 1)
+    torch.cuda.synchronize()
+    w = A.to(torch.complex128) @ Q[m - 1]
+    norm = torch.linalg.vector_norm(w)
+    c1 = Q.conj() @ w
+    w1 = w - Q.T @ c1
+    w2 = w1 - Q.T @ (Q.conj() @ w1)
+    got = host[1].to(dev)
+    # sums of n FP64 products: n eps sqrt-wise; 1e-13 covers n = 2,049
+    assert torch.linalg.vector_norm(got[:m] - c1) < 1e-13 * norm
+    assert abs(got[m].real.sqrt() - norm) < 1e-13 * norm
+    assert abs(got[2 * m + 1].real.sqrt() - torch.linalg.vector_norm(w2)) < 1e-13 * norm
+    if n > m:  # else nothing is left of w but rounding
+        assert torch.linalg.vector_norm(V[m] - w2 / torch.linalg.vector_norm(w2)) < 1e-12
+    assert torch.equal(V[:m], Q)
+
+
+@pytest.mark.parametrize("rows,cols,ld", [(1, 1, 2), (3, 1001, 1002), (2048, 33, 34), (2049, 70, 72), (5000, 1030, 1032)])
+@pytest.mark.parametrize("dtype", ["float32", "float64", "complex64", "complex128"])
+def test_product_by_whole_rows(rows, cols, ld, dtype, hip_available):
+    """Products whose 32-row tiles would not fill the chip: one or two rows per wavefront, remainders of rows
+    and of 16-byte loads (float32 takes rows of a multiple of 4, the others of 2 values)."""
+    import torch
+
+    from bempp_amd.core import hip_backend as hb
+
+    torch.manual_seed(rows)
+    ld = (ld + 3) // 4 * 4
+    A = torch.randn((rows, ld), dtype=getattr(torch, dtype), device=hb.device())[:, :cols]
+    x = torch.randn(cols, dtype=torch.complex128, device=hb.device())
+    y = hb.dense_matvec(A, x)
+    ref = A.to(torch.complex128) @ x
+    assert torch.linalg.vector_norm(y - ref) < 1e-14 * cols**0.5 * torch.linalg.vector_norm(ref)
