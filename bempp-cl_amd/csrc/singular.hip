@@ -5,8 +5,8 @@
 // A workgroup of W waves takes 64 / G consecutive pairs; in every wave G lanes share a pair and the
 // pair's points are split over the W G lanes. The pair table lists the pairs of one rule (kind and
 // local vertices) together, so a wave's pairs share the points: the wave stages its part of them in LDS
-// with coalesced loads and reads them as broadcasts (a wave whose pairs have several rules runs them one
-// after the other). Each lane accumulates the moment block S[a][b] = sum_k G_k w_k u_a(xi_k) u_b(eta_k),
+// with coalesced loads and reads them as broadcasts (the pairs of a wave that spans several rules read
+// their points from memory). Each lane accumulates the moment block S[a][b] = sum_k G_k w_k u_a(xi_k) u_b(eta_k),
 // u = (1, xi_0, xi_1), of its points; the partial blocks are summed by shuffles and through LDS, scaled
 // by J_test J_trial and turned into the local matrix block exactly as for regular pairs. The entries are
 // added to the dense output with hardware atomics, real and imaginary part on neighbouring lanes (one
@@ -33,15 +33,20 @@ struct SingularArgs {
 // LDS of one workgroup: the staged points, then the partial moments and the local blocks
 template <int NV, int W, int G>
 union SingularShared {
-    static constexpr int kChunk = G == 1 ? 64 : 96;  // points a wave stages at a time
-    double2 points[W][kChunk][3];                     // (xi_0, xi_1), (eta_0, eta_1), (w, -)
+    // points a wave stages at a time, with their loads in flight together: a vertex pair's part (128) in one
+    // step; one load each where the lanes take all of them (10 registers less)
+    static constexpr int kLoads = G == 1 ? 1 : 2, kChunk = 64 * kLoads;
+    struct {
+        double2 points[W][kChunk][2];  // (xi_0, xi_1), (eta_0, eta_1)
+        double weights[W][kChunk];
+    } st;
     double moments[W][NV][64 / G];
 };
 
 // DUAL: OP is a single layer; the double layer of the same family (sharing r and e^{ikr} at
 // every point) goes to a.out2.
 template <int OP, int NTS, int NSS, typename OutT, bool DUAL, int W, int G>
-__global__ __launch_bounds__(64 * W, W == 4 && !(DUAL && NTS * NSS == 9) ? 3 : 2) void singular_kernel(const SingularArgs a) {
+__global__ __launch_bounds__(64 * W, !(DUAL && NTS * NSS == 9) ? 3 : 2) void singular_kernel(const SingularArgs a) {
     constexpr bool CPLX = OpTraits<OP>::is_complex;
     constexpr int NC = CPLX ? 2 : 1, NB = NTS * NSS, NV = NB * NC, NOPS = DUAL ? 2 : 1;
     constexpr int PP = 64 / G;  // pairs per workgroup
@@ -95,58 +100,76 @@ __global__ __launch_bounds__(64 * W, W == 4 && !(DUAL && NTS * NSS == 9) ? 3 : 2
 
     auto points = [&](auto phase_tag) {
         constexpr int PH = decltype(phase_tag)::value;
-        unsigned long long todo = __ballot(active);
-        while (todo) {
-            // the rule of the first pair left, and the lanes that share it
-            const int lead = __ffsll(todo) - 1;
-            const int to = __builtin_amdgcn_readlane(toff, lead), so = __builtin_amdgcn_readlane(soff, lead);
-            const int wo = __builtin_amdgcn_readlane(woff, lead), n = __builtin_amdgcn_readlane(np, lead);
-            const bool mine = active && toff == to && soff == so && woff == wo && np == n;
-            todo &= ~__ballot(mine);
-            const int per = (n + W - 1) / W, k0 = min(wave * per, n), k1 = min(k0 + per, n);
-            for (int kb = k0; kb < k1; kb += Shared::kChunk) {
-                const int count = min(Shared::kChunk, k1 - kb);
-                // the wave's own part of LDS: its accesses complete in order, no barrier
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                for (int k = lane; k < count; k += 64) {
-                    const int64_t kk = kb + k;
-                    sh.points[wave][k][0] = *reinterpret_cast<const double2 *>(a.tpts + 2 * (to + kk));
-                    sh.points[wave][k][1] = *reinterpret_cast<const double2 *>(a.spts + 2 * (so + kk));
-                    sh.points[wave][k][2].x = a.wts[wo + kk];
-                }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                if (!mine) continue;
-#pragma unroll 2
-                for (int k = sub; k < count; k += G) {
-                    const double2 px = sh.points[wave][k][0], py = sh.points[wave][k][1];
-                    const double xi0 = px.x, xi1 = px.y, et0 = py.x, et1 = py.y, w = sh.points[wave][k][2].x;
-                    // the two points, then their difference: the swapped points of a coincident pair get exactly
-                    // opposite differences, so that its double layer cancels
-                    double d[3];
+        // one point: xi, eta and its weight
+        auto point = [&](double xi0, double xi1, double et0, double et1, double w) {
+            // the two points, then their difference: the swapped points of a coincident pair get exactly
+            // opposite differences, so that its double layer cancels
+            double d[3];
 #pragma unroll
-                    for (int m = 0; m < 3; ++m)
-                        d[m] = fma(gf[6 + m], et1, fma(gf[3 + m], et0, gf[m])) -
-                               fma(gt[6 + m], xi1, fma(gt[3 + m], xi0, gt[m]));
-                    const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-                    double g[2][2];
-                    green2<green_op<OP>(), DUAL, double, PH>(d[0], d[1], d[2], r2, nx, ny, a.kr, a.ki, g[0][0], g[0][1],
-                                                             g[1][0], g[1][1]);
+            for (int m = 0; m < 3; ++m)
+                d[m] = fma(gf[6 + m], et1, fma(gf[3 + m], et0, gf[m])) -
+                       fma(gt[6 + m], xi1, fma(gt[3 + m], xi0, gt[m]));
+            const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+            double g[2][2];
+            green2<green_op<OP>(), DUAL, double, PH>(d[0], d[1], d[2], r2, nx, ny, a.kr, a.ki, g[0][0], g[0][1],
+                                                     g[1][0], g[1][1]);
 #pragma unroll
-                    for (int o = 0; o < NOPS; ++o)
+            for (int o = 0; o < NOPS; ++o)
 #pragma unroll
-                        for (int z = 0; z < NC; ++z) {
-                            const double t0 = g[o][z] * w;
-                            const double t[3] = {t0, t0 * et0, t0 * et1};
+                for (int z = 0; z < NC; ++z) {
+                    const double t0 = g[o][z] * w;
+                    const double t[3] = {t0, t0 * et0, t0 * et1};
 #pragma unroll
-                            for (int j = 0; j < NSS; ++j) {
-                                S[o][z][0][j] += t[j];
-                                if constexpr (NTS == 3) {
-                                    S[o][z][1][j] = fma(t[j], xi0, S[o][z][1][j]);
-                                    S[o][z][2][j] = fma(t[j], xi1, S[o][z][2][j]);
-                                }
-                            }
+                    for (int j = 0; j < NSS; ++j) {
+                        S[o][z][0][j] += t[j];
+                        if constexpr (NTS == 3) {
+                            S[o][z][1][j] = fma(t[j], xi0, S[o][z][1][j]);
+                            S[o][z][2][j] = fma(t[j], xi1, S[o][z][2][j]);
                         }
+                    }
                 }
+        };
+        // the rule of the first pair, and whether the wave's pairs share it
+        const int to = __builtin_amdgcn_readfirstlane(toff), so = __builtin_amdgcn_readfirstlane(soff);
+        const int wo = __builtin_amdgcn_readfirstlane(woff), n = __builtin_amdgcn_readfirstlane(np);
+        if (!__all(!active || (toff == to && soff == so && woff == wo && np == n))) {
+            // each pair reads its own rule
+            if (active) {
+                const int per = (np + W - 1) / W, k1 = min((wave + 1) * per, np);
+                for (int k = wave * per + sub; k < k1; k += G) {
+                    const double2 px = *reinterpret_cast<const double2 *>(a.tpts + 2 * ((int64_t)toff + k));
+                    const double2 py = *reinterpret_cast<const double2 *>(a.spts + 2 * ((int64_t)soff + k));
+                    point(px.x, px.y, py.x, py.y, a.wts[(int64_t)woff + k]);
+                }
+            }
+            return;
+        }
+        const int per = (n + W - 1) / W, k0 = min(wave * per, n), k1 = min(k0 + per, n);
+        for (int kb = k0; kb < k1; kb += Shared::kChunk) {
+            const int count = min(Shared::kChunk, k1 - kb);
+            // the wave's own part of LDS: its accesses complete in order, no barrier
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            double2 xt[Shared::kLoads], xs[Shared::kLoads];
+            double xw[Shared::kLoads];
+#pragma unroll
+            for (int u = 0; u < Shared::kLoads; ++u) {
+                const int64_t kk = kb + min(64 * u + lane, count - 1);
+                xt[u] = *reinterpret_cast<const double2 *>(a.tpts + 2 * (to + kk));
+                xs[u] = *reinterpret_cast<const double2 *>(a.spts + 2 * (so + kk));
+                xw[u] = a.wts[wo + kk];
+            }
+#pragma unroll
+            for (int u = 0; u < Shared::kLoads; ++u) {
+                sh.st.points[wave][64 * u + lane][0] = xt[u];
+                sh.st.points[wave][64 * u + lane][1] = xs[u];
+                sh.st.weights[wave][64 * u + lane] = xw[u];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (!active) continue;
+#pragma unroll 2
+            for (int k = sub; k < count; k += G) {
+                const double2 px = sh.st.points[wave][k][0], py = sh.st.points[wave][k][1];
+                point(px.x, px.y, py.x, py.y, sh.st.weights[wave][k]);
             }
         }
     };
@@ -240,14 +263,22 @@ __global__ __launch_bounds__(64 * W, W == 4 && !(DUAL && NTS * NSS == 9) ? 3 : 2
 
 // Lanes of a wave per pair (G) and waves (W): the points of a pair are split W G ways. The coincident
 // pairs' lanes form the longest chain (1536 / (W G) points), a split costs the set-up of more workgroups.
-// Kernel times with (W, G) = (4, 1) / (4, 4) / (8, 2) / (8, 16), against lanes striding over a pair's
+// Few pairs also leave waves whose pairs follow several rules; one rule after the other, with the other
+// lanes idle, doubled and more the longest chain (6,400 pairs, electric field, (4, 4): 54 against 32 us).
+// Kernel times with (W, G) = (4, 1) / (4, 4) / (4, 8) / (4, 16), against lanes striding over a pair's
 // points with loads of their own before:
-//   266,000 pairs, Helmholtz single + double layer P1:   737 / 866 / 1006 us   (before 1117)
-//    66,500 pairs, electric field operator:              179 / 160 /  203 us   (305)
-//    43,900 pairs, Helmholtz double layer P1, FP64:      163 / 126 /  164 us   (207)
-//    16,600 pairs, Laplace DP0, FP64:                     62 /  27 /   31 us   (29)
-//     1,000 pairs, Laplace P1, FP64:                       - /  - /    - / 9 us (14)
-constexpr int kSingLargePairs = 131072, kSingSmallPairs = 4096;
+//   203,800 pairs, Helmholtz double layer P1, FP64:     430 / 464 / 526 / 720 us
+//    66,500 pairs, the same:                            165 / 157 / 174 / 257 us
+//    12,700 pairs, the same:                             96 /  41 /  43 /  58 us
+//     6,400 pairs, the same:                            103 /  34 /  30 /  36 us
+//     2,300 pairs, the same:                            104 /  33 /  22 /  21 us
+//   203,800 pairs, electric field operator:             382 / 447 / 492 / 729 us
+//    66,500 pairs, the same:                            135 / 149 / 168 / 244 us (305)
+//     6,400 pairs, Helmholtz DP0, FP64, damped:         112 /  37 /  27 /  27 us (55)
+//     2,300 pairs, Laplace DP0, FP64:                    52 /  18 /  13 /   9 us
+// The electric field operator's local blocks take longer (one lane per pair and entry), so that it
+// prefers many pairs per wave earlier.
+constexpr int kSingLargePairs = 131072, kSingLargePairsEfie = 49152, kSingMediumPairs = 10240, kSingSmallPairs = 3072;
 
 template <int OP, typename OutT, bool DUAL, int W, int G>
 static int launch_sing_split(const SingularArgs &a, hipStream_t s) {
@@ -278,9 +309,11 @@ static int launch_sing_split(const SingularArgs &a, hipStream_t s) {
 template <int OP, typename OutT, bool DUAL>
 static int launch_sing(const SingularArgs &a, hipStream_t s) {
     if (a.n_pairs == 0) return BEM_OK;
-    if (a.n_pairs >= kSingLargePairs) return launch_sing_split<OP, OutT, DUAL, 4, 1>(a, s);
-    if (a.n_pairs >= kSingSmallPairs) return launch_sing_split<OP, OutT, DUAL, 4, 4>(a, s);
-    return launch_sing_split<OP, OutT, DUAL, 8, 16>(a, s);
+    if (a.n_pairs >= (OP == kMaxwellEFIE ? kSingLargePairsEfie : kSingLargePairs))
+        return launch_sing_split<OP, OutT, DUAL, 4, 1>(a, s);
+    if (a.n_pairs >= kSingMediumPairs) return launch_sing_split<OP, OutT, DUAL, 4, 4>(a, s);
+    if (a.n_pairs >= kSingSmallPairs) return launch_sing_split<OP, OutT, DUAL, 4, 8>(a, s);
+    return launch_sing_split<OP, OutT, DUAL, 4, 16>(a, s);
 }
 
 template <int OP, bool DUAL = false>

@@ -7,12 +7,13 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-# 3, 63 and 4,095 pairs: the smallest launches and their last workgroup; 4,096 to 15,777: the split of
-# medium launches (16 pairs per workgroup, remainder 1); 131,073: one lane per pair (64 pairs, remainder 1)
+# 3, 63 and 3,071 pairs: the smallest launches and their last workgroup (4 pairs, remainder 3); 3,072 to
+# 10,239: 8 pairs per workgroup; 10,241: 16 pairs, remainder 1; 49,153 (electric field) and 131,073: one lane per pair (64 pairs,
+# remainder 1)
 @pytest.mark.parametrize("op,space,k", [("laplace_single_layer", "P1", 0.0), ("helmholtz_double_layer", "DP0", 2.0),
                                         ("helmholtz_hypersingular", "P1", 2.0 + 0.3j),
                                         ("maxwell_electric_field", "RWG", 3.0)])
-@pytest.mark.parametrize("count", [3, 63, 4095, 4096, 15777, 131073])
+@pytest.mark.parametrize("count", [3, 63, 3071, 3072, 4095, 4096, 10239, 10241, 15777, 49153, 131073])
 def test_singular_pairs_in_any_order(op, space, k, count, hip_available):
     """A table of `count` pairs gives the same sum whether the pairs of one rule stand together (every
     wave reads one set of points) or the table is shuffled (every wave runs many rules)."""
