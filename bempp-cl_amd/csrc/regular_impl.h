@@ -97,7 +97,7 @@ struct TestTile {
     ET ee[EF ? TM : 1][2][3];
     ET el[EF ? TM : 1][3];
     ET ej[EF ? TM : 1];
-    ET en[EF && sizeof(ET) == 8 ? TM : 1][3];  // normal times the normal multiplier
+    ET en[EF && sizeof(ET) == 8 ? TM : 0][3];  // normal times the normal multiplier
 };
 
 // test elements staged per SYM work item (a run of test tiles)
@@ -770,13 +770,18 @@ __device__ __forceinline__ void store_direct(void *out, int64_t ld, int row, int
 // adds the transpose afterwards: S_fe = S_ef^T); with DUAL also its double-layer block to a.out2
 // at (e, f) and the double layer of the reversed pair (test normal) to a.out2 at (f, e) (REV).
 // waves per SIMD the launch bound asks for: the FP32 fused pass and the symmetric single layer
-// fit 3; the symmetric single + double layer pass and the mixed EFIE passes (ordered and
-// symmetric) keep more state (2);
+// fit 3, the real symmetric single + double layer pass too; the complex one and the mixed EFIE passes
+// (ordered and symmetric) keep more state (2);
 // the single-operator FP64 passes, ordered or symmetric, 2 (their few spills lie outside the
 // point-pair loops); the others leave it to the compiler
-template <int OP, bool MIXED, bool DUAL, bool SYM>
+template <int OP, bool MIXED, bool DUAL, bool SYM, bool KAHAN, int QT, typename OutT>
 constexpr int regular_waves() {
-    return !MIXED ? (DUAL ? 1 : 2) : SYM ? (DUAL || is_rwg_op<OP>() ? 2 : 3) : DUAL ? 3 : is_rwg_op<OP>() ? 2 : 1;
+    if (!MIXED) return DUAL && QT > 0 ? 1 : 2;
+    if (!SYM) return DUAL ? 3 : is_rwg_op<OP>() ? 2 : 1;
+    if (DUAL) return OpTraits<OP>::is_complex || KAHAN ? 2 : 3;
+    // LDS allows five workgroups a CU; 98 registers would leave four (2,880 triangles: 111 -> 130 us)
+    if (OP == kLaplaceHS && QT > 0 && sizeof(OutT) == 4) return 5;
+    return is_rwg_op<OP>() ? 2 : 3;
 }
 
 // UPPER (direct DP0 stores, a symmetric operator on one space): only the pairs whose trial element
@@ -785,7 +790,7 @@ constexpr int regular_waves() {
 // ORB: a.rule is a 6-point rule in orbit order (orbit_rule); the FP32 pairs use the orbit moments.
 template <int OP, int NTS, int NSS, int QT, int TM, bool MIXED, bool KAHAN, bool TILE, int MAXU_T, int MAXU_S,
           typename OutT, bool DUAL = false, bool SYM = false, bool UPPER = false, bool ORB = false>
-__global__ __launch_bounds__(kRegThreads, (regular_waves<OP, MIXED, DUAL, SYM>())) void regular_kernel(
+__global__ __launch_bounds__(kRegThreads, (regular_waves<OP, MIXED, DUAL, SYM, KAHAN, QT, OutT>())) void regular_kernel(
     const RegularArgs a) {
     static_assert(!SYM || TILE, "the symmetric pass is tiled");
     // REV: the double layer of the reversed pair (symmetric single + double layer pass)
@@ -816,11 +821,13 @@ __global__ __launch_bounds__(kRegThreads, (regular_waves<OP, MIXED, DUAL, SYM>()
     static_assert(!MFX || (MIXED && TILE && !DUAL && NTS == 3 && NSS == 3), "the tiled MFIE pass is mixed precision");
     // EFD, HSD: the same blocks in FP64, once per pair (local_value derives edge lengths and edge products
     // anew for each of the 9 entries, 24 square roots a pair for the EFIE); the trial side's edge data in
-    // LDS. EFIE, 1,620 triangles: regular kernel 441 -> 336 us
-    constexpr bool EFD = OP == kMaxwellEFIE && !MIXED && TILE;
-    constexpr bool HSD = is_hypersingular<OP>() && !MIXED && TILE;
+    // LDS. EFIE, 1,620 triangles: regular kernel 441 -> 336 us. Rules of any number of points (QT = 0)
+    // stage more test points, and the edge data would leave one workgroup per CU instead of two
+    constexpr bool EFD = OP == kMaxwellEFIE && !MIXED && TILE && QT > 0;
+    constexpr bool HSD = is_hypersingular<OP>() && !MIXED && TILE && QT > 0;
     constexpr bool EDGES = EFX || HSX || MFX || EFD || HSD;
-    __shared__ TestTile<TMC, MIXED ? 1 : TMC, QC, EDGES, typename std::conditional<MIXED, float, double>::type> T_;
+    using EdgeT = typename std::conditional<MIXED || !EDGES, float, double>::type;
+    __shared__ TestTile<TMC, MIXED ? 1 : TMC, QC, EDGES, EdgeT> T_;
     // EFD, HSD: edge vectors, edge lengths (HSD: normal times nm) and 1 / J (HSD: nm / J) of the lane's element
     __shared__ double trial_edges[EFD || HSD ? 10 : 1][EFD || HSD ? kRegThreads : 1];
     __shared__ AccT acc[TILE ? MAXU_T * MAXU_S * NC : 1];
