@@ -526,28 +526,41 @@ struct SingularPair {
     int64_t base;
 };
 
-// visit this lane's points: f(weight / r, r)
-template <typename F>
+// Lanes per pair (W) in the moments mode. The sums over the lanes cost log2 W shuffle steps for 64 / W pairs
+// at once, and the lanes of a pair share the wavenumbers; few pairs need more lanes each to fill the chip.
+// Kernel times, against a wavefront per pair with square root and division before:
+//    pairs    W = 8 / 16 / 32 / 64   (before), us, 32 wavenumbers
+//    66,500     213 / 227 / 277 / 362  (357)
+//    37,400     130 / 131 / 153 / 196  (186)
+//    21,000      87 /  78 /  89 / 112  (111)
+//    12,700      61 /  49 /  51 /  65  (77)
+//     6,400      59 /  33 /  30 /  36  (45)
+//     2,300      41 /  23 /  17 /  16  (18)
+constexpr int kSingPairs8 = 32768, kSingPairs16 = 10240, kSingPairs32 = 2560;
+
+// visit this lane's points (lanes of a group of W): f(weight / r, r)
+template <int W, typename F>
 __device__ __forceinline__ void singular_points(const SingularPair &P, int lane, F &&f) {
     const double *gt = P.gt, *gf = P.gf;
-    for (int kk = lane; kk < P.np; kk += 64) {
-        const double xi0 = P.tp[2 * kk], xi1 = P.tp[2 * kk + 1];
-        const double et0 = P.sp[2 * kk], et1 = P.sp[2 * kk + 1];
-        const double dx = (gf[0] + gf[3] * et0 + gf[6] * et1) - (gt[0] + gt[3] * xi0 + gt[6] * xi1);
-        const double dy = (gf[1] + gf[4] * et0 + gf[7] * et1) - (gt[1] + gt[4] * xi0 + gt[7] * xi1);
-        const double dz = (gf[2] + gf[5] * et0 + gf[8] * et1) - (gt[2] + gt[5] * xi0 + gt[8] * xi1);
-        const double r = sqrt(dx * dx + dy * dy + dz * dz);
-        f(P.w[kk] / r, r);
+#pragma unroll 2
+    for (int kk = lane; kk < P.np; kk += W) {
+        const double2 x = reinterpret_cast<const double2 *>(P.tp)[kk], y = reinterpret_cast<const double2 *>(P.sp)[kk];
+        const double dx = (gf[0] + gf[3] * y.x + gf[6] * y.y) - (gt[0] + gt[3] * x.x + gt[6] * x.y);
+        const double dy = (gf[1] + gf[4] * y.x + gf[7] * y.y) - (gt[1] + gt[4] * x.x + gt[7] * x.y);
+        const double dz = (gf[2] + gf[5] * y.x + gf[8] * y.y) - (gt[2] + gt[5] * x.x + gt[8] * x.y);
+        const double r2 = dx * dx + dy * dy + dz * dz, rinv = rsqrt_t(r2);
+        f(P.w[kk] * rinv, r2 * rinv);
     }
 }
 
-// mixed mode: moments about rc = (diam_e + diam_f) / 2, the centre of the distance range
-template <int NM, typename OutT>
+// mixed mode: moments about rc = (diam_e + diam_f) / 2, the centre of the distance range; lane: within the
+// pair's W lanes
+template <int W, int NM, typename OutT>
 __device__ __forceinline__ void singular_pair_moments(const Args &a, const SingularPair &P, int lane, double rc) {
     double c[NM + 1];
 #pragma unroll
     for (int n = 0; n <= NM; ++n) c[n] = 0.0;
-    singular_points(P, lane, [&](double g, double r) {
+    singular_points<W>(P, lane, [&](double g, double r) {
         const double dl = r - rc;
         double pw = g;
 #pragma unroll
@@ -557,15 +570,25 @@ __device__ __forceinline__ void singular_pair_moments(const Args &a, const Singu
         }
     });
 #pragma unroll
-    for (int n = 0; n <= NM; ++n) c[n] = wave_sum64(c[n]);
+    for (int n = 0; n <= NM; ++n)
+#pragma unroll
+        for (int off = W / 2; off >= 1; off >>= 1) c[n] += __shfl_xor(c[n], off, W);
     scale_factorials<NM>(c, P.scale);
-    // lane m evaluates wavenumber m
-    for (int km = lane; km < a.nk; km += 64) {
-        const double k = a.k[km];
+    // lane m evaluates the wavenumbers m, m + W, ...; the two parts of a value go to memory from
+    // neighbouring lanes (one atomic request)
+    for (int k0 = 0; k0 < a.nk; k0 += W) {
+        const double k = a.k[min(k0 + lane, a.nk - 1)];
         double re, im, s, cs;
         taylor_eval<NM>(c, k, re, im);
         sincos_fast(k * rc, &s, &cs);
-        add_c(a.out, km * a.kstride + P.base, (OutT)(cs * re - s * im), (OutT)(cs * im + s * re));
+        const OutT vr = (OutT)(cs * re - s * im), vi = (OutT)(cs * im + s * re);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int src = h * (W / 2) + lane / 2, km = k0 + src;
+            const OutT pr = __shfl(vr, src, W), pi = __shfl(vi, src, W);
+            if (km < a.nk && P.np > 0)
+                atomic_add(reinterpret_cast<OutT *>(a.out) + 2 * (km * a.kstride + P.base) + (lane & 1), lane & 1 ? pi : pr);
+        }
     }
 }
 
@@ -574,7 +597,7 @@ __device__ __forceinline__ void singular_pair_direct(const Args &a, const Singul
     for (int km = 0; km < a.nk; ++km) {
         const double k = a.k[km];
         double sr = 0.0, si = 0.0;
-        singular_points(P, lane, [&](double g, double r) {
+        singular_points<64>(P, lane, [&](double g, double r) {
             double s, c;
             sincos_fast(k * r, &s, &c);
             sr += c * g;
@@ -586,15 +609,8 @@ __device__ __forceinline__ void singular_pair_direct(const Args &a, const Singul
     }
 }
 
-// one wavefront per pair; MOMENTS: mixed-mode expansion, otherwise direct FP64 evaluation
-template <bool MOMENTS, typename OutT>
-__global__ __launch_bounds__(256) void kbatch_singular_kernel(const Args a, int n_pairs, const int32_t *pd_all,
-                                                              const double *tpts, const double *spts,
-                                                              const double *wts) {
-    const int lane = threadIdx.x & 63;
-    const int pair = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (pair >= n_pairs) return;  // uniform per wavefront
-    const int32_t *pd = pd_all + 6 * (int64_t)pair;
+__device__ __forceinline__ SingularPair singular_pair(const Args &a, const int32_t *pd, const double *tpts,
+                                                      const double *spts, const double *wts) {
     const int e = pd[0], f = pd[1];
     SingularPair P;
     P.gt = a.test.geom + (int64_t)e * BEM_GEOM_STRIDE;
@@ -605,21 +621,62 @@ __global__ __launch_bounds__(256) void kbatch_singular_kernel(const Args a, int 
     P.np = pd[5];
     P.scale = P.gt[12] * P.gf[12] * kInv4Pi * a.test.mult[e] * a.trial.mult[f];
     P.base = (int64_t)a.test.l2g[e] * a.ld + a.trial.l2g[f];
-    if constexpr (MOMENTS) {
-        // any two points of triangles sharing a vertex are at most diam_e + diam_f apart
-        const double rc = 0.5 * (P.gt[13] + P.gf[13]);
-        const int N = taylor_order(a.kmax * rc * 1.0001, kTolMoments, 32);
-        const int bucket = __builtin_amdgcn_readfirstlane(N <= 8 ? 0 : N <= 16 ? 1 : N <= 24 ? 2 : N <= 32 ? 3 : 4);
-        switch (bucket) {
-        case 0: singular_pair_moments<8, OutT>(a, P, lane, rc); break;
-        case 1: singular_pair_moments<16, OutT>(a, P, lane, rc); break;
-        case 2: singular_pair_moments<24, OutT>(a, P, lane, rc); break;
-        case 3: singular_pair_moments<32, OutT>(a, P, lane, rc); break;
-        default: singular_pair_direct<OutT>(a, P, lane); break;
+    return P;
+}
+
+// direct evaluation, one wavefront per pair
+template <typename OutT>
+__global__ __launch_bounds__(256) void kbatch_singular_direct_kernel(const Args a, int n_pairs, const int32_t *pd_all,
+                                                                     const double *tpts, const double *spts,
+                                                                     const double *wts) {
+    const int lane = threadIdx.x & 63;
+    const int pair = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (pair >= n_pairs) return;  // uniform per wavefront
+    singular_pair_direct<OutT>(a, singular_pair(a, pd_all + 6 * (int64_t)pair, tpts, spts, wts), lane);
+}
+
+// mixed-mode expansion, W lanes per pair
+template <int W>
+__global__ __launch_bounds__(256) void kbatch_singular_kernel(const Args a, int n_pairs, const int32_t *pd_all,
+                                                              const double *tpts, const double *spts,
+                                                              const double *wts) {
+    const int lane = threadIdx.x % W;
+    const int pair = (int)(((int64_t)blockIdx.x * 256 + threadIdx.x) / W);
+    // lanes without a pair stay with the wave (its order is uniform) and take the last pair's geometry and no points
+    SingularPair P = singular_pair(a, pd_all + 6 * (int64_t)min(pair, n_pairs - 1), tpts, spts, wts);
+    if (pair >= n_pairs) P.np = 0;
+    // any two points of triangles sharing a vertex are at most diam_e + diam_f apart
+    const double rc = 0.5 * (P.gt[13] + P.gf[13]);
+    const int N = wave_max64(taylor_order(a.kmax * rc * 1.0001, kTolMoments, 32));
+    const int bucket = __builtin_amdgcn_readfirstlane(N <= 8 ? 0 : N <= 16 ? 1 : N <= 24 ? 2 : N <= 32 ? 3 : 4);
+    switch (bucket) {
+    case 0: singular_pair_moments<W, 8, float>(a, P, lane, rc); break;
+    case 1: singular_pair_moments<W, 16, float>(a, P, lane, rc); break;
+    case 2: singular_pair_moments<W, 24, float>(a, P, lane, rc); break;
+    case 3: singular_pair_moments<W, 32, float>(a, P, lane, rc); break;
+    default:
+        // the wave's pairs one after the other, with all its lanes
+        for (int q = 0; q < 64 / W; ++q) {
+            const int64_t p = (int64_t)blockIdx.x * (256 / W) + (threadIdx.x >> 6) * (64 / W) + q;
+            if (p >= n_pairs) break;  // uniform per wavefront
+            singular_pair_direct<float>(a, singular_pair(a, pd_all + 6 * p, tpts, spts, wts), threadIdx.x & 63);
         }
-    } else {
-        singular_pair_direct<OutT>(a, P, lane);
     }
+}
+
+template <int W>
+void launch_singular_lanes(const Args &a, int n, const int32_t *pairs, const double *tpts, const double *spts,
+                           const double *wts, hipStream_t s) {
+    const dim3 grid((unsigned)(((int64_t)n * W + 255) / 256));
+    hipLaunchKernelGGL(kbatch_singular_kernel<W>, grid, dim3(256), 0, s, a, n, pairs, tpts, spts, wts);
+}
+
+void launch_singular(const Args &a, int n, const int32_t *pairs, const double *tpts, const double *spts,
+                     const double *wts, hipStream_t s) {
+    if (n >= kSingPairs8) return launch_singular_lanes<8>(a, n, pairs, tpts, spts, wts, s);
+    if (n >= kSingPairs16) return launch_singular_lanes<16>(a, n, pairs, tpts, spts, wts, s);
+    if (n >= kSingPairs32) return launch_singular_lanes<32>(a, n, pairs, tpts, spts, wts, s);
+    launch_singular_lanes<64>(a, n, pairs, tpts, spts, wts, s);
 }
 
 }  // namespace kb
@@ -730,13 +787,11 @@ extern "C" int bem_kbatch_assemble(const bem_space_t *test, const bem_space_t *t
         if ((rc = check_launch("kbatch_near_kernel"))) return rc;
     }
     if ((parts & BEM_KBATCH_SINGULAR) && n_singular > 0) {
-        const dim3 grid((n_singular + 3) / 4);
         if (mixed)
-            hipLaunchKernelGGL((kb::kbatch_singular_kernel<true, float>), grid, dim3(256), 0, s, a, n_singular,
-                               singular_pairs, test_points, trial_points, weights);
+            kb::launch_singular(a, n_singular, singular_pairs, test_points, trial_points, weights, s);
         else
-            hipLaunchKernelGGL((kb::kbatch_singular_kernel<false, double>), grid, dim3(256), 0, s, a, n_singular,
-                               singular_pairs, test_points, trial_points, weights);
+            hipLaunchKernelGGL((kb::kbatch_singular_direct_kernel<double>), dim3((n_singular + 3) / 4), dim3(256), 0, s, a,
+                               n_singular, singular_pairs, test_points, trial_points, weights);
         if ((rc = check_launch("kbatch_singular_kernel"))) return rc;
     }
     return BEM_OK;

@@ -169,3 +169,41 @@ def test_autotuner_caches_choice(dp0, default_parameters, tmp_path, monkeypatch,
     fixed = hip_kbatch_assemble(dp0, dp0, ks, "single", parameters=default_parameters, config=cfg).cpu().numpy()
     assert np.array_equal(tuned, fixed)
     autotune.clear_memory()
+
+
+# 3 and 2,559 pairs: a wavefront per pair; 2,561 to 10,239: 32 lanes (remainders 1 and 7 of 8 pairs per
+# workgroup); 10,241: 16 lanes; 32,769: 8 lanes (32 pairs per workgroup, remainder 1)
+@pytest.mark.parametrize("count", [3, 2559, 2561, 10239, 10241, 32769])
+@pytest.mark.parametrize("ks", [np.linspace(0.1, 0.5, 3), np.linspace(0.5, 8.0, 19)], ids=["3k", "19k"])
+def test_singular_part_of_any_size(count, ks, hip_available):
+    """The singular pairs of a mixed sweep against one FP64 assembly per wavenumber, in shuffled order."""
+    import torch
+
+    from bempp_amd.api import function_space
+    from bempp_amd.api.grid.shapes import icosphere
+    from bempp_amd.core import hip_backend as hb
+    from bempp_amd.api.integration.triangle_gauss import rule as triangle_rule
+    from bempp_amd.core.singular_assembler import singular_rule
+
+    grid = icosphere(3 if count <= 15000 else 4)
+    sp = function_space(grid, "DP", 0)
+    rule = singular_rule(grid, 4, sp.support, sp.support)
+    chosen = np.random.default_rng(count).permutation(len(rule.host.pairs))[:count]
+    n = sp.global_dof_count
+
+    class Part:
+        pairs = torch.from_numpy(np.ascontiguousarray(rule.host.pairs[chosen])).to(hb.device())
+        test_points, trial_points, weights = rule.test_points, rule.trial_points, rule.weights
+
+    ds = hb.device_space(sp)
+    out = torch.zeros((len(ks), n, n), dtype=torch.complex64, device=hb.device())
+    points, weights = triangle_rule(4)
+    hb.kbatch_assemble(ds, ds, True, hb.quad_rule(points, weights), ks, hb.PRECISION_MIXED, 2.0, (16, 4), out,
+                       singular=Part, parts=hb.KBATCH_SINGULAR)
+    for m, k in enumerate(ks):
+        ref = torch.zeros((n, n), dtype=torch.complex128, device=hb.device())
+        hb.singular_assemble("helmholtz_single_layer", ds, ds, Part.pairs, Part.test_points, Part.trial_points,
+                             Part.weights, k, ref)
+        assert torch.linalg.norm(ref) > 0
+        # one rounding to FP32 per entry, and the moments' 1e-10
+        assert torch.linalg.norm(out[m].to(torch.complex128) - ref) < (2.0**-24 + 1e-9) * torch.linalg.norm(ref)
