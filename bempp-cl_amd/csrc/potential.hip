@@ -138,14 +138,15 @@ __device__ __forceinline__ void tile_extent_stage(double y2, double *wmax) {
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = y2;
 }
 
-// Wave-uniform: a real wavenumber and |k| (|x| + max |y|) < 2^25 for every active lane's target x
-// over the tile's sources, so every phase |k r| (r <= |x| + |y|) or |k xh.y| takes the branch-free
-// reduction (kPhReduced | kPhReal).
-__device__ __forceinline__ bool tile_phase_reduced(double kr, double ki, double xnorm, const double *wmax) {
+// Wave-uniform: |Re k| (|x| + max |y|) < 2^25 for every active lane's target x over the tile's sources,
+// so every phase |k r| (r <= |x| + |y|) or |k xh.y| takes the branch-free reduction (kPhReduced; damped
+// wavenumbers keep their exponential: 320 triangles, 1,791 points, electric field:
+// 194 -> 29 us together with the split chunks).
+__device__ __forceinline__ bool tile_phase_reduced(double kr, double xnorm, const double *wmax) {
     double y2 = wmax[0];
 #pragma unroll
     for (int w = 1; w < kPotThreads / 64; ++w) y2 = fmax(y2, wmax[w]);
-    return ki == 0.0 && __all(fabs(kr) * (xnorm + sqrt(y2)) < 0x1p25);
+    return __all(fabs(kr) * (xnorm + sqrt(y2)) < 0x1p25);
 }
 
 // One source's FP64 contribution to the potential at x (the body of potential_eval_fp64, also the
@@ -274,8 +275,11 @@ __global__ __launch_bounds__(kPotThreads) void potential_eval_fp64(const PotArgs
             for (int j = 0; j < nt; ++j)
                 fp64_source<OP, PH>([&](int k) { return sh[k][j]; }, x0, x1, x2, kr, ki, alr, ali, accr, acci);
         };
-        if (OpTraits<OP>::is_complex && tile_phase_reduced(kr, ki, xnorm, wmax))
+        const bool reduced = OpTraits<OP>::is_complex && tile_phase_reduced(kr, xnorm, wmax);
+        if (reduced && ki == 0.0)
             sources(std::integral_constant<int, kPhReduced | kPhReal>{});
+        else if (reduced)
+            sources(std::integral_constant<int, kPhReduced>{});
         else
             sources(std::integral_constant<int, 0>{});
     }
@@ -795,8 +799,11 @@ __global__ __launch_bounds__(kPotThreads) void far_field_eval_fp64(const PotArgs
             }
         }
         };
-        if (tile_phase_reduced(kr, ki, xnorm, wmax))
+        const bool reduced = tile_phase_reduced(kr, xnorm, wmax);
+        if (reduced && ki == 0.0)
             sources(std::integral_constant<int, kPhReduced | kPhReal>{});
+        else if (reduced)
+            sources(std::integral_constant<int, kPhReduced>{});
         else
             sources(std::integral_constant<int, 0>{});
     }
@@ -1091,7 +1098,13 @@ __global__ __launch_bounds__(256) void potential_reduce_kernel(const PotArgs a, 
     o[2 * (int64_t)i + 1] = (OutT)si;
 }
 
-static void plan(int npts, int nsrc, int *nchunk, int *chunk_len, int *nsrc_pad) {
+// Chunks of the sources: whole tiles for at least 4,096 workgroups where there are that many. In FP64, where
+// a lane's chain of sources is long, launches that leave less than 4 workgroups per CU that way split their
+// tiles (down to 32 sources): electric field, 390 triangles, 3,251 points 75 -> 40 us; Laplace, 720
+// triangles, 500 points 19 -> 8 us. With 1,024 workgroups or more the whole tiles are as fast.
+constexpr int kPotSplitWorkgroups = 1024;
+
+static void plan(int npts, int nsrc, int precision, int *nchunk, int *chunk_len, int *nsrc_pad) {
     *nsrc_pad = ((nsrc + kPotTile - 1) / kPotTile) * kPotTile;
     const int tblocks = max(1, (npts + kPotThreads - 1) / kPotThreads);  // no points: one block's plan
     const int ntiles = max(1, *nsrc_pad / kPotTile);                     // no sources: one empty chunk
@@ -1101,6 +1114,8 @@ static void plan(int npts, int nsrc, int *nchunk, int *chunk_len, int *nsrc_pad)
     if (want < 1) want = 1;
     int tiles_per_chunk = (ntiles + want - 1) / want;
     *chunk_len = tiles_per_chunk * kPotTile;
+    if (precision != BEM_PRECISION_MIXED && tiles_per_chunk == 1)
+        while (*chunk_len > 32 && (int64_t)tblocks * (*nsrc_pad / *chunk_len) < kPotSplitWorkgroups) *chunk_len /= 2;
     *nchunk = (*nsrc_pad + *chunk_len - 1) / *chunk_len;
 }
 
@@ -1172,10 +1187,10 @@ using namespace bem;
 
 extern "C" size_t bem_potential_workspace_size(int op, const bem_space_t *space, const bem_quad_rule_t *rule,
                                                int n_points, int precision) {
-    (void)precision;
     if (!space || !rule || n_points < 0) return 0;
     int nsrc = space->n_elements * rule->n_points, nchunk, chunk_len, nsrc_pad;
-    plan(n_points, nsrc, &nchunk, &chunk_len, &nsrc_pad);
+    (void)precision;  // one size for both: the FP64 plan has at least as many chunks
+    plan(n_points, nsrc, BEM_PRECISION_FP64, &nchunk, &chunk_len, &nsrc_pad);
     int kd = is_vector_potential_op(op) ? 3 : 1;
     return sizeof(double) * ((size_t)kSrcFields * nsrc_pad + (size_t)2 * nchunk * kd * n_points) + 256;
 }
@@ -1223,7 +1238,7 @@ static int potential_evaluate(int op, const bem_space_t *space, const void *coef
     a.kr = (op == BEM_LAPLACE_SINGLE_LAYER || op == BEM_LAPLACE_DOUBLE_LAYER) ? 0.0 : k_re;
     a.ki = (op == BEM_LAPLACE_SINGLE_LAYER || op == BEM_LAPLACE_DOUBLE_LAYER) ? 0.0 : k_im;
     a.nsrc = space->n_elements * rule->n_points;
-    plan(n_points, a.nsrc, &a.nchunk, &a.chunk_len, &a.nsrc_pad);
+    plan(n_points, a.nsrc, precision, &a.nchunk, &a.chunk_len, &a.nsrc_pad);
     uintptr_t base = ((uintptr_t)workspace + 255) & ~(uintptr_t)255;
     a.src = (double *)base;
     a.partial = a.src + (size_t)kSrcFields * a.nsrc_pad;

@@ -1,0 +1,36 @@
+"""FP64 potentials of few points split the sources into chunks of less than a tile; many points do not."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# 320 triangles: 1,920 sources, 8 tiles of 256. 32,768 points fill the chip with whole tiles; 1 and 255 points
+# take chunks of 32, 2,049 points of 64, 16,385 points of 128 sources. 20 triangles: 120 sources, less than a tile
+@pytest.mark.parametrize("family,name,k", [("laplace", "double_layer", 0.0), ("helmholtz", "single_layer", 2.0),
+                                           ("helmholtz", "double_layer", 2.0 + 0.5j),
+                                           ("maxwell", "electric_field", 1.5 + 0.2j),
+                                           ("maxwell", "magnetic_field", 1.5)])
+@pytest.mark.parametrize("level", [0, 2])
+def test_few_points_equal_many(family, name, k, level, hip_available):
+    import bempp_amd.api as bempp
+    from bempp_amd.api.grid.shapes import icosphere
+
+    space = bempp.function_space(icosphere(level), *(("RWG", 0) if family == "maxwell" else ("DP", 0)))
+    rng = np.random.default_rng(level)
+    coefficients = rng.standard_normal(space.global_dof_count) + 1j * rng.standard_normal(space.global_dof_count)
+    fun = bempp.GridFunction(space, coefficients=coefficients)
+    points = rng.standard_normal((3, 262144 if level == 0 else 32768))
+    points *= rng.uniform(1.5, 3.0, points.shape[1]) / np.linalg.norm(points, axis=0)
+    make = getattr(getattr(bempp.operators.potential, family), name)
+
+    def evaluate(x):
+        options = () if family == "laplace" else (k,)
+        return make(space, np.ascontiguousarray(x), *options, precision="double").evaluate(fun)
+
+    many = evaluate(points)
+    for count in (1, 255, 2049, 16385):
+        few = evaluate(points[:, :count])
+        # the same terms summed in another grouping: about sqrt(1,920) roundings of terms that partly cancel
+        assert np.linalg.norm(few - many[:, :count]) < 1e-13 * np.linalg.norm(many[:, :count])
