@@ -1098,11 +1098,20 @@ __global__ __launch_bounds__(256) void potential_reduce_kernel(const PotArgs a, 
     o[2 * (int64_t)i + 1] = (OutT)si;
 }
 
-// Chunks of the sources: whole tiles for at least 4,096 workgroups where there are that many. In FP64, where
-// a lane's chain of sources is long, launches that leave less than 4 workgroups per CU that way split their
-// tiles (down to 32 sources): electric field, 390 triangles, 3,251 points 75 -> 40 us; Laplace, 720
-// triangles, 500 points 19 -> 8 us. With 1,024 workgroups or more the whole tiles are as fast.
-constexpr int kPotSplitWorkgroups = 1024;
+// Chunks of the sources: whole tiles for at least 4,096 workgroups where there are that many. Launches that
+// leave the chip idle that way (less than 4 workgroups per CU in FP64, where a lane's chain of sources is
+// long, 2 in mixed precision) split their tiles, down to 32 sources in FP64 and two reference groups in mixed
+// precision (the same groups: the same values up to the order of the chunk sums). Kernel times: FP64 electric
+// field, 390 triangles, 3,251 points 75 -> 40 us; Laplace, 720 triangles, 500 points 19 -> 8 us; whole calls in
+// mixed precision: electric field, 80 triangles, 11,938 points 261 -> 144 us, 1,620 triangles, 2,000 points
+// 228 -> 159 us. Beyond: 456 triangles, 11,869 points (517 workgroups, mixed) 159 us whole, 166 us split.
+constexpr int kPotSplitWorkgroups = 1024, kPotSplitWorkgroupsMixed = 512;
+
+// Scalar potentials of up to this many (point, source) pairs are evaluated in FP64 in either mode: the pairs
+// take less than the call's other launches (25 M pairs: 15 us Laplace, 40 us Helmholtz in FP64), and on meshes
+// that small the targets are close to the sources, where the FP32 path would be least accurate (720 triangles,
+// Laplace: 1.1e-7 against 3e-8 before, when most groups took the FP64 path one by one).
+constexpr int64_t kPotFp64Pairs = 3 << 23;
 
 static void plan(int npts, int nsrc, int precision, int *nchunk, int *chunk_len, int *nsrc_pad) {
     *nsrc_pad = ((nsrc + kPotTile - 1) / kPotTile) * kPotTile;
@@ -1114,8 +1123,10 @@ static void plan(int npts, int nsrc, int precision, int *nchunk, int *chunk_len,
     if (want < 1) want = 1;
     int tiles_per_chunk = (ntiles + want - 1) / want;
     *chunk_len = tiles_per_chunk * kPotTile;
-    if (precision != BEM_PRECISION_MIXED && tiles_per_chunk == 1)
-        while (*chunk_len > 32 && (int64_t)tblocks * (*nsrc_pad / *chunk_len) < kPotSplitWorkgroups) *chunk_len /= 2;
+    const bool mixed = precision == BEM_PRECISION_MIXED;
+    const int least = mixed ? 64 : 32, enough = mixed ? kPotSplitWorkgroupsMixed : kPotSplitWorkgroups;
+    if (tiles_per_chunk == 1)
+        while (*chunk_len > least && (int64_t)tblocks * (*nsrc_pad / *chunk_len) < enough) *chunk_len /= 2;
     *nchunk = (*nsrc_pad + *chunk_len - 1) / *chunk_len;
 }
 
@@ -1238,6 +1249,8 @@ static int potential_evaluate(int op, const bem_space_t *space, const void *coef
     a.kr = (op == BEM_LAPLACE_SINGLE_LAYER || op == BEM_LAPLACE_DOUBLE_LAYER) ? 0.0 : k_re;
     a.ki = (op == BEM_LAPLACE_SINGLE_LAYER || op == BEM_LAPLACE_DOUBLE_LAYER) ? 0.0 : k_im;
     a.nsrc = space->n_elements * rule->n_points;
+    if (!is_vector_potential_op(op) && !is_far_field_op(op) && (int64_t)a.nsrc * n_points <= kPotFp64Pairs)
+        precision = BEM_PRECISION_FP64;
     plan(n_points, a.nsrc, precision, &a.nchunk, &a.chunk_len, &a.nsrc_pad);
     uintptr_t base = ((uintptr_t)workspace + 255) & ~(uintptr_t)255;
     a.src = (double *)base;

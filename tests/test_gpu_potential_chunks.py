@@ -1,4 +1,4 @@
-"""FP64 potentials of few points split the sources into chunks of less than a tile; many points do not."""
+"""Potentials of few points split the sources into chunks of less than a tile; many points do not."""
 
 import numpy as np
 import pytest
@@ -34,3 +34,26 @@ def test_few_points_equal_many(family, name, k, level, hip_available):
         few = evaluate(points[:, :count])
         # the same terms summed in another grouping: about sqrt(1,920) roundings of terms that partly cancel
         assert np.linalg.norm(few - many[:, :count]) < 1e-13 * np.linalg.norm(many[:, :count])
+
+
+# 1,920 sources: 2,049 points take chunks of 64, 8,193 of 128 sources (electric field); scalar potentials of up
+# to 13,107 points (25,165,440 pairs) are evaluated in FP64, 13,108 in FP32
+@pytest.mark.parametrize("family,name,k", [("laplace", "double_layer", 0.0), ("helmholtz", "single_layer", 2.0),
+                                           ("maxwell", "electric_field", 1.5),
+                                           ("maxwell", "magnetic_field", 1.5 + 0.2j)])
+@pytest.mark.parametrize("count", [1, 2049, 8193, 13107, 13108])
+def test_mixed_against_fp64(family, name, k, count, hip_available):
+    import bempp_amd.api as bempp
+    from bempp_amd.api.grid.shapes import icosphere
+
+    space = bempp.function_space(icosphere(2), *(("RWG", 0) if family == "maxwell" else ("DP", 0)))
+    rng = np.random.default_rng(count)
+    fun = bempp.GridFunction(space, coefficients=1.0 + rng.random(space.global_dof_count))
+    points = rng.standard_normal((3, count))
+    points *= rng.uniform(1.5, 3.0, count) / np.linalg.norm(points, axis=0)
+    options = () if family == "laplace" else (k,)
+    make = getattr(getattr(bempp.operators.potential, family), name)
+    single, double = (make(space, points, *options, precision=p).evaluate(fun) for p in ("single", "double"))
+    # the mode's stated accuracy; a scalar call in FP64 rounds its output only
+    exact = family != "maxwell" and count * 1920 <= 3 << 23
+    assert np.linalg.norm(single - double) < (1e-7 if exact else 2e-6) * np.linalg.norm(double)
