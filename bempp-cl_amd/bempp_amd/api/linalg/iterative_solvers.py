@@ -82,6 +82,20 @@ def device_gmres(tensor, b, rtol=1e-5, restart=None, maxiter=None, callback=None
 def krylov_gmres(matvec, b, dev, rtol=1e-5, restart=None, maxiter=None, callback=None, matrix=None):
     """Restarted GMRES with the operator given as matvec (complex128 tensors on dev). matrix: the operator's
     row-major device matrix, if it has one: an Arnoldi step is then one library call."""
+    try:
+        return _krylov_gmres(matvec, b, dev, rtol, restart, maxiter, callback, matrix)
+    except BaseException:
+        # A step issued ahead of the host may still be copying into page-locked memory. torch's host
+        # allocator does not know of the library's copy and would hand the memory out again: wait
+        # here, where the exception's traceback still holds the buffers.
+        if dev.type == "cuda":
+            import torch
+
+            torch.cuda.synchronize(dev)
+        raise
+
+
+def _krylov_gmres(matvec, b, dev, rtol, restart, maxiter, callback, matrix):
     import torch
     from scipy.linalg import solve_triangular
 

@@ -479,7 +479,8 @@ def gmres_cgs2(V, k, w, out, v_next=None, eps=0.0):
 def gmres_stepper(A, V, w, out, host, eps):
     """step(k, b): one Arnoldi step of GMRES on the current stream in one library call (w = A V[k - 1], CGS2 of
     w against V[:k], next basis vector into V[k], the 2k + 2 coefficients into the page-locked tensor host[b]).
-    The checks are made and the addresses read once per solve; the function keeps the tensors alive."""
+    The checks are made and the addresses read once per solve; the function keeps the tensors alive. The copy
+    to host[b] is the library's: host memory of torch's allocator must stay alive until the stream has done it."""
     torch = _torch()
     n = V.shape[1]
     if A.shape != (n, n) or A.stride(1) != 1 or V.dtype != torch.complex128 or not V.is_contiguous():

@@ -295,3 +295,51 @@ def test_product_by_whole_rows(rows, cols, ld, dtype, hip_available):
     y = hb.dense_matvec(A, x)
     ref = A.to(torch.complex128) @ x
     assert torch.linalg.vector_norm(y - ref) < 1e-14 * cols**0.5 * torch.linalg.vector_norm(ref)
+
+
+def _delayed_stepper(monkeypatch, cycles):
+    """Each library step of GMRES behind `cycles` of device time."""
+    import torch
+
+    from bempp_amd.core import hip_backend as hb
+
+    make = hb.gmres_stepper
+
+    def delayed(*args):
+        step = make(*args)
+
+        def slow(k, b):
+            torch.cuda._sleep(cycles)
+            step(k, b)
+
+        return slow
+
+    monkeypatch.setattr(hb, "gmres_stepper", delayed)
+
+
+@pytest.mark.parametrize("stop_at", [1, 3])
+def test_gmres_left_by_an_exception_waits_for_its_copies(stop_at, monkeypatch, hip_available):
+    """A callback that raises leaves while the next step is in flight: its copy into page-locked memory is
+    finished before the exception reaches the caller, who frees that memory."""
+    import torch
+
+    from bempp_amd.api.linalg.iterative_solvers import device_gmres
+    from bempp_amd.core import hip_backend as hb
+
+    _delayed_stepper(monkeypatch, 20_000_000)  # about 10 ms each
+    rng = np.random.default_rng(0)
+    n, count = 60, 0
+    A = torch.from_numpy(np.eye(n) + 0.05 * rng.standard_normal((n, n))).to(hb.device())
+
+    class Stop(Exception):
+        pass
+
+    def callback(residual):
+        nonlocal count
+        count += 1
+        if count == stop_at:
+            raise Stop
+
+    with pytest.raises(Stop):
+        device_gmres(A, rng.standard_normal(n), rtol=1e-12, callback=callback)
+    assert torch.cuda.current_stream().query()
