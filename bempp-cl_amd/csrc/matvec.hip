@@ -10,7 +10,8 @@
 //  * op = N, 16-byte aligned rows: workgroups of 32 rows x 1024 columns; the x chunk is staged in
 //    LDS once per workgroup, each wavefront streams 8 rows with 16-byte loads (8 independent loads
 //    in flight per lane), and the column chunks' FP64 sums are combined with FP64 atomics.
-//  * op = N, 16-byte aligned rows, too few such tiles for the chip: one wavefront per one or two rows.
+//  * op = N, 16-byte aligned rows, too few such tiles for the chip and no wide matrix: one wavefront per
+//    one or two rows.
 //  * op = N otherwise: one wavefront per row; lanes read consecutive columns, x from L2.
 //  * op = T/C: each workgroup owns 256 consecutive columns and a band of rows; every lane
 //    walks its column down the band, and the band sums are added to y with FP64 atomics.
@@ -104,11 +105,21 @@ constexpr int kMvRows = 32;          // rows per workgroup
 constexpr int kMvRowsPerWave = 8;    // rows per wavefront
 constexpr int kMvCols = 1024;        // columns per workgroup (x chunk: 16 KB of LDS)
 
-// below this many 32 x 1024 tiles a wavefront takes whole rows instead (kMvSingleRows: one row each up to
-// here, else two): complex64, n = 1,002 12.5 -> 9.8 us (calls back to back), 2,562 14.6 -> 11.9,
-// 4,000 26.6 -> 21.3 us
+// below this many 32 x 1024 tiles a wavefront takes whole rows instead (one row each, or two above kSingleRows
+// rows, in FP32 earlier, where a 16-byte load of the matrix needs 64 bytes of x): complex64, n = 1,002
+// 9.8 -> 4.0 us, 2,562 14.6 -> 12.0, 4,000 26.4 -> 21.8, 5,120 38.9 -> 30.9 us
 constexpr int64_t kMvTiles = 1024;
-constexpr int64_t kMvSingleRows = 2048;
+
+template <typename AT>
+constexpr int64_t kSingleRows = sizeof(AT) == 4 ? 1024 : 2048;
+
+// Whole rows are rows / 4 workgroups whatever the number of columns, tiles share the columns too: matrices of
+// more than twice as many columns as rows keep their tiles, unless they are small (complex64, tiles against
+// whole rows: 32 x 1,000,000 193 against 3126 us, 256 x 20,480 14.8 against 54, 1,002 x 4,008 12.2 against
+// 14.1; 1,000 x 2,000 10.1 against 5.0, 256 x 4,096 9.8 against 6.9 us).
+inline bool whole_rows(int64_t rows, int64_t cols, int64_t ntiles) {
+    return ntiles < kMvTiles && (cols <= 2 * rows + 256 || (cols <= 4096 && ntiles <= 32));
+}
 
 // y_i += sum_{j in the chunk} A_ij x_j (y zeroed beforehand); rows start 16-byte aligned
 template <typename AT>
@@ -293,8 +304,8 @@ int launch(int trans, const void *A, int64_t rows, int64_t cols, int64_t ld, con
     const bool aligned = reinterpret_cast<uintptr_t>(A) % 16 == 0 && (ld * (int64_t)sizeof(AT)) % 16 == 0;
     const int64_t nchunks = (cols + kMvCols - 1) / kMvCols;
     const int64_t ntiles = (rows + kMvRows - 1) / kMvRows * nchunks;
-    if (trans == 0 && aligned && reinterpret_cast<uintptr_t>(x) % 16 == 0 && ntiles < kMvTiles) {
-        if (rows <= kMvSingleRows)
+    if (trans == 0 && aligned && reinterpret_cast<uintptr_t>(x) % 16 == 0 && whole_rows(rows, cols, ntiles)) {
+        if (rows <= kSingleRows<AT>)
             hipLaunchKernelGGL((matvec_n_rows_kernel<AT, 1>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, A, rows,
                                cols, ld, x, y);
         else

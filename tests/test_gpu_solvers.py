@@ -343,3 +343,57 @@ def test_gmres_left_by_an_exception_waits_for_its_copies(stop_at, monkeypatch, h
     with pytest.raises(Stop):
         device_gmres(A, rng.standard_normal(n), rtol=1e-12, callback=callback)
     assert torch.cuda.current_stream().query()
+
+
+def _product_error(A, x):
+    """|A x - ref| / |ref| against the FP64 product, the reference by chunks of columns."""
+    import torch
+
+    from bempp_amd.core import hip_backend as hb
+
+    ref = sum(A[:, c : c + 50000].to(torch.complex128) @ x[c : c + 50000] for c in range(0, A.shape[1], 50000))
+    return (torch.linalg.vector_norm(hb.dense_matvec(A, x) - ref) / torch.linalg.vector_norm(ref)).item()
+
+
+# tiles of 32 x 1,024: more than 1,023 of them (remainders of rows, columns and 16-byte loads); wide matrices of
+# fewer; the last shapes that take whole rows (1,022 tiles; 2 x rows + 256 columns; 32 tiles) and their
+# neighbours that do not
+@pytest.mark.parametrize("rows,cols", [(6001, 6003), (33, 600001), (64, 20480), (5, 70001), (4672, 7168), (4673, 7168),
+                                       (640, 1536), (640, 1537), (256, 4096), (257, 4096), (1024, 1030), (1025, 1030)])
+@pytest.mark.parametrize("dtype", ["float32", "float64", "complex64", "complex128"])
+def test_product_by_tiles_and_by_rows(rows, cols, dtype, hip_available):
+    import torch
+
+    from bempp_amd.core import hip_backend as hb
+
+    torch.manual_seed(rows)
+    A = torch.randn((rows, (cols + 7) // 4 * 4), dtype=getattr(torch, dtype), device=hb.device())[:, :cols]
+    x = torch.randn(cols, dtype=torch.complex128, device=hb.device())
+    # sums of cols FP64 products: rounding grows with the root of their number
+    assert _product_error(A, x) < 1e-15 * cols**0.5
+
+
+def test_product_of_a_wide_matrix_fills_the_chip(hip_available):
+    """32 rows x 1,000,000 columns: about twice the time of a copy of the matrix when the columns are shared among
+    workgroups, 30 times when every row is one wavefront's."""
+    import torch
+
+    from bempp_amd.core import hip_backend as hb
+
+    A = torch.randn((32, 1000000), dtype=torch.complex64, device=hb.device())
+    x = torch.randn(1000000, dtype=torch.complex128, device=hb.device())
+    B, y = torch.empty_like(A), torch.empty(32, dtype=torch.complex128, device=hb.device())
+
+    def best(f):
+        times = []
+        for _ in range(6):
+            start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            f()
+            stop.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(stop))
+        return min(times)
+
+    assert best(lambda: hb.dense_matvec(A, x, out=y)) < 8 * best(lambda: B.copy_(A))
+    assert _product_error(A, x) < 1e-15 * 1000000**0.5
