@@ -491,7 +491,7 @@ def gmres_stepper(A, V, w, out, host, eps):
     m = V.shape[0]
     if w.shape != (n,) or any(t.numel() < 2 * m for t in (*out, *host)):
         raise ValueError("w must have length n, out and host 2 * rows of V values")
-    fn, a, dtype, ld, v, wp, s = lib().bem_gmres_step, ptr(A), _dtype_code(A), A.stride(0), ptr(V), ptr(w), stream_handle()
+    fn, a, dtype, ld, v, wp = lib().bem_gmres_step, ptr(A), _dtype_code(A), A.stride(0), ptr(V), ptr(w)
     outs, hosts = [ptr(t) for t in out], [ptr(t) for t in host]
 
     keep = (A, V, w, tuple(out), tuple(host))
@@ -499,7 +499,8 @@ def gmres_stepper(A, V, w, out, host, eps):
     def step(k, b, keep=keep):
         if not 1 <= k < m:
             raise ValueError("k must leave a row of V for the next basis vector")
-        check(fn(a, dtype, n, ld, v, n, k, wp, outs[b], hosts[b], eps, s))
+        # the stream of this step, on which the caller records the event that it waits for
+        check(fn(a, dtype, n, ld, v, n, k, wp, outs[b], hosts[b], eps, stream_handle()))
 
     return step
 

@@ -397,3 +397,36 @@ def test_product_of_a_wide_matrix_fills_the_chip(hip_available):
 
     assert best(lambda: hb.dense_matvec(A, x, out=y)) < 8 * best(lambda: B.copy_(A))
     assert _product_error(A, x) < 1e-15 * 1000000**0.5
+
+
+def test_gmres_callback_may_change_the_stream(monkeypatch, hip_available):
+    """A callback that finishes the work of one stream and makes another current: later steps run on the new
+    stream, and the host reads their coefficients only after they have arrived."""
+    import torch
+
+    from bempp_amd.api.linalg.iterative_solvers import device_gmres
+    from bempp_amd.core import hip_backend as hb
+
+    rng = np.random.default_rng(1)
+    n = 60
+    A = torch.from_numpy(np.eye(n) + 0.05 * rng.standard_normal((n, n))).to(hb.device())
+    b = rng.standard_normal(n)
+    expected, _ = device_gmres(A, b, rtol=1e-10)
+    _delayed_stepper(monkeypatch, 2_000_000)
+    first, other, calls = torch.cuda.current_stream(), torch.cuda.Stream(), 0
+
+    def callback(residual):
+        nonlocal calls
+        calls += 1
+        if calls == 2:
+            torch.cuda.synchronize()
+            torch.cuda.set_stream(other)
+
+    try:
+        x, info = device_gmres(A, b, rtol=1e-10, callback=callback)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_stream(first)
+    assert info == 0 and calls > 4
+    # the same arithmetic: atomics of the product may reorder a row's sums, times the condition (below 100)
+    assert torch.linalg.vector_norm(x - expected) < 1e-12 * torch.linalg.vector_norm(expected)
