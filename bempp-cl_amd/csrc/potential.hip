@@ -21,6 +21,7 @@
 #include "bem_device.h"
 #include "bem_internal.h"
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -1105,7 +1106,7 @@ __global__ __launch_bounds__(256) void potential_reduce_kernel(const PotArgs a, 
 // field, 390 triangles, 3,251 points 75 -> 40 us; Laplace, 720 triangles, 500 points 19 -> 8 us; whole calls in
 // mixed precision: electric field, 80 triangles, 11,938 points 261 -> 144 us, 1,620 triangles, 2,000 points
 // 228 -> 159 us. Beyond: 456 triangles, 11,869 points (517 workgroups, mixed) 159 us whole, 166 us split.
-constexpr int kPotSplitWorkgroups = 1024, kPotSplitWorkgroupsMixed = 512;
+constexpr int kPotWorkgroups = 4096, kPotSplitWorkgroups = 1024, kPotSplitWorkgroupsMixed = 512;
 
 // Scalar potentials of up to this many (point, source) pairs are evaluated in FP64 in either mode: the pairs
 // take less than the call's other launches (25 M pairs: 15 us Laplace, 40 us Helmholtz in FP64), and on meshes
@@ -1117,7 +1118,7 @@ static void plan(int npts, int nsrc, int precision, int *nchunk, int *chunk_len,
     *nsrc_pad = ((nsrc + kPotTile - 1) / kPotTile) * kPotTile;
     const int tblocks = max(1, (npts + kPotThreads - 1) / kPotThreads);  // no points: one block's plan
     const int ntiles = max(1, *nsrc_pad / kPotTile);                     // no sources: one empty chunk
-    int want = (4096 + tblocks - 1) / tblocks;  // aim at >= 4096 workgroups
+    int want = (kPotWorkgroups + tblocks - 1) / tblocks;
     if (want > ntiles) want = ntiles;
     if (want > 65535) want = 65535;
     if (want < 1) want = 1;
@@ -1196,20 +1197,39 @@ static int run_potential(PotArgs &a, int precision, int out_dtype, hipStream_t s
 
 using namespace bem;
 
+static int evaluated_precision(int op, int nsrc, int n_points, int precision) {
+    const bool scalar = !is_vector_potential_op(op) && !is_far_field_op(op);
+    return scalar && (int64_t)nsrc * n_points <= kPotFp64Pairs ? BEM_PRECISION_FP64 : precision;
+}
+
+// Workspace of one evaluation: the source records and the chunk partials.
+static size_t workspace_bytes(int kd, int nsrc_pad, int nchunk, int n_points) {
+    return sizeof(double) * ((size_t)kSrcFields * nsrc_pad + (size_t)2 * nchunk * kd * n_points) + 256;
+}
+
+// The size for up to n_points points: fewer points may be split into more chunks, so that the size of one
+// evaluation alone does not grow with its points (320 triangles in FP64: 24,000 points 6.4 MB, 32,768 points 4.4 MB).
 extern "C" size_t bem_potential_workspace_size(int op, const bem_space_t *space, const bem_quad_rule_t *rule,
                                                int n_points, int precision) {
     if (!space || !rule || n_points < 0) return 0;
-    int nsrc = space->n_elements * rule->n_points, nchunk, chunk_len, nsrc_pad;
+    const int nsrc = space->n_elements * rule->n_points, kd = is_vector_potential_op(op) ? 3 : 1;
     (void)precision;  // one size for both: the FP64 plan has at least as many chunks
+    size_t size = 0;
+    int nchunk, chunk_len, nsrc_pad;
+    // the plan depends on the number of target blocks, and is one chunk from kPotWorkgroups blocks on
+    const int blocks = n_points / kPotThreads;
+    for (int b = 1; b <= min(blocks, kPotWorkgroups); ++b) {
+        plan(b * kPotThreads, nsrc, BEM_PRECISION_FP64, &nchunk, &chunk_len, &nsrc_pad);
+        size = std::max(size, workspace_bytes(kd, nsrc_pad, nchunk, b * kPotThreads));
+    }
     plan(n_points, nsrc, BEM_PRECISION_FP64, &nchunk, &chunk_len, &nsrc_pad);
-    int kd = is_vector_potential_op(op) ? 3 : 1;
-    return sizeof(double) * ((size_t)kSrcFields * nsrc_pad + (size_t)2 * nchunk * kd * n_points) + 256;
+    return std::max(size, workspace_bytes(kd, nsrc_pad, nchunk, n_points));
 }
 
 // Checks, workspace layout and launches of bem_potential_evaluate.
 static int potential_evaluate(int op, const bem_space_t *space, const void *coefficients, int n_points,
                               const double *points, const bem_quad_rule_t *rule, double k_re, double k_im,
-                              int precision, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
+                              int precision, void *out, int out_dtype, void *workspace, size_t workspace_size,
                               hipStream_t s) {
     // no points: points and out may be null (an empty tensor has no storage)
     if (!space || !rule || !coefficients || (n_points > 0 && (!points || !out)) || !workspace) {
@@ -1234,13 +1254,16 @@ static int potential_evaluate(int op, const bem_space_t *space, const void *coef
         set_error("quadrature rule must have 1..%d points", BEM_QUAD_MAX_POINTS);
         return BEM_ERR_INVALID_ARGUMENT;
     }
-    size_t need = bem_potential_workspace_size(op, space, rule, n_points, precision);
-    if (workspace_bytes < need) {
-        set_error("workspace too small: %zu < %zu bytes", workspace_bytes, need);
+    PotArgs a;
+    a.nsrc = space->n_elements * rule->n_points;
+    precision = evaluated_precision(op, a.nsrc, n_points, precision);
+    plan(n_points, a.nsrc, precision, &a.nchunk, &a.chunk_len, &a.nsrc_pad);
+    const size_t need = workspace_bytes(is_vector_potential_op(op) ? 3 : 1, a.nsrc_pad, a.nchunk, n_points);
+    if (workspace_size < need) {
+        set_error("workspace too small: %zu < %zu bytes", workspace_size, need);
         return BEM_ERR_WORKSPACE;
     }
     if (n_points == 0) return BEM_OK;
-    PotArgs a;
     a.sp = to_args(space);
     a.rule = to_args_wide(rule);
     a.coeffs = (const double *)coefficients;
@@ -1248,10 +1271,6 @@ static int potential_evaluate(int op, const bem_space_t *space, const void *coef
     a.pts = points;
     a.kr = (op == BEM_LAPLACE_SINGLE_LAYER || op == BEM_LAPLACE_DOUBLE_LAYER) ? 0.0 : k_re;
     a.ki = (op == BEM_LAPLACE_SINGLE_LAYER || op == BEM_LAPLACE_DOUBLE_LAYER) ? 0.0 : k_im;
-    a.nsrc = space->n_elements * rule->n_points;
-    if (!is_vector_potential_op(op) && !is_far_field_op(op) && (int64_t)a.nsrc * n_points <= kPotFp64Pairs)
-        precision = BEM_PRECISION_FP64;
-    plan(n_points, a.nsrc, precision, &a.nchunk, &a.chunk_len, &a.nsrc_pad);
     uintptr_t base = ((uintptr_t)workspace + 255) & ~(uintptr_t)255;
     a.src = (double *)base;
     a.partial = a.src + (size_t)kSrcFields * a.nsrc_pad;
@@ -1329,7 +1348,11 @@ extern "C" int bem_potential_evaluate_noalloc(int op, const bem_space_t *space, 
         set_error("null argument");
         return BEM_ERR_INVALID_ARGUMENT;
     }
-    size_t need = bem_potential_workspace_size(op, space, rule, n_points, precision);
+    // of this evaluation, not of up to n_points points
+    const int nsrc = space->n_elements * rule->n_points;
+    int nchunk, chunk_len, nsrc_pad;
+    plan(n_points, nsrc, evaluated_precision(op, nsrc, n_points, precision), &nchunk, &chunk_len, &nsrc_pad);
+    const size_t need = workspace_bytes(is_vector_potential_op(op) ? 3 : 1, nsrc_pad, nchunk, n_points);
     if (need > (size_t)BEM_POTENTIAL_SCRATCH_BYTES) {
         set_error("potential needs %zu bytes of workspace, more than the %zu-byte scratch buffer of "
                   "bem_potential_evaluate_noalloc; use bem_potential_evaluate with a caller workspace",

@@ -280,7 +280,8 @@ int bem_singular_assemble_sl_dl(int op, const bem_space_t *test, const bem_space
  *   n_points = 0, points and out may be null; a space without elements gives zeros.
  * Only BEM_LAPLACE_SINGLE_LAYER, BEM_LAPLACE_DOUBLE_LAYER, BEM_HELMHOLTZ_SINGLE_LAYER,
  * BEM_HELMHOLTZ_DOUBLE_LAYER and BEM_MAXWELL_ELECTRIC_FIELD are potentials.
- * workspace: device memory of at least bem_potential_workspace_size(...) bytes.
+ * workspace: device memory of at least bem_potential_workspace_size(...) bytes, the size for any
+ *   call of up to n_points points (in either precision).
  */
 size_t bem_potential_workspace_size(int op, const bem_space_t *space, const bem_quad_rule_t *rule, int n_points,
                                     int precision);
@@ -294,8 +295,8 @@ int bem_potential_evaluate(int op, const bem_space_t *space, const void *coeffic
  * cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc). Same arguments and results as bem_potential_evaluate without the
  * workspace: it uses a library-owned static device buffer of BEM_POTENTIAL_SCRATCH_BYTES per
- * GPU (held until the process ends) and calls no allocator. Returns BEM_ERR_WORKSPACE when
- * bem_potential_workspace_size(...) exceeds that size (the level-5 P1 potential at 16,384
+ * GPU (held until the process ends) and calls no allocator. Returns BEM_ERR_WORKSPACE when the
+ * call's source records and partial sums exceed that size (the level-5 P1 potential at 16,384
  * points needs 29.5 MB, the level-4 RWG potential at 65,536 points 50.6 MB). All calls on one
  * GPU share the buffer: calls that overlap on one GPU (other streams, other threads) race.
  */

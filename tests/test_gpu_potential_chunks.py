@@ -57,3 +57,32 @@ def test_mixed_against_fp64(family, name, k, count, hip_available):
     # the mode's stated accuracy; a scalar call in FP64 rounds its output only
     exact = family != "maxwell" and count * 1920 <= 3 << 23
     assert np.linalg.norm(single - double) < (1e-7 if exact else 2e-6) * np.linalg.norm(double)
+
+
+@pytest.mark.parametrize("precision", ["double", "single"])
+def test_workspace_of_the_largest_batch_serves_smaller_ones(precision, hip_available):
+    """320 triangles: 24,000 points take more chunks than 32,768, and fit the workspace sized for these."""
+    import ctypes
+
+    import torch
+
+    import bempp_amd.api as bempp
+    from bempp_amd.api.grid.shapes import icosphere
+    from bempp_amd.api.integration.triangle_gauss import rule as triangle_rule
+    from bempp_amd.core import hip_backend as hb
+
+    L = hb.lib()
+    space = hb.device_space(bempp.function_space(icosphere(2), "DP", 0))
+    rule = hb.quad_rule(*triangle_rule(4))
+    mode = hb.PRECISION_FP64 if precision == "double" else hb.PRECISION_MIXED
+    size = L.bem_potential_workspace_size(3, ctypes.byref(space.struct), ctypes.byref(rule), 32768, mode)
+    work = torch.empty(size, dtype=torch.uint8, device=hb.device())
+    c = torch.ones(320, dtype=torch.complex128, device=hb.device())
+    points = torch.randn((32768, 3), dtype=torch.float64, device=hb.device())
+    points *= 2.0 / torch.linalg.vector_norm(points, dim=1, keepdim=True)
+    for count in (32768, 24000, 5000, 1):
+        out = torch.empty((1, count), dtype=torch.complex128, device=hb.device())
+        hb.check(L.bem_potential_evaluate(3, ctypes.byref(space.struct), hb.ptr(c), count, hb.ptr(points), ctypes.byref(rule),
+                                          2.0, 0.0, mode, hb.ptr(out), hb.DTYPES["complex128"], hb.ptr(work), size,
+                                          hb.stream_handle()))
+        assert torch.isfinite(torch.view_as_real(out)).all()

@@ -109,3 +109,21 @@ def test_potential_workspace_size_empty_sets(n_elements, n_points):
     for op in (0, 3, 6):
         need = L.bem_potential_workspace_size(op, ctypes.byref(sp), ctypes.byref(rule), n_points, 1)
         assert need >= 256
+
+
+@pytest.mark.parametrize("op", [0, 3, 6, 9], ids=["laplace", "helmholtz", "electric", "far"])
+@pytest.mark.parametrize("n_elements", [20, 320, 1280, 5120, 20480])
+def test_potential_workspace_size_grows_with_the_points(op, n_elements):
+    """A workspace sized for the largest batch serves every smaller one, although fewer points are split into
+    more chunks."""
+    from bempp_amd.core import hip_backend
+
+    L = hip_backend.lib()
+    rule = hip_backend.BemQuadRule()
+    rule.n_points = 6
+    sp = hip_backend.BemSpace()
+    sp.n_elements = n_elements
+    for precision in (0, 1):
+        points = sorted({int(256 * 1.07**j) + d for j in range(130) for d in (-1, 0, 1)} | {0, 1, 24000, 32768, 1 << 22})
+        sizes = [L.bem_potential_workspace_size(op, ctypes.byref(sp), ctypes.byref(rule), n, precision) for n in points]
+        assert sizes == sorted(sizes)
