@@ -192,7 +192,7 @@ def _make_functions():
             # points to the host and map the coefficients there, twice the time of the kernels on small meshes
             mode = problem.mode()
             op = "laplace_single_layer" if problem.wavenumber == 0.0 else "helmholtz_single_layer"
-            dspace = hb.potential_space(space, op, mode)
+            dspace = hb.device_space(space)
             out = torch.empty((1, pts.shape[0]), dtype=torch.complex64 if mode == hb.PRECISION_MIXED else torch.complex128,
                               device=dev)
             hb.potential_evaluate(op, dspace, _full_coefficients(dspace, c), pts, _device_rule(problem.parameters),

@@ -36,6 +36,7 @@ def hip_potential_assembler(space, operator_descriptor, points, parameters):
                   "maxwell_magnetic_field"):
         raise KeyError(f"Unsupported potential kernel {op}")
     dev = hb.device()
+    dspace = hb.device_space(space)
     pts = _np.asarray(points, dtype=_np.float64)
     if pts.ndim != 2 or pts.shape[0] != 3:
         raise ValueError("points must have shape (3, npoints)")
@@ -43,7 +44,6 @@ def hip_potential_assembler(space, operator_descriptor, points, parameters):
     qp, qw = triangle_rule(parameters.quadrature.regular)
     rule = hb.quad_rule(qp, qw)
     mode = hb.PRECISION_MIXED if operator_descriptor.precision == "single" else hb.PRECISION_FP64
-    dspace = hb.potential_space(space, op, mode)
     kdim = operator_descriptor.kernel_dimension
     out_dtype = torch.complex64 if operator_descriptor.precision == "single" else torch.complex128
     k = _wavenumber(operator_descriptor)

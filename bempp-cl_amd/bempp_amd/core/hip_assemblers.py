@@ -236,7 +236,7 @@ def potential_assembler(device_interface, space, operator_descriptor, points, pa
     out_t = getattr(torch, complex_t)
     kdim = int(operator_descriptor.kernel_dimension)
     k = _wavenumber(operator_descriptor)
-    dspace = hb.potential_space(view, op, mode)
+    dspace = hb.device_space(view)
 
     def evaluator(x):
         coeffs = torch.from_numpy(_np.ascontiguousarray(_np.asarray(x, dtype=_np.complex128))).to(dev)

@@ -31,7 +31,6 @@ OPERATORS = {
     "maxwell_magnetic_far_field": 12,
     "maxwell_magnetic_field": 13,
 }
-_SCALAR_POTENTIALS = ("laplace_single_layer", "laplace_double_layer", "helmholtz_single_layer", "helmholtz_double_layer")
 SHAPESETS = {"p0_discontinuous": 0, "p1_discontinuous": 1, "rwg0": 2, "snc0": 2}
 DTYPES = {"float32": 0, "float64": 1, "complex64": 2, "complex128": 3}
 PRECISION_FP64 = 0
@@ -278,29 +277,6 @@ def device_space(space):
     key = space.id
     if key not in _SPACE_CACHE:
         _SPACE_CACHE[key] = DeviceSpace(space)
-    return _SPACE_CACHE[key]
-
-
-def potential_space(space, op, precision):
-    """The device copy of a space for a potential. The mixed kernel of the scalar potentials groups
-    consecutive sources around a reference: for it the support elements are listed along a
-    space-filling curve of their centroids, so that groups are compact whatever the order of the
-    mesh file (20,480 triangles in rows, 16,384 points: 1.62 -> 1.28 ms)."""
-    from bempp_amd.core.blocking import _morton_keys
-
-    base = device_space(space)
-    if precision != PRECISION_MIXED or op not in _SCALAR_POTENTIALS:
-        return base
-    key = (space.id, "potential")
-    if key not in _SPACE_CACHE:
-        elements = space.support_elements.astype(np.int64)
-        order = np.argsort(_morton_keys(space.grid.centroids[elements]), kind="stable")
-        ordered = object.__new__(DeviceSpace)
-        ordered.__dict__.update(base.__dict__)
-        ordered.elements = _torch().from_numpy(np.ascontiguousarray(elements[order], dtype=np.int32)).to(device())
-        ordered.struct = BemSpace.from_buffer_copy(base.struct)
-        ordered.struct.elements = ordered.elements.data_ptr()
-        _SPACE_CACHE[key] = ordered
     return _SPACE_CACHE[key]
 
 

@@ -569,9 +569,9 @@ __global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_efie(const P
 // GS: the radius of a group decides how many (target, group) pairs take the FP64 path and how large
 // k (r - r0) gets; the FP64 part costs about 70 instructions a group and target. 20,480 triangles,
 // 16,384 targets 0.5 to 2 off the surface (whole pass): one reference per tile of 256 7.3 ms
-// (4.5 ms by rsqrt_t alone), groups of 64 2.31, of 32 1.62 ms; with the elements along a space-filling
-// curve (hip_backend.potential_space) 1.63, 1.34 and 1.28 ms, errors 2.5e-7, 1.2e-7 and 8.4e-8. The
-// inner loop is bound by its 17.5 instructions, 4 of them transcendental.
+// (4.5 ms by rsqrt_t alone), groups of 64 2.31, of 32 1.62 ms. The inner loop is bound by its 17.5
+// instructions, 4 of them transcendental. The elements keep the order of the mesh: along a space-filling
+// curve the call takes 1.28 ms, but the order of each new mesh takes 6 ms on the host.
 template <int OP, bool DAMP>
 __global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_scalar(const PotArgs a) {
     constexpr int GS = 32;

@@ -249,6 +249,36 @@ def test_autograd_loss(precision, default_parameters, hip_available):
 
 
 @pytest.mark.parametrize("precision", ["single", "double"])
+def test_potential_of_moved_vertices_sorts_nothing_on_the_host(precision, default_parameters, monkeypatch, hip_available):
+    """The forward of the differentiable potential on new vertices equals the potential operator's, and takes the
+    elements in the order of the mesh: no ordering of each new mesh on the host."""
+    import torch
+
+    from bempp_amd.api.assembly.grid_function import GridFunction
+    from bempp_amd.api.differentiable import SingleLayerProblem, _dp0_space, single_layer_potential
+    from bempp_amd.api.grid.shapes import icosphere
+    from bempp_amd.core import blocking
+
+    grid = icosphere(2)
+    rng = np.random.default_rng(17)
+    c = _complex(rng, grid.number_of_elements)
+    points = rng.standard_normal((13200, 3))  # 25.3 M (point, source) pairs: beyond the calls evaluated in FP64
+    points *= 2.0 / np.linalg.norm(points, axis=1)[:, None]
+    prob = SingleLayerProblem(grid.elements, 2.0, precision=precision, parameters=default_parameters)
+
+    def refuse(points):
+        raise AssertionError("the elements of a potential are not sorted")
+
+    monkeypatch.setattr(blocking, "_morton_keys", refuse)
+    for scale in (1.0, 1.1):
+        v = torch.from_numpy(_vtx(grid) * scale)
+        u = single_layer_potential(v, torch.from_numpy(c), torch.from_numpy(points), prob).cpu().numpy()
+        sp = _dp0_space(prob.grid(v))
+        ref = prob.potential(sp, points.T).evaluate(GridFunction(sp, coefficients=c))[0]
+        np.testing.assert_array_equal(u, ref)
+
+
+@pytest.mark.parametrize("precision", ["single", "double"])
 def test_moving_vertices_do_not_accumulate_device_memory(hip_available, precision):
     """A shape-optimisation loop (new vertex positions every step) keeps device memory flat:
     the problem releases the previous grid's and space's cached device copies."""
