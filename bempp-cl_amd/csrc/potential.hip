@@ -218,11 +218,12 @@ __device__ __forceinline__ void fp64_magnetic_source(F field, double x0, double 
 // kNearTileFactor times the radius R of the tile's sources around the reference takes the FP64
 // path: the FP32 offsets lose relative accuracy once the target comes within a fraction of R of
 // the sources (targets just off the surface), while targets beyond r0 >= 1.5 R stay within 1e-6
-// of FP64 (measured for the single, double layer and EFIE potentials on icosphere levels 2 and 4).
+// of FP64 (measured for the single, double layer and EFIE potentials on icosphere levels 2 and 4). Scalar
+// potentials: see potential_eval_mixed_scalar.
 constexpr double kNearTileFactor = 1.5;
 
 // The FP64 path of the mixed kernels for the sources [s_begin, s_end) of the workspace.
-template <int OP, int KD>
+template <int OP, int KD, int PH = 0>
 __device__ __forceinline__ void sources_fp64_near(const PotArgs &a, int s_begin, int s_end, double x0, double x1,
                                                double x2, double alr, double ali, double *accr, double *acci) {
     double ar[KD], ai[KD];
@@ -230,7 +231,7 @@ __device__ __forceinline__ void sources_fp64_near(const PotArgs &a, int s_begin,
     for (int d = 0; d < KD; ++d) ar[d] = ai[d] = 0.0;
     const int64_t P = a.nsrc_pad;
     for (int s = s_begin; s < s_end; ++s)
-        fp64_source<OP, 0>([&](int k) { return a.src[k * P + s]; }, x0, x1, x2, a.kr, a.ki, alr, ali, ar, ai);
+        fp64_source<OP, PH>([&](int k) { return a.src[k * P + s]; }, x0, x1, x2, a.kr, a.ki, alr, ali, ar, ai);
 #pragma unroll
     for (int d = 0; d < KD; ++d) {
         accr[d] += ar[d];
@@ -557,33 +558,80 @@ __global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_efie(const P
     }
 }
 
-// MIXED scalar potentials (Laplace and Helmholtz single and double layer). The sources of a tile
-// of 256 are staged once as FP32 records relative to the reference source c (the middle one) of
-// their group of GS:
-//   u = c - y, |u|^2, the weights c_j / (4 pi) and, for the double layer, n_y and u.n_y,
-// read by every lane as LDS broadcasts. Per (target, group) the FP64 part forms v = x - c,
-// r0^2 = |v|^2, r0 and e^{i k r0}; per source only
-//   t = r^2 - r0^2 = 2 v.u + |u|^2,  r = sqrt(r0^2 + t),  k (r - r0) / 2 pi = t / ((r + r0) K)
-// (K = 2 pi / k) are needed in FP32, with the hardware rsq, rcp, sin and cos (revolutions). DAMP:
-// complex wavenumber, e^{-Im(k) (r - r0)} per source (exp2), e^{-Im(k) r0} per group.
-// GS: the radius of a group decides how many (target, group) pairs take the FP64 path and how large
-// k (r - r0) gets; the FP64 part costs about 70 instructions a group and target. 20,480 triangles,
-// 16,384 targets 0.5 to 2 off the surface (whole pass): one reference per tile of 256 7.3 ms
-// (4.5 ms by rsqrt_t alone), groups of 64 2.31, of 32 1.62 ms. The inner loop is bound by its 17.5
-// instructions, 4 of them transcendental. The elements keep the order of the mesh: along a space-filling
-// curve the call takes 1.28 ms, but the order of each new mesh takes 6 ms on the host.
+// e^{ik delta} - 1 for the scalar potentials (Re k; see efie_em1 for MODE 0 to 2: |y| <= 1, y = k delta).
+// MODE 3 (|y| <= 2): the series in y through y^12 and y^13 (remainders 1e-7 and 2e-8 of the leading
+// terms). MODE 4, any y: the hardware sine and cosine (revolutions), whose absolute error of about 1e-7
+// is no larger than the rounding of values of order one.
+template <int MODE>
+__device__ __forceinline__ void scalar_em1(float delta, float kr, float kr_rev, const EfieSeries &e, float &em1r,
+                                           float &em1i, float &si) {
+    if constexpr (MODE < 3) {
+        efie_em1<MODE>(delta, e, em1r, em1i, si);
+    } else if constexpr (MODE == 3) {
+        const float y = kr * delta, y2 = y * y;
+        float p = fmaf(y2, 1.f / 479001600.f, -1.f / 3628800.f);
+        p = fmaf(y2, p, 1.f / 40320.f);
+        p = fmaf(y2, p, -1.f / 720.f);
+        p = fmaf(y2, p, 1.f / 24.f);
+        p = fmaf(y2, p, -0.5f);
+        em1r = y2 * p;
+        float q = fmaf(y2, 1.f / 6227020800.f, -1.f / 39916800.f);
+        q = fmaf(y2, q, 1.f / 362880.f);
+        q = fmaf(y2, q, -1.f / 5040.f);
+        q = fmaf(y2, q, 1.f / 120.f);
+        q = fmaf(y2, q, -1.f / 6.f);
+        em1i = fmaf(y * y2, q, y);
+        si = 0.f;
+    } else {
+        const float ph = kr_rev * delta;
+        em1r = __builtin_amdgcn_cosf(ph) - 1.f;
+        em1i = __builtin_amdgcn_sinf(ph);
+        si = 0.f;
+    }
+}
+
+// MIXED scalar potentials (Laplace and Helmholtz single and double layer), per (target, group of 32
+// neighbouring sources). With c the group's middle source, v = x - c, u = c - y (so x - y = v + u), r0 = |v|,
+// t = r^2 - r0^2 = 2 v.u + |u|^2, delta = r - r0 = t / (r + r0) and E = e^{ik delta}, the FP64 part forms r0 and
+// e^{ik r0}; the sources, staged per tile of 256 as FP32 records and read as LDS broadcasts, take one of three
+// paths, chosen per wave by the distance of its targets:
+//  * away from the whole tile (kNearTileFactor times its radius): E / r itself, with the hardware rsq, rcp, sin
+//    and cos, 17.5 instructions (single layer), error about 1e-7 of each term;
+//  * closer to the tile, away from the group: the sums split into a group-centre term from FP64 group sums and
+//    a remainder of small differences in FP32 (as potential_eval_mixed_efie),
+//      single layer  sum_j c_j G        = e^{ik r0} / 4 pi [ sum_j c_j / r0 + sum_j f c_j ],  f = (E - 1) / r - q,
+//      double layer  sum_j c_j dG/dn_y  = e^{ik r0} / 4 pi [ h(r0) (v . sum_j c_j n_j + sum_j c_j u_j.n_j)
+//                                                            + sum_j b c_j (v + u_j).n_j ],
+//      h(r) = 1/r^3 - ik/r^2,  b = h(r) - h(r0) + (E - 1) h(r),  q = 1/r0 - 1/r = delta / (r r0),
+//      h(r) - h(r0) = -q (1/r^2 + 1/(r r0) + 1/r0^2) + ik q (1/r + 1/r0):
+//    the FP32 rounding is relative to the remainder, about |u| / r0 + |k u| of the sum;
+//  * close to the group, where that is no small part: FP64.
+// The tile decides as if all its sources had one reference, so that no pair that would be summed in FP64 then is
+// left to plain FP32; the small groups only save FP64 work. kNearScalar: sized for errors that stay at the FP32
+// rounding of the result. Random densities, points 1.5 to 3 from the centre of spheres and screens of 80 to
+// 15,680 triangles, up to the wavenumber of 8 elements a wavelength, against FP64: 2.5e-8 to 3.1e-8 where all
+// tiles are close (720 triangles; one reference per tile with FP64 near it 2.5e-8, E / r for all groups away from
+// 1.5 times their own radius 6e-8 to 1.1e-7), up to 1.5e-7 on large meshes (2.3e-7, 1.7e-7).
+// 20,480 triangles in rows, 16,384 points (whole call): 1.56 ms single layer (one reference per tile 7.5, E / r
+// for all groups 1.62), 2.2 ms double layer (9.1, 2.3). 15,680 triangles, 20,000 points, Helmholtz single layer,
+// kernel: points 10 to 20 from the centre 1.19 ms (1.01, 1.13), 1.02 to 1.3 2.6 ms (10.5, 3.4).
+// DAMP: complex wavenumber, E = e^{-Im(k) delta} e^{i Re(k) delta}.
 template <int OP, bool DAMP>
-__global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_scalar(const PotArgs a) {
+__global__ __launch_bounds__(kPotThreads, 4) void potential_eval_mixed_scalar(const PotArgs a) {
     constexpr int GS = 32;
     constexpr int NG = kPotTile / GS;
     constexpr bool HELM = OP == kHelmholtzSL || OP == kHelmholtzDL;
     constexpr bool DL = OP == kLaplaceDL || OP == kHelmholtzDL;
+    constexpr double kNearScalar = DL ? 2.5 : 1.5, kNearScalarPhase = 1.5;
+    constexpr int NW = DL ? 8 : 2;  // FP64 group sums: c (single layer); c n and c u.n (double layer), over 4 pi
     static_assert(!DAMP || HELM, "only Helmholtz wavenumbers are complex");
     __shared__ float4 shu[kPotTile];           // u, |u|^2
     __shared__ float4 shw[kPotTile];           // Re c / 4 pi, Im c / 4 pi, u.n_y, -
     __shared__ float4 shn[DL ? kPotTile : 1];  // n_y, -
     __shared__ double sc[NG][3];
-    __shared__ float srad2[NG];  // max |u|^2 of the group's sources
+    __shared__ double wsum[NG][NW];
+    __shared__ float srad[NG];  // max |u| of the group's sources (bounds |delta|)
+    __shared__ float trad2[kPotThreads / 64];  // per wave: max |c_tile - y|^2 of the whole tile's sources
     const int m = blockIdx.x * kPotThreads + threadIdx.x;
     const int chunk = blockIdx.y;
     const int s0 = chunk * a.chunk_len;
@@ -597,14 +645,26 @@ __global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_scalar(const
     double accr = 0.0, acci = 0.0;
     const float kr_f = (float)a.kr, ki_f = (float)a.ki;
     const float kr_rev = (float)(a.kr * 0.15915494309189533577);
-    const float ki_log2e = (float)(a.ki * 1.4426950408889634);
-    const float kinv = 1.f / kr_rev;  // K (infinite for k = 0: the phase is then 0)
+    const float kabs = fabsf(kr_f), kinv = 1.f / kr_rev;  // kinv: infinite for k = 0 (the phase is then 0)
+    const float ki_log2e = (float)(a.ki * 1.4426950408889634), kmax = fmaxf(kabs, fabsf(ki_f));
+    const EfieSeries &ser = a.ser;
     const int P = a.nsrc_pad;
     for (int t0 = s0; t0 < s1; t0 += kPotTile) {
         const int nt = min(kPotTile, s1 - t0);
+        // the whole tile that the staged sources are from (a chunk may be a part of one) and its middle source
+        const int tb = t0 - t0 % kPotTile, tn = min(kPotTile, a.nsrc - tb), tc = tb + min(kPotTile / 2, tn - 1);
+        const double tc0 = a.src[tc], tc1 = a.src[(int64_t)P + tc], tc2 = a.src[2 * (int64_t)P + tc];
         __syncthreads();
         {
             const int j = threadIdx.x, g = j / GS, s = t0 + j;
+            float t2 = 0.f;
+            if (j < tn) {
+                const double u0 = tc0 - a.src[tb + j], u1 = tc1 - a.src[(int64_t)P + tb + j], u2 = tc2 - a.src[2 * (int64_t)P + tb + j];
+                t2 = (float)(u0 * u0 + u1 * u1 + u2 * u2);
+            }
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) t2 = fmaxf(t2, __shfl_xor(t2, off, 64));
+            if ((j & 63) == 0) trad2[j >> 6] = t2;
             const int cidx = t0 + min(g * GS + GS / 2, nt - 1);
             double c[3];
             for (int d = 0; d < 3; ++d) c[d] = a.src[(int64_t)d * P + cidx];
@@ -612,105 +672,241 @@ __global__ __launch_bounds__(kPotThreads) void potential_eval_mixed_scalar(const
                 for (int d = 0; d < 3; ++d) sc[g][d] = c[d];
             float4 U = make_float4(0.f, 0.f, 0.f, 0.f), W = make_float4(0.f, 0.f, 0.f, 0.f);
             float4 N = make_float4(0.f, 0.f, 0.f, 0.f);
+            double uu = 0.0, w[NW];
+#pragma unroll
+            for (int k = 0; k < NW; ++k) w[k] = 0.0;
             if (j < nt) {
                 const double u0 = c[0] - a.src[s], u1 = c[1] - a.src[(int64_t)P + s], u2 = c[2] - a.src[2 * (int64_t)P + s];
-                U = make_float4((float)u0, (float)u1, (float)u2, (float)(u0 * u0 + u1 * u1 + u2 * u2));
-                W.x = (float)(kInv4Pi * a.src[6 * (int64_t)P + s]);
-                W.y = (float)(kInv4Pi * a.src[7 * (int64_t)P + s]);
+                uu = u0 * u0 + u1 * u1 + u2 * u2;
+                U = make_float4((float)u0, (float)u1, (float)u2, (float)uu);
+                const double cr = kInv4Pi * a.src[6 * (int64_t)P + s], ci = kInv4Pi * a.src[7 * (int64_t)P + s];
+                W.x = (float)cr;
+                W.y = (float)ci;
                 if constexpr (DL) {
-                    const double n0 = a.src[3 * (int64_t)P + s], n1 = a.src[4 * (int64_t)P + s],
-                                 n2 = a.src[5 * (int64_t)P + s];
-                    N = make_float4((float)n0, (float)n1, (float)n2, 0.f);
-                    W.z = (float)(u0 * n0 + u1 * n1 + u2 * n2);
+                    const double n[3] = {a.src[3 * (int64_t)P + s], a.src[4 * (int64_t)P + s], a.src[5 * (int64_t)P + s]};
+                    const double un = u0 * n[0] + u1 * n[1] + u2 * n[2];
+                    N = make_float4((float)n[0], (float)n[1], (float)n[2], 0.f);
+                    W.z = (float)un;
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        w[2 * d] = cr * n[d];
+                        w[2 * d + 1] = ci * n[d];
+                    }
+                    w[6] = cr * un;
+                    w[7] = ci * un;
+                } else {
+                    w[0] = cr;
+                    w[1] = ci;
                 }
             }
             shu[j] = U;
             shw[j] = W;
             if constexpr (DL) shn[j] = N;
-            float w2 = U.w;
 #pragma unroll
-            for (int off = GS / 2; off >= 1; off >>= 1) w2 = fmaxf(w2, __shfl_xor(w2, off, 64));
-            if (j % GS == 0) srad2[g] = w2;
+            for (int k = 0; k < NW; ++k) {
+#pragma unroll
+                for (int off = GS / 2; off >= 1; off >>= 1) w[k] += __shfl_xor(w[k], off, 64);
+            }
+#pragma unroll
+            for (int off = GS / 2; off >= 1; off >>= 1) uu = fmax(uu, __shfl_xor(uu, off, 64));
+            if (j % GS == 0) {
+#pragma unroll
+                for (int k = 0; k < NW; ++k) wsum[g][k] = w[k];
+                srad[g] = (float)(sqrt(uu) * (1.0 + 1e-6));
+            }
         }
         __syncthreads();
+        // wave-uniform: every target is away from the tile
+        float R2 = trad2[0];
+#pragma unroll
+        for (int w = 1; w < kPotThreads / 64; ++w) R2 = fmaxf(R2, trad2[w]);
+        const double q0 = x0 - tc0, q1 = x1 - tc1, q2 = x2 - tc2;
+        const bool far = !__any(m < a.npts && q0 * q0 + q1 * q1 + q2 * q2 <
+                                                  kNearTileFactor * kNearTileFactor * (double)R2 * (1.0 + 1e-6));
         for (int g = 0; g < NG && g * GS < nt; ++g) {
             const int j0 = g * GS, j1 = min(j0 + GS, nt);
+            // |Re(k) delta| <= |Re(k)| max |u| (wave-uniform)
+            const float ymax = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(kabs * srad[g])));
             // per (target, group): FP64 reference distance and phase
             const double v0d = x0 - sc[g][0], v1d = x1 - sc[g][1], v2d = x2 - sc[g][2];
             const double r0sq_d = v0d * v0d + v1d * v1d + v2d * v2d;
             // targets close to the group's sources: the group in FP64 for the whole wave
-            if (__any(m < a.npts && r0sq_d < kNearTileFactor * kNearTileFactor * (double)srad2[g] * (1.0 + 1e-6))) {
-                sources_fp64_near<OP, 1>(a, t0 + j0, t0 + j1, x0, x1, x2, 0.0, 0.0, &accr, &acci);
+            const double rn = (far ? kNearTileFactor : kNearScalar + kNearScalarPhase * (double)(kmax * srad[g])) * (double)srad[g];
+            if (__any(m < a.npts && r0sq_d < rn * rn)) {
+                // every phase is at most |Re k| (r0 + R)
+                const bool reduced = HELM && __all(fabs(a.kr) * (sqrt(r0sq_d) + (double)srad[g]) < 0x1p25);
+                if (reduced)
+                    sources_fp64_near<OP, 1, kPhReduced | (DAMP ? 0 : kPhReal)>(a, t0 + j0, t0 + j1, x0, x1, x2, 0.0, 0.0,
+                                                                               &accr, &acci);
+                else
+                    sources_fp64_near<OP, 1>(a, t0 + j0, t0 + j1, x0, x1, x2, 0.0, 0.0, &accr, &acci);
                 continue;
             }
-            const double r0d = r0sq_d * rsqrt_t(r0sq_d);
+            const double i0 = rsqrt_t(r0sq_d), i2 = i0 * i0, r0d = r0sq_d * i0;
             const float tv0 = (float)(2.0 * v0d), tv1 = (float)(2.0 * v1d), tv2 = (float)(2.0 * v2d);
             const float v0 = (float)v0d, v1 = (float)v1d, v2 = (float)v2d;
-            const float r0sq = (float)r0sq_d, r0 = (float)r0d;
-            const float r0k = r0 * kinv;
+            const float r0sq = (float)r0sq_d, r0 = (float)r0d, r0inv = (float)i0, r0inv2 = (float)i2;
+            // h(r0) (double layer)
+            const double h0rd = HELM ? fma(a.ki, i2, i2 * i0) : i2 * i0, h0id = HELM ? -a.kr * i2 : 0.0;
+            const float h0r = (float)h0rd, h0i = (float)h0id;
             float Ar = 0.f, Ai = 0.f;
+            auto sources = [&](auto mode, auto damping) {
+                constexpr int MODE = decltype(mode)::value;
 #pragma unroll 4
-            for (int j = j0; j < j1; ++j) {
-                const float4 U = shu[j];
-                const float4 W = shw[j];
-                const float tt = tv0 * U.x + (tv1 * U.y + (tv2 * U.z + U.w));  // r^2 - r0^2
-                const float r2 = r0sq + tt;
-                const float rinv = __builtin_amdgcn_rsqf(r2);
-                float er = rinv, ei = 0.f;  // e^{ik(r - r0)} / r (Laplace: 1 / r)
-                float r = 0.f;
-                if constexpr (HELM) {
-                    r = r2 * rinv;
-                    float ph, amp = rinv;
-                    if constexpr (DAMP) {
-                        const float delta = tt * __builtin_amdgcn_rcpf(r + r0);
-                        ph = kr_rev * delta;
-                        amp *= __builtin_amdgcn_exp2f(-ki_log2e * delta);
-                    } else {
-                        ph = tt * __builtin_amdgcn_rcpf(r * kinv + r0k);
-                    }
-                    const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
-                    if constexpr (!DL) {
-                        // single layer: the weight times e^{ik(r - r0)} first, then one FMA by the amplitude
-                        Ar += amp * (cs * W.x - sn * W.y);
-                        Ai += amp * (cs * W.y + sn * W.x);
-                        continue;
-                    }
-                    er = cs * amp;
-                    ei = sn * amp;
-                }
-                if constexpr (DL) {
-                    // (i k r - 1) (y - x).n_y / r^2 with y - x = -(v + u)
-                    const float4 N = shn[j];
-                    const float dot = -(v0 * N.x + (v1 * N.y + (v2 * N.z + W.z)));
-                    const float f = dot * rinv * rinv;
+                for (int j = j0; j < j1; ++j) {
+                    const float4 U = shu[j];
+                    const float4 W = shw[j];
+                    const float tt = fmaf(tv0, U.x, fmaf(tv1, U.y, fmaf(tv2, U.z, U.w)));  // r^2 - r0^2
+                    const float r2 = r0sq + tt;
+                    const float rinv = rsqrt_t(r2);
+                    const float delta = tt * __builtin_amdgcn_rcpf(fmaf(r2, rinv, r0));
+                    const float D = delta * rinv, q = D * r0inv;  // q = 1/r0 - 1/r
+                    float em1r = 0.f, em1i = 0.f, si = 0.f;       // E - 1
                     if constexpr (HELM) {
-                        const float ar = DAMP ? -1.f - ki_f * r : -1.f, ai = kr_f * r;
-                        const float pr = (ar * er - ai * ei) * f, pi = (ar * ei + ai * er) * f;
-                        er = pr;
-                        ei = pi;
+                        scalar_em1<MODE>(delta, kr_f, kr_rev, ser, em1r, em1i, si);
+                        if constexpr (DAMP) {
+                            const float x = -ki_f * delta;
+                            float dm1;  // e^x - 1
+                            if constexpr (decltype(damping)::value) {
+                                dm1 = expm1f(x);
+                            } else {  // |x| <= 0.25: through x^6 (remainder 5e-8 of the leading term)
+                                dm1 = fmaf(x, 1.f / 720.f, 1.f / 120.f);
+                                dm1 = fmaf(x, dm1, 1.f / 24.f);
+                                dm1 = fmaf(x, dm1, 1.f / 6.f);
+                                dm1 = fmaf(x, dm1, 0.5f);
+                                dm1 = fmaf(x * x, dm1, x);
+                            }
+                            em1r = fmaf(dm1, em1r, em1r + dm1);
+                            em1i = fmaf(dm1, em1i, em1i);
+                        }
+                    }
+                    if constexpr (!DL) {
+                        const float fr = HELM ? fmaf(em1r, rinv, -q) : -q;
+                        Ar = fmaf(fr, W.x, Ar);
+                        Ai = fmaf(fr, W.y, Ai);
+                        if constexpr (HELM) {
+                            const float fi = !DAMP && MODE < 3 ? D * si : em1i * rinv;
+                            Ar = fmaf(-fi, W.y, Ar);
+                            Ai = fmaf(fi, W.x, Ai);
+                        }
                     } else {
-                        er = -er * f;
+                        const float4 N = shn[j];
+                        const float dot = fmaf(v0, N.x, fmaf(v1, N.y, fmaf(v2, N.z, W.z)));  // (x - y).n_y
+                        const float s1 = rinv + r0inv, q2 = q * s1;
+                        const float q3 = q * fmaf(s1, rinv, r0inv2);
+                        if constexpr (HELM) {
+                            const float dhr = DAMP ? fmaf(-ki_f, q2, -q3) : -q3, dhi = kr_f * q2;
+                            const float hr = h0r + dhr, hi = h0i + dhi;
+                            const float br = dot * fmaf(em1r, hr, fmaf(-em1i, hi, dhr));
+                            const float bi = dot * fmaf(em1r, hi, fmaf(em1i, hr, dhi));
+                            Ar = fmaf(br, W.x, fmaf(-bi, W.y, Ar));
+                            Ai = fmaf(br, W.y, fmaf(bi, W.x, Ai));
+                        } else {
+                            const float br = -dot * q3;
+                            Ar = fmaf(br, W.x, Ar);
+                            Ai = fmaf(br, W.y, Ai);
+                        }
                     }
                 }
-                if constexpr (HELM) {
-                    Ar += er * W.x - ei * W.y;
-                    Ai += er * W.y + ei * W.x;
-                } else {
+            };
+            using std::integral_constant;
+            constexpr std::false_type series{};
+            // the folded series need k^10 / 10! in FP32 range (|k| < 1000)
+            const bool folded = kabs < 1000.f;
+            if (far) {
+                // the amplitude e^{ik delta} / r itself
+                const float r0k = r0 * kinv;
+#pragma unroll 4
+                for (int j = j0; j < j1; ++j) {
+                    const float4 U = shu[j];
+                    const float4 W = shw[j];
+                    const float tt = fmaf(tv0, U.x, fmaf(tv1, U.y, fmaf(tv2, U.z, U.w)));
+                    const float r2 = r0sq + tt;
+                    const float rinv = rsqrt_t(r2);
+                    float er = rinv, ei = 0.f;  // e^{ik(r - r0)} / r (Laplace: 1 / r)
+                    float r = 0.f;
+                    if constexpr (HELM) {
+                        r = r2 * rinv;
+                        float ph, amp = rinv;
+                        if constexpr (DAMP) {
+                            const float delta = tt * __builtin_amdgcn_rcpf(r + r0);
+                            ph = kr_rev * delta;
+                            amp *= __builtin_amdgcn_exp2f(-ki_log2e * delta);
+                        } else {
+                            ph = tt * __builtin_amdgcn_rcpf(r * kinv + r0k);
+                        }
+                        const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
+                        if constexpr (!DL) {
+                            // the weight times e^{ik(r - r0)} first, then one FMA by the amplitude
+                            Ar += amp * (cs * W.x - sn * W.y);
+                            Ai += amp * (cs * W.y + sn * W.x);
+                            continue;
+                        }
+                        er = cs * amp;
+                        ei = sn * amp;
+                    }
+                    if constexpr (DL) {
+                        // (1 - i k r) (x - y).n_y / r^2
+                        const float4 N = shn[j];
+                        const float f = (v0 * N.x + (v1 * N.y + (v2 * N.z + W.z))) * rinv * rinv;
+                        if constexpr (HELM) {
+                            const float ar = DAMP ? 1.f + ki_f * r : 1.f, ai = -kr_f * r;
+                            const float pr = (ar * er - ai * ei) * f, pi = (ar * ei + ai * er) * f;
+                            er = pr;
+                            ei = pi;
+                        } else {
+                            er *= f;
+                        }
+                    }
                     Ar += er * W.x;
                     Ai += er * W.y;
+                    if constexpr (HELM) {
+                        Ar -= ei * W.y;
+                        Ai += ei * W.x;
+                    }
+                }
+            } else if constexpr (!HELM) {
+                sources(integral_constant<int, 0>{}, series);
+            } else if (DAMP && fabsf(ki_f) * srad[g] > 0.24f) {
+                if (ymax <= 1.96f)
+                    sources(integral_constant<int, 3>{}, std::true_type{});
+                else
+                    sources(integral_constant<int, 4>{}, std::true_type{});
+            } else if (ymax <= 0.24f && folded) {
+                sources(integral_constant<int, 0>{}, series);
+            } else if (ymax <= 0.49f && folded) {
+                sources(integral_constant<int, 1>{}, series);
+            } else if (ymax <= 0.98f && folded) {
+                sources(integral_constant<int, 2>{}, series);
+            } else if (ymax <= 1.96f) {
+                sources(integral_constant<int, 3>{}, series);
+            } else {
+                sources(integral_constant<int, 4>{}, series);
+            }
+            // the group-centre term, plus the remainder, times e^{i k r0} (e^{-Im(k) r0}) in FP64
+            double cr = Ar, ci = Ai;
+            if (!far) {
+                if constexpr (DL) {
+                    const double nr = v0d * wsum[g][0] + v1d * wsum[g][2] + v2d * wsum[g][4] + wsum[g][6];
+                    const double ni = v0d * wsum[g][1] + v1d * wsum[g][3] + v2d * wsum[g][5] + wsum[g][7];
+                    cr += h0rd * nr - (HELM ? h0id * ni : 0.0);
+                    ci += h0rd * ni + (HELM ? h0id * nr : 0.0);
+                } else {
+                    cr += i0 * wsum[g][0];
+                    ci += i0 * wsum[g][1];
                 }
             }
-            // multiply the group's sum by e^{i k r0} (e^{-Im(k) r0}) in FP64
-            double pr = 1.0, pi = 0.0;
             if constexpr (HELM) {
                 double sn, cs;
                 sincos_fast(a.kr * r0d, &sn, &cs);
                 const double damp0 = DAMP ? exp(-a.ki * r0d) : 1.0;
-                pr = cs * damp0;
-                pi = sn * damp0;
+                const double pr = cs * damp0, pi = sn * damp0;
+                accr += pr * cr - pi * ci;
+                acci += pr * ci + pi * cr;
+            } else {
+                accr += cr;
+                acci += ci;
             }
-            accr += pr * Ar - pi * Ai;
-            acci += pr * Ai + pi * Ar;
         }
     }
     if (m < a.npts) {
@@ -1108,10 +1304,12 @@ __global__ __launch_bounds__(256) void potential_reduce_kernel(const PotArgs a, 
 // 228 -> 159 us. Beyond: 456 triangles, 11,869 points (517 workgroups, mixed) 159 us whole, 166 us split.
 constexpr int kPotWorkgroups = 4096, kPotSplitWorkgroups = 1024, kPotSplitWorkgroupsMixed = 512;
 
-// Scalar potentials of up to this many (point, source) pairs are evaluated in FP64 in either mode: the pairs
-// take less than the call's other launches (25 M pairs: 15 us Laplace, 40 us Helmholtz in FP64), and on meshes
-// that small the targets are close to the sources, where the FP32 path would be least accurate (720 triangles,
-// Laplace: 1.1e-7 against 3e-8 before, when most groups took the FP64 path one by one).
+// Scalar potentials of up to this many (point, source) pairs are evaluated in FP64 in either mode: most of such
+// a call are its launches and copies, and a target is close to most tiles of a mesh that small, where the mixed
+// kernel sums much of it in FP64 anyway (with loads per lane). Kernels, 25 to 30 M pairs, FP64 / mixed with points
+// 1.5 to 3 / 10 to 20 from the centre: 980 triangles, 5,000 points, Laplace single layer 37 / 34 / 25 us, Helmholtz
+// single layer 75 / 86 / 39, double layer 88 / 135 / 64 us; 5,120 triangles, 1,000 points 43 / 32 / 28, 80 / 63 / 45,
+// 92 / 112 / 67 us.
 constexpr int64_t kPotFp64Pairs = 3 << 23;
 
 static void plan(int npts, int nsrc, int precision, int *nchunk, int *chunk_len, int *nsrc_pad) {

@@ -86,3 +86,83 @@ def test_workspace_of_the_largest_batch_serves_smaller_ones(precision, hip_avail
                                           2.0, 0.0, mode, hb.ptr(out), hb.DTYPES["complex128"], hb.ptr(work), size,
                                           hb.stream_handle()))
         assert torch.isfinite(torch.view_as_real(out)).all()
+
+
+FP64_PAIRS = 3 << 23  # scalar potentials of up to this many (point, source) pairs are evaluated in FP64 in either mode
+
+
+def _mixed_error(space, family, name, k, points, seed):
+    """Error of the single precision potential of a random density against the double precision one."""
+    import bempp_amd.api as bempp
+
+    rng = np.random.default_rng(seed)
+    c = rng.standard_normal(space.global_dof_count)
+    if family == "helmholtz":
+        c = c + 1j * rng.standard_normal(space.global_dof_count)
+    fun = bempp.GridFunction(space, coefficients=c)
+    make = getattr(getattr(bempp.operators.potential, family), name)
+    single, double = (make(space, points, *(() if family == "laplace" else (k,)), precision=p).evaluate(fun)
+                      for p in ("single", "double"))
+    return np.linalg.norm(single - double) / np.linalg.norm(double)
+
+
+def _shell(count, low, high, seed=5):
+    rng = np.random.default_rng(seed)
+    points = rng.standard_normal((3, count))
+    return points * rng.uniform(low, high, count) / np.linalg.norm(points, axis=0)
+
+
+# 320 and 1,280 triangles: every target is close to its tiles of 43 triangles, away from most groups of 5 or 6
+@pytest.mark.parametrize("family,name,k", [("laplace", "single_layer", 0.0), ("laplace", "double_layer", 0.0),
+                                           ("helmholtz", "single_layer", 1.2), ("helmholtz", "double_layer", 1.2),
+                                           ("helmholtz", "single_layer", 1.2 + 0.12j),
+                                           ("helmholtz", "double_layer", 1.2 + 0.12j)])
+@pytest.mark.parametrize("level,count,low,high", [(2, 13200, 1.5, 3.0), (3, 3300, 1.02, 1.3)])
+@pytest.mark.parametrize("kind", ["P", "DP"])
+def test_mixed_rounds_the_result_only_close_to_the_mesh(kind, level, count, low, high, family, name, k, hip_available):
+    import bempp_amd.api as bempp
+    from bempp_amd.api.grid.shapes import icosphere
+
+    space = bempp.function_space(icosphere(level), kind, int(kind == "P"))
+    sources = 6 * space.grid.number_of_elements
+    assert sources * count > FP64_PAIRS
+    # the result's rounding to FP32, 2.5e-8 (2^-24 / sqrt 6), and a remainder of some tenths of the sum in FP32
+    assert _mixed_error(space, family, name, k, _shell(count, low, high), level) < 4e-8
+
+
+# 7,680 sources, 30 tiles. k h = 0.07 to 3.5 of a group's radius and beyond: all series of e^{ik delta} - 1, the
+# hardware sine, both forms of the damping
+@pytest.mark.parametrize("family,k", [("laplace", 0.0)] + [("helmholtz", k) for k in (0.5, 2.0, 5.0, 8.0, 12.0, 30.0, 2.0 + 0.5j,
+                                                                                      30.0 + 2.0j, 3.0 + 5.0j, 2.0 - 0.3j)])
+@pytest.mark.parametrize("name", ["single_layer", "double_layer"])
+@pytest.mark.parametrize("kind", ["P", "DP"])
+def test_mixed_scalar_at_every_distance(kind, name, family, k, hip_available):
+    import bempp_amd.api as bempp
+    from bempp_amd.api.grid.shapes import icosphere
+
+    space = bempp.function_space(icosphere(3), kind, int(kind == "P"))
+    for low, high in ((0.9, 1.1), (1.02, 1.05), (1.2, 2.5), (6.0, 12.0)):
+        points = _shell(3300, low, high)
+        assert 7680 * points.shape[1] > FP64_PAIRS
+        assert _mixed_error(space, family, name, k, points, 7) < 1e-6  # the mode's stated accuracy
+
+
+@pytest.mark.parametrize("family,name,k", [("laplace", "double_layer", 0.0), ("helmholtz", "single_layer", 6.0),
+                                           ("helmholtz", "double_layer", 4.0 + 0.4j)])
+def test_parts_of_a_tile_take_the_paths_of_the_tile(family, name, k, hip_available):
+    """30,720 sources: 1,024 points take parts of 128 sources, 9,216 points whole tiles of 256; the sums differ in
+    the order of FP64 additions only, so their roundings to FP32 by at most a unit."""
+    import bempp_amd.api as bempp
+    from bempp_amd.api.grid.shapes import icosphere
+
+    space = bempp.function_space(icosphere(4), "DP", 0)
+    rng = np.random.default_rng(3)
+    fun = bempp.GridFunction(space, coefficients=rng.standard_normal(space.global_dof_count))
+    points = _shell(9216, 1.02, 3.0)
+    assert 30720 * 1024 > FP64_PAIRS
+    make = getattr(getattr(bempp.operators.potential, family), name)
+    many, few = (make(space, np.ascontiguousarray(points[:, :n]), *(() if family == "laplace" else (k,)),
+                      precision="single").evaluate(fun) for n in (9216, 1024))
+    many = many[:, :1024]
+    for a, b in ((few.real, many.real), (few.imag, many.imag)):
+        np.testing.assert_array_max_ulp(a.astype(np.float32), b.astype(np.float32), maxulp=1)
