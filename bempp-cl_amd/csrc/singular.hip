@@ -31,11 +31,10 @@ struct SingularArgs {
 };
 
 // LDS of one workgroup: the staged points, then the partial moments and the local blocks
-template <int NV, int W, int G>
+template <int NV, int W, int G, int L>
 union SingularShared {
-    // points a wave stages at a time, with their loads in flight together: a vertex pair's part (128) in one
-    // step; one load each where the lanes take all of them (10 registers less)
-    static constexpr int kLoads = G == 1 ? 1 : 2, kChunk = 64 * kLoads;
+    // points a wave stages at a time, with their loads in flight together
+    static constexpr int kLoads = L, kChunk = 64 * kLoads;
     struct {
         double2 points[W][kChunk][2];  // (xi_0, xi_1), (eta_0, eta_1)
         double weights[W][kChunk];
@@ -45,12 +44,12 @@ union SingularShared {
 
 // DUAL: OP is a single layer; the double layer of the same family (sharing r and e^{ikr} at
 // every point) goes to a.out2.
-template <int OP, int NTS, int NSS, typename OutT, bool DUAL, int W, int G>
-__global__ __launch_bounds__(64 * W, !(DUAL && NTS * NSS == 9) ? 3 : 2) void singular_kernel(const SingularArgs a) {
+template <int OP, int NTS, int NSS, typename OutT, bool DUAL, int W, int G, int L>
+__global__ __launch_bounds__(64 * W, (DUAL && NTS * NSS == 9) || L > 2 ? 2 : 3) void singular_kernel(const SingularArgs a) {
     constexpr bool CPLX = OpTraits<OP>::is_complex;
     constexpr int NC = CPLX ? 2 : 1, NB = NTS * NSS, NV = NB * NC, NOPS = DUAL ? 2 : 1;
     constexpr int PP = 64 / G;  // pairs per workgroup
-    using Shared = SingularShared<NV, W, G>;
+    using Shared = SingularShared<NV, W, G, L>;
     __shared__ Shared sh;
     __shared__ int32_t rows[NTS][PP], cols[NSS][PP];
     __shared__ double mult[NTS + NSS][PP];
@@ -231,10 +230,8 @@ __global__ __launch_bounds__(64 * W, !(DUAL && NTS * NSS == 9) ? 3 : 2) void sin
                 M[i][j].re = sh.moments[0][(i * NSS + j) * NC][p];
                 M[i][j].im = CPLX ? sh.moments[0][(i * NSS + j) * NC + NC - 1][p] : 0.0;
             }
-        // entry l is formed by wave l % W (lanes of sub 0)
-#pragma unroll
-        for (int l = 0; l < NB; ++l) {
-            if (l % W != wave || sub != 0) continue;
+        // the W G lanes of a pair share its entries
+        for (int l = wave * G + sub; l < NB; l += W * G) {
             const int i = l / NSS, j = l % NSS;
             const double m = mult[i][p] * mult[NTS + j][p];
             C2d v = {0.0, 0.0};
@@ -261,47 +258,53 @@ __global__ __launch_bounds__(64 * W, !(DUAL && NTS * NSS == 9) ? 3 : 2) void sin
     }
 }
 
-// Lanes of a wave per pair (G) and waves (W): the points of a pair are split W G ways. The coincident
-// pairs' lanes form the longest chain (1536 / (W G) points), a split costs the set-up of more workgroups.
-// Few pairs also leave waves whose pairs follow several rules; one rule after the other, with the other
-// lanes idle, doubled and more the longest chain (6,400 pairs, electric field, (4, 4): 54 against 32 us).
-// Kernel times with (W, G) = (4, 1) / (4, 4) / (4, 8) / (4, 16), against lanes striding over a pair's
-// points with loads of their own before:
-//   203,800 pairs, Helmholtz double layer P1, FP64:     430 / 464 / 526 / 720 us
-//    66,500 pairs, the same:                            165 / 157 / 174 / 257 us
-//    12,700 pairs, the same:                             96 /  41 /  43 /  58 us
-//     6,400 pairs, the same:                            103 /  34 /  30 /  36 us
-//     2,300 pairs, the same:                            104 /  33 /  22 /  21 us
-//   203,800 pairs, electric field operator:             382 / 447 / 492 / 729 us
-//    66,500 pairs, the same:                            135 / 149 / 168 / 244 us (305)
-//     6,400 pairs, Helmholtz DP0, FP64, damped:         112 /  37 /  27 /  27 us (55)
-//     2,300 pairs, Laplace DP0, FP64:                    52 /  18 /  13 /   9 us
-// The electric field operator's local blocks take longer (one lane per pair and entry), so that it
-// prefers many pairs per wave earlier.
-constexpr int kSingLargePairs = 131072, kSingLargePairsEfie = 49152, kSingMediumPairs = 10240, kSingSmallPairs = 3072;
+// Lanes of a wave per pair (G), waves (W = 4) and loads in flight per lane (L). The points of a pair are split
+// W G ways. The coincident pairs' lanes form the longest chain (1536 / (W G) points), a split costs the set-up
+// of more workgroups. Few pairs also leave waves whose pairs follow several rules; one rule after the other,
+// with the other lanes idle, doubled and more the longest chain (6,400 pairs, electric field, G = 4: 54 against
+// 32 us). Kernel times, G = 16 / 8 / 4 / 1, against lanes striding over a pair's points with loads of their
+// own before (32 lanes a pair below 32,768 pairs, else 8), us:
+//    pairs     Laplace P1 FP64       Laplace DP0 FP64     Helmholtz P1 SL + DL  electric field         Helmholtz DL P1 FP64
+//     2,280   11/ 14/ 19  (14)       9/ 13/ 18  (12)      22/ 25/ 38  (28)     19/ 20/ 30  (21)      20/ 21/ 32  (23)
+//     6,440   20/ 16/ 21  (19)      17/ 14/ 19  (17)      45/ 36/ 40  (46)     31/ 27/ 32  (31)      33/ 28/ 33  (43)
+//    12,680   30/ 25/ 27/ 59 (29)   25/ 20/ 21/ 53 (25)   77/ 54/ 52/110 (65)  52/ 42/ 43/ 96 (52)   50/ 40/ 40/ 94 (59)
+//    21,000   44/ 37/ 41/ 62 (45)   37/ 25/ 24/ 53 (38)  121/ 83/ 72/112 (102) 76/ 58/ 59/ 97 (103)  75/ 59/ 59/ 96 (89)
+//    43,880   83/ 60/ 55/ 68 (75)   70/ 44/ 40/ 57 (68)  244/162/139/147 (177) 142/105/ 98/106 (140) 147/114/107/117 (155)
+//    66,500       92/ 86/ 92 (109)      67/ 62/ 75 (91)      254/219/201 (257)     165/150/140 (206)     181/165/171 (226)
+//   103,940      143/126/123 (157)     101/ 90/ 93 (136)     395/336/305 (404)     254/230/211 (306)     277/252/236 (346)
+//   203,780      275/242/225 (284)     196/171/162 (243)     767/650/587 (735)     488/442/399 (584)     540/484/449 (644)
+// G = 8 up to kSingMediumPairs (real operators kSingMediumPairsReal: 12,680 pairs, Laplace double layer 29.1 / 31.0,
+// single and double layer 34.2 / 37.0 us with G = 8 / 4). The electric field operator takes G = 1 earlier.
+// L: a vertex pair's part (128 points) in one step of two loads; G = 1 one load (10 registers less). Up to
+// kSingWholePairs the chip holds at most two workgroups per CU, nothing hides the latency of a step, and a wave
+// loads its whole part (384 points, 61 KB of LDS) at once. L = 2 / 6: 4,100 pairs, Helmholtz hypersingular
+// 25.1 / 19.6 (22.0), electric field 22.4 / 19.3 (21.2), Laplace single and double layer 18.2 / 16.3 us (17.0);
+// 4,500 pairs 26.5 / 20.8, 23.5 / 19.9, 20.1 / 18.3; 5,400 pairs 26.6 / 26.3, 23.5 / 25.8, 19.7 / 22.7 us.
+constexpr int kSingLargePairs = 131072, kSingLargePairsEfie = 49152, kSingMediumPairs = 10240,
+              kSingMediumPairsReal = 16384, kSingWholePairs = 4608, kSingSmallPairs = 3072;
 
-template <int OP, typename OutT, bool DUAL, int W, int G>
+template <int OP, typename OutT, bool DUAL, int W, int G, int L>
 static int launch_sing_split(const SingularArgs &a, hipStream_t s) {
     constexpr int PP = 64 / G;
     const dim3 grid((unsigned)(((int64_t)a.n_pairs + PP - 1) / PP)), threads(64 * W);
     if constexpr (OP == kMaxwellEFIE) {
-        hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, false, W, G>), grid, threads, 0, s, a);
+        hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, false, W, G, L>), grid, threads, 0, s, a);
     } else if constexpr (is_hypersingular<OP>()) {
         if (nshape_of(a.test.shape) != 3 || nshape_of(a.trial.shape) != 3) {
             set_error("hypersingular operators need P1 shape functions on both sides");
             return BEM_ERR_INVALID_ARGUMENT;
         }
-        hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, false, W, G>), grid, threads, 0, s, a);
+        hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, false, W, G, L>), grid, threads, 0, s, a);
     } else {
         int nt = nshape_of(a.test.shape), ns = nshape_of(a.trial.shape);
         if (nt == 1 && ns == 1)
-            hipLaunchKernelGGL((singular_kernel<OP, 1, 1, OutT, DUAL, W, G>), grid, threads, 0, s, a);
+            hipLaunchKernelGGL((singular_kernel<OP, 1, 1, OutT, DUAL, W, G, L>), grid, threads, 0, s, a);
         else if (nt == 1 && ns == 3)
-            hipLaunchKernelGGL((singular_kernel<OP, 1, 3, OutT, DUAL, W, G>), grid, threads, 0, s, a);
+            hipLaunchKernelGGL((singular_kernel<OP, 1, 3, OutT, DUAL, W, G, L>), grid, threads, 0, s, a);
         else if (nt == 3 && ns == 1)
-            hipLaunchKernelGGL((singular_kernel<OP, 3, 1, OutT, DUAL, W, G>), grid, threads, 0, s, a);
+            hipLaunchKernelGGL((singular_kernel<OP, 3, 1, OutT, DUAL, W, G, L>), grid, threads, 0, s, a);
         else
-            hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, DUAL, W, G>), grid, threads, 0, s, a);
+            hipLaunchKernelGGL((singular_kernel<OP, 3, 3, OutT, DUAL, W, G, L>), grid, threads, 0, s, a);
     }
     return check_launch("singular_kernel");
 }
@@ -310,10 +313,12 @@ template <int OP, typename OutT, bool DUAL>
 static int launch_sing(const SingularArgs &a, hipStream_t s) {
     if (a.n_pairs == 0) return BEM_OK;
     if (a.n_pairs >= (OP == kMaxwellEFIE ? kSingLargePairsEfie : kSingLargePairs))
-        return launch_sing_split<OP, OutT, DUAL, 4, 1>(a, s);
-    if (a.n_pairs >= kSingMediumPairs) return launch_sing_split<OP, OutT, DUAL, 4, 4>(a, s);
-    if (a.n_pairs >= kSingSmallPairs) return launch_sing_split<OP, OutT, DUAL, 4, 8>(a, s);
-    return launch_sing_split<OP, OutT, DUAL, 4, 16>(a, s);
+        return launch_sing_split<OP, OutT, DUAL, 4, 1, 1>(a, s);
+    if (a.n_pairs >= (OpTraits<OP>::is_complex ? kSingMediumPairs : kSingMediumPairsReal))
+        return launch_sing_split<OP, OutT, DUAL, 4, 4, 2>(a, s);
+    if (a.n_pairs >= kSingWholePairs) return launch_sing_split<OP, OutT, DUAL, 4, 8, 2>(a, s);
+    if (a.n_pairs >= kSingSmallPairs) return launch_sing_split<OP, OutT, DUAL, 4, 8, 6>(a, s);
+    return launch_sing_split<OP, OutT, DUAL, 4, 16, 2>(a, s);
 }
 
 template <int OP, bool DUAL = false>

@@ -8,13 +8,16 @@ pytestmark = pytest.mark.gpu
 
 
 # 3, 63 and 3,071 pairs: the smallest launches and their last workgroup (4 pairs, remainder 3); 3,072 to
-# 10,239: 8 pairs per workgroup; 10,241: 16 pairs, remainder 1; 49,153 (electric field) and 131,073: one lane per pair (64 pairs,
-# remainder 1)
+# 4,607 and 4,608 to 10,239 (Laplace 16,383): 8 pairs per workgroup, whole parts and chunks of points; 10,241:
+# 16 pairs, remainder 1; 49,153 (electric field) and 131,073: one lane per pair (64 pairs, remainder 1). Order 2:
+# up to 96 points a pair, less than one chunk; order 5: 3,750, several chunks of 64, 128 and 384 points
 @pytest.mark.parametrize("op,space,k", [("laplace_single_layer", "P1", 0.0), ("helmholtz_double_layer", "DP0", 2.0),
                                         ("helmholtz_hypersingular", "P1", 2.0 + 0.3j),
                                         ("maxwell_electric_field", "RWG", 3.0)])
-@pytest.mark.parametrize("count", [3, 63, 3071, 3072, 4095, 4096, 10239, 10241, 15777, 49153, 131073])
-def test_singular_pairs_in_any_order(op, space, k, count, hip_available):
+@pytest.mark.parametrize("count,order", [(c, 2) for c in (3, 63, 3071, 3072, 4095, 4096, 4607, 4608, 10239, 10241, 15777, 16383,
+                                                          16385, 49153, 131073)] +
+                         [(c, 5) for c in (65, 3073, 4609, 10241, 16385, 49153, 131073)])
+def test_singular_pairs_in_any_order(op, space, k, count, order, hip_available):
     """A table of `count` pairs gives the same sum whether the pairs of one rule stand together (every
     wave reads one set of points) or the table is shuffled (every wave runs many rules)."""
     import torch
@@ -26,7 +29,7 @@ def test_singular_pairs_in_any_order(op, space, k, count, hip_available):
 
     grid = icosphere(3 if count <= 15777 else 5)
     sp = function_space(grid, *{"P1": ("P", 1), "DP0": ("DP", 0), "RWG": ("RWG", 0)}[space])
-    rule = singular_rule(grid, 2, sp.support, sp.support)
+    rule = singular_rule(grid, order, sp.support, sp.support)
     rng = np.random.default_rng(count)
     chosen = np.sort(rng.permutation(len(rule.host.pairs))[:count])
     complex_op = not op.startswith("laplace")
