@@ -514,8 +514,8 @@ __global__ __launch_bounds__(64 * kSingWaves, 3) void adjoint_singular_kernel(co
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 for (int k = lane; k < count; k += 64) {
                     const int64_t kk = kb + k;
-                    sh.points[wave][k][0] = *reinterpret_cast<const double2 *>(tpts + 2 * (to + kk));
-                    sh.points[wave][k][1] = *reinterpret_cast<const double2 *>(spts + 2 * (so + kk));
+                    sh.points[wave][k][0] = load_pair(tpts + 2 * (to + kk));
+                    sh.points[wave][k][1] = load_pair(spts + 2 * (so + kk));
                     sh.points[wave][k][2].x = wts[wo + kk];
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

@@ -57,6 +57,13 @@ struct OpTraits {
     static constexpr bool needs_test_normal = OP == kLaplaceADL || OP == kHelmholtzADL;
 };
 
+// Two consecutive doubles of a caller's table, which is aligned to 8 bytes only, in one load.
+__device__ __forceinline__ double2 load_pair(const double *p) {
+    using Pair = double __attribute__((ext_vector_type(2), aligned(8)));
+    const Pair v = *reinterpret_cast<const Pair *>(p);
+    return make_double2(v.x, v.y);
+}
+
 // 1 / sqrt(x) for positive normal x: the hardware estimate y (v_rsq_f64, relative error up to about
 // 1e-5) with one fourth-order correction, 1 / sqrt(x) = y (1 - e)^(-1/2) =
 // y (1 + e / 2 + 3 e^2 / 8 + 5 e^3 / 16 + O(e^4)), e = 1 - x y^2 (remainder 35 e^4 / 128, below 1e-19).

@@ -544,7 +544,7 @@ __device__ __forceinline__ void singular_points(const SingularPair &P, int lane,
     const double *gt = P.gt, *gf = P.gf;
 #pragma unroll 2
     for (int kk = lane; kk < P.np; kk += W) {
-        const double2 x = reinterpret_cast<const double2 *>(P.tp)[kk], y = reinterpret_cast<const double2 *>(P.sp)[kk];
+        const double2 x = load_pair(P.tp + 2 * kk), y = load_pair(P.sp + 2 * kk);
         const double dx = (gf[0] + gf[3] * y.x + gf[6] * y.y) - (gt[0] + gt[3] * x.x + gt[6] * x.y);
         const double dy = (gf[1] + gf[4] * y.x + gf[7] * y.y) - (gt[1] + gt[4] * x.x + gt[7] * x.y);
         const double dz = (gf[2] + gf[5] * y.x + gf[8] * y.y) - (gt[2] + gt[5] * x.x + gt[8] * x.y);

@@ -136,8 +136,8 @@ __global__ __launch_bounds__(64 * W, (DUAL && NTS * NSS == 9) || L > 2 ? 2 : 3) 
             if (active) {
                 const int per = (np + W - 1) / W, k1 = min((wave + 1) * per, np);
                 for (int k = wave * per + sub; k < k1; k += G) {
-                    const double2 px = *reinterpret_cast<const double2 *>(a.tpts + 2 * ((int64_t)toff + k));
-                    const double2 py = *reinterpret_cast<const double2 *>(a.spts + 2 * ((int64_t)soff + k));
+                    const double2 px = load_pair(a.tpts + 2 * ((int64_t)toff + k));
+                    const double2 py = load_pair(a.spts + 2 * ((int64_t)soff + k));
                     point(px.x, px.y, py.x, py.y, a.wts[(int64_t)woff + k]);
                 }
             }
@@ -153,8 +153,8 @@ __global__ __launch_bounds__(64 * W, (DUAL && NTS * NSS == 9) || L > 2 ? 2 : 3) 
 #pragma unroll
             for (int u = 0; u < Shared::kLoads; ++u) {
                 const int64_t kk = kb + min(64 * u + lane, count - 1);
-                xt[u] = *reinterpret_cast<const double2 *>(a.tpts + 2 * (to + kk));
-                xs[u] = *reinterpret_cast<const double2 *>(a.spts + 2 * (so + kk));
+                xt[u] = load_pair(a.tpts + 2 * (to + kk));
+                xs[u] = load_pair(a.spts + 2 * (so + kk));
                 xw[u] = a.wts[wo + kk];
             }
 #pragma unroll

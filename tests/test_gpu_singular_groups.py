@@ -44,3 +44,36 @@ def test_singular_pairs_in_any_order(op, space, k, count, order, hip_available):
     assert torch.linalg.norm(results[0]) > 0
     # the same FP64 terms in another order of the atomics: a few roundings per entry
     assert torch.linalg.norm(results[0] - results[1]) < 1e-14 * torch.linalg.norm(results[0])
+
+
+@pytest.mark.parametrize("op,space,count", [("laplace_single_layer", "DP0", 500), ("helmholtz_double_layer", "P1", 3500),
+                                            ("maxwell_electric_field", "RWG", 12000)])
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_point_tables_of_any_double_alignment(op, space, count, shuffled, hip_available):
+    """The points of the rules may start at any double, not only at a multiple of 16 bytes."""
+    import torch
+
+    from bempp_amd.api import function_space
+    from bempp_amd.api.grid.shapes import icosphere
+    from bempp_amd.core import hip_backend as hb
+    from bempp_amd.core.singular_assembler import singular_rule
+
+    sp = function_space(icosphere(3), *{"P1": ("P", 1), "DP0": ("DP", 0), "RWG": ("RWG", 0)}[space])
+    rule = singular_rule(sp.grid, 4, sp.support, sp.support)
+    pairs = rule.pairs[torch.randperm(count, generator=torch.Generator().manual_seed(1)) if shuffled else slice(count)]
+    pairs = pairs.contiguous()
+
+    def shifted(table):
+        out = torch.empty(table.numel() + 1, dtype=torch.float64, device=table.device)[1:]
+        return out.copy_(table.reshape(-1))
+
+    results = []
+    for points in ((rule.test_points, rule.trial_points), (shifted(rule.test_points), shifted(rule.trial_points))):
+        out = torch.zeros((sp.global_dof_count,) * 2, dtype=torch.complex128 if "laplace" not in op else torch.float64,
+                          device=hb.device())
+        ds = hb.device_space(sp)
+        hb.singular_assemble(op, ds, ds, pairs, *points, rule.weights, 2.0, out)
+        results.append(out)
+    assert points[0].data_ptr() % 16 == 8
+    # the same terms, only the order of the atomics may differ
+    assert torch.linalg.norm(results[0] - results[1]) < 1e-14 * torch.linalg.norm(results[0])
