@@ -23,6 +23,13 @@ _EDGE_OFFSET_INDEX = _np.array([[-1, 0, 4], [1, -1, 2], [5, 3, -1]])
 _CACHE = {}
 
 
+def _by_rule(adjacency, test_support, trial_support, rules):
+    """Columns of an adjacency table whose elements are in the supports, in the order of their rules (0..63)."""
+    columns = _np.flatnonzero(test_support[adjacency[0]] & trial_support[adjacency[1]])
+    # one gather for the selection and the order; the sort of bytes is linear
+    return adjacency.take(columns[rules[columns].astype(_np.uint8).argsort(kind="stable")], axis=1)
+
+
 class SingularRule(object):
     """Host arrays of all singular pairs of a grid for given supports."""
 
@@ -45,41 +52,34 @@ class SingularRule(object):
         self.weights = _np.hstack([co_w, ed_w, ve_w])
 
         coincident = _np.flatnonzero(test_support & trial_support)
+        # the pairs of one rule (kind and local vertices) together, the kinds in order: the device kernel
+        # reads a rule's points once for its consecutive pairs
         ea = grid.edge_adjacency
-        ea = ea[:, test_support[ea[0]] & trial_support[ea[1]]]
+        ea = _by_rule(ea, test_support, trial_support,
+                      _EDGE_OFFSET_INDEX.take(3 * ea[2] + ea[3]) * 6 + _EDGE_OFFSET_INDEX.take(3 * ea[4] + ea[5]))
         va = grid.vertex_adjacency
-        va = va[:, test_support[va[0]] & trial_support[va[1]]]
+        va = _by_rule(va, test_support, trial_support, 3 * va[2] + va[3])
 
-        edge_offsets = nco + ned * _EDGE_OFFSET_INDEX
-        vertex_offsets = nco + 6 * ned + nve * _np.arange(3)
+        edge_offsets = (nco + ned * _EDGE_OFFSET_INDEX).astype(_np.int32)
+        vertex_offsets = (nco + 6 * ned + nve * _np.arange(3)).astype(_np.int32)
 
         n = len(coincident) + ea.shape[1] + va.shape[1]
-        pairs = _np.zeros((n, 6), dtype=_np.int32)
+        pairs = _np.empty((n, 6), dtype=_np.int32)
         i0, i1 = len(coincident), len(coincident) + ea.shape[1]
         pairs[:i0, 0] = coincident
         pairs[:i0, 1] = coincident
-        pairs[:i0, 2] = 0
-        pairs[:i0, 3] = 0
-        pairs[:i0, 4] = 0
-        pairs[:i0, 5] = nco
+        pairs[:i0, 2:] = (0, 0, 0, nco)
         pairs[i0:i1, 0] = ea[0]
         pairs[i0:i1, 1] = ea[1]
-        pairs[i0:i1, 2] = edge_offsets[ea[2], ea[3]]
-        pairs[i0:i1, 3] = edge_offsets[ea[4], ea[5]]
-        pairs[i0:i1, 4] = nco
-        pairs[i0:i1, 5] = ned
+        pairs[i0:i1, 2] = edge_offsets.take(3 * ea[2] + ea[3])
+        pairs[i0:i1, 3] = edge_offsets.take(3 * ea[4] + ea[5])
+        pairs[i0:i1, 4:] = (nco, ned)
         pairs[i1:, 0] = va[0]
         pairs[i1:, 1] = va[1]
-        pairs[i1:, 2] = vertex_offsets[va[2]]
-        pairs[i1:, 3] = vertex_offsets[va[3]]
-        pairs[i1:, 4] = nco + ned
-        pairs[i1:, 5] = nve
-        # pairs of one rule (kind and local vertices) together, the kinds in order: the device kernel
-        # reads a rule's points once for 64 consecutive pairs
-        rules = _np.zeros(n, dtype=_np.int16)
-        rules[i0:i1] = 1 + 6 * _EDGE_OFFSET_INDEX[ea[2], ea[3]] + _EDGE_OFFSET_INDEX[ea[4], ea[5]]
-        rules[i1:] = 37 + 3 * va[2] + va[3]
-        self.pairs = pairs[_np.argsort(rules, kind="stable")]
+        pairs[i1:, 2] = vertex_offsets.take(va[2])
+        pairs[i1:, 3] = vertex_offsets.take(va[3])
+        pairs[i1:, 4:] = (nco + ned, nve)
+        self.pairs = pairs
         self.counts = {"coincident": i0, "edge_adjacent": i1 - i0, "vertex_adjacent": n - i1}
 
     @property

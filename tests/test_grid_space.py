@@ -119,3 +119,24 @@ def test_gmsh_roundtrip(tmp_path, sphere_grid):
     g = import_grid(fname)
     np.testing.assert_allclose(g.vertices, sphere_grid.vertices)
     assert np.array_equal(g.elements, sphere_grid.elements)
+
+
+@pytest.mark.parametrize("share", [1.0, 0.5, 0.0])
+def test_singular_pairs_of_one_rule_stand_together(share):
+    """The pair table: every element pair that shares a vertex and lies in the supports once, coincident, edge and
+    vertex pairs in this order, and the pairs of one rule in one run."""
+    from bempp_amd.api.grid.shapes import icosphere
+    from bempp_amd.core.singular_assembler import SingularRule
+
+    grid = icosphere(1)
+    rng = np.random.default_rng(2)
+    test, trial = (rng.random(grid.number_of_elements) < share for _ in range(2))
+    rule = SingularRule(grid, 3, test, trial)
+    el = grid.elements
+    shared = (el[:, None, :, None] == el[None, :, None, :]).sum(axis=(0, 1))
+    expected = {(e, f): shared[e, f] for e in np.flatnonzero(test) for f in np.flatnonzero(trial) if shared[e, f]}
+    got = {(e, f): kind for (e, f), kind in zip(rule.pairs[:, :2].tolist(),
+                                                np.repeat([3, 2, 1], list(rule.counts.values())).tolist())}
+    assert got == expected and len(rule.pairs) == len(expected)
+    runs = 1 + np.count_nonzero((np.diff(rule.pairs[:, 2:], axis=0) != 0).any(axis=1)) if len(rule.pairs) else 0
+    assert runs == len(np.unique(rule.pairs[:, 2:], axis=0))
