@@ -134,13 +134,15 @@ def _krylov_gmres(matvec, b, dev, rtol, restart, maxiter, callback, matrix):
 
         def issue(c):
             b = c % 2
+            # the step and the event that the host waits for belong on one stream, which a callback may change
+            stream = torch.cuda.current_stream()
             if step is not None:
-                step(c + 1, b)
+                step(c + 1, b, stream)
             else:
                 wv = matvec(V[c]).to(torch.complex128).contiguous()
                 hb.gmres_cgs2(V, c + 1, wv, gs_out[b], V[c + 1], eps)
                 gs_host[b][: 2 * c + 4].copy_(gs_out[b][: 2 * c + 4], non_blocking=True)
-            gs_event[b].record()
+            gs_event[b].record(stream)
 
     h = _np.zeros((restart, restart + 1), dtype=_np.complex128)
     gc, gs = [0.0] * restart, [0j] * restart  # Givens rotations (c real, s complex)

@@ -453,7 +453,8 @@ def gmres_cgs2(V, k, w, out, v_next=None, eps=0.0):
 
 
 def gmres_stepper(A, V, w, out, host, eps):
-    """step(k, b): one Arnoldi step of GMRES on the current stream in one library call (w = A V[k - 1], CGS2 of
+    """step(k, b, stream): one Arnoldi step of GMRES on a stream (default: the current one) in one library call
+    (w = A V[k - 1], CGS2 of
     w against V[:k], next basis vector into V[k], the 2k + 2 coefficients into the page-locked tensor host[b]).
     The checks are made and the addresses read once per solve; the function keeps the tensors alive. The copy
     to host[b] is the library's: host memory of torch's allocator must stay alive until the stream has done it."""
@@ -472,11 +473,11 @@ def gmres_stepper(A, V, w, out, host, eps):
 
     keep = (A, V, w, tuple(out), tuple(host))
 
-    def step(k, b, keep=keep):
+    def step(k, b, stream=None, keep=keep):
         if not 1 <= k < m:
             raise ValueError("k must leave a row of V for the next basis vector")
-        # the stream of this step, on which the caller records the event that it waits for
-        check(fn(a, dtype, n, ld, v, n, k, wp, outs[b], hosts[b], eps, stream_handle()))
+        handle = stream_handle() if stream is None else ctypes.c_void_p(stream.cuda_stream)
+        check(fn(a, dtype, n, ld, v, n, k, wp, outs[b], hosts[b], eps, handle))
 
     return step
 

@@ -308,9 +308,9 @@ def _delayed_stepper(monkeypatch, cycles):
     def delayed(*args):
         step = make(*args)
 
-        def slow(k, b):
+        def slow(*args):
             torch.cuda._sleep(cycles)
-            step(k, b)
+            step(*args)
 
         return slow
 
