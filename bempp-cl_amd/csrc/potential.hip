@@ -1411,17 +1411,18 @@ extern "C" size_t bem_potential_workspace_size(int op, const bem_space_t *space,
                                                int n_points, int precision) {
     if (!space || !rule || n_points < 0) return 0;
     const int nsrc = space->n_elements * rule->n_points, kd = is_vector_potential_op(op) ? 3 : 1;
-    (void)precision;  // one size for both: the FP64 plan has at least as many chunks
     size_t size = 0;
-    int nchunk, chunk_len, nsrc_pad;
-    // the plan depends on the number of target blocks, and is one chunk from kPotWorkgroups blocks on
-    const int blocks = n_points / kPotThreads;
-    for (int b = 1; b <= min(blocks, kPotWorkgroups); ++b) {
-        plan(b * kPotThreads, nsrc, BEM_PRECISION_FP64, &nchunk, &chunk_len, &nsrc_pad);
-        size = std::max(size, workspace_bytes(kd, nsrc_pad, nchunk, b * kPotThreads));
-    }
-    plan(n_points, nsrc, BEM_PRECISION_FP64, &nchunk, &chunk_len, &nsrc_pad);
-    return std::max(size, workspace_bytes(kd, nsrc_pad, nchunk, n_points));
+    // the plan depends on the number of target blocks, and is one chunk from kPotWorkgroups blocks on; the
+    // precision of a block's smallest count has at least as many chunks as the others'
+    auto up_to = [&](int block, int points) {
+        const int smallest = max(0, block - 1) * kPotThreads + 1;
+        int nchunk, chunk_len, nsrc_pad;
+        plan(points, nsrc, evaluated_precision(op, nsrc, smallest, precision), &nchunk, &chunk_len, &nsrc_pad);
+        size = std::max(size, workspace_bytes(kd, nsrc_pad, nchunk, points));
+    };
+    for (int b = 1; b <= min(n_points / kPotThreads, kPotWorkgroups); ++b) up_to(b, b * kPotThreads);
+    up_to((n_points + kPotThreads - 1) / kPotThreads, n_points);
+    return size;
 }
 
 // Checks, workspace layout and launches of bem_potential_evaluate.

@@ -281,7 +281,7 @@ int bem_singular_assemble_sl_dl(int op, const bem_space_t *test, const bem_space
  * Only BEM_LAPLACE_SINGLE_LAYER, BEM_LAPLACE_DOUBLE_LAYER, BEM_HELMHOLTZ_SINGLE_LAYER,
  * BEM_HELMHOLTZ_DOUBLE_LAYER and BEM_MAXWELL_ELECTRIC_FIELD are potentials.
  * workspace: device memory of at least bem_potential_workspace_size(...) bytes, the size for any
- *   call of up to n_points points (in either precision).
+ *   call of up to n_points points in this precision.
  */
 size_t bem_potential_workspace_size(int op, const bem_space_t *space, const bem_quad_rule_t *rule, int n_points,
                                     int precision);
