@@ -440,6 +440,14 @@ def test_potentials_edge_point_sets(op, sk, k, ico2, default_parameters, hip_ava
               flush=True)
         assert err64 < 1e-12
         assert err32 < 1e-6
+    if kdim == 1:
+        # small calls of scalar potentials run in FP64 in either precision: as many points as the mixed kernel takes
+        g = rng.standard_normal((3, 13200))
+        near = 1.05 * g / np.linalg.norm(g, axis=0)
+        assert 6 * ico2.number_of_elements * near.shape[1] > 3 << 23
+        u64, u32 = (factory(space, near, k, parameters=default_parameters, precision=p).evaluate(fun)
+                    for p in ("double", "single"))
+        assert rel_fro(u32, u64) < 1e-6
 
 
 @pytest.mark.parametrize("radius", [1.02, 1.2])
@@ -490,7 +498,7 @@ def test_mixed_potentials_large_wavenumber(k, hip_available):
         rwg.global_dof_count))
     fp = bempp.GridFunction(p1, coefficients=rng.standard_normal(p1.global_dof_count) + 1j * rng.standard_normal(
         p1.global_dof_count))
-    x = rng.standard_normal((3, 400))
+    x = rng.standard_normal((3, 3300))  # 25.3 M (point, source) pairs: scalar potentials of fewer run in FP64
     xh = x / np.linalg.norm(x, axis=0)
     cases = [(P.maxwell.electric_field, rwg, fr, 2 * xh), (P.maxwell.magnetic_field, rwg, fr, 2 * xh),
              (P.helmholtz.single_layer, p1, fp, 2 * xh), (P.helmholtz.double_layer, p1, fp, 1.05 * xh)]

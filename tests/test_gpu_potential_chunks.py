@@ -6,8 +6,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-# 320 triangles: 1,920 sources, 8 tiles of 256. 32,768 points fill the chip with whole tiles; 1 and 255 points
-# take chunks of 32, 2,049 points of 64, 16,385 points of 128 sources. 20 triangles: 120 sources, less than a tile
+# 320 triangles: 1,920 sources, 8 tiles of 256. 32,768 points fill the chip with whole tiles; 1, 255 and 2,049
+# points take chunks of 32, 8,193 points of 64, 16,385 points of 128 sources. 20 triangles: 120 sources, less than a tile
 @pytest.mark.parametrize("family,name,k", [("laplace", "double_layer", 0.0), ("helmholtz", "single_layer", 2.0),
                                            ("helmholtz", "double_layer", 2.0 + 0.5j),
                                            ("maxwell", "electric_field", 1.5 + 0.2j),
@@ -30,7 +30,7 @@ def test_few_points_equal_many(family, name, k, level, hip_available):
         return make(space, np.ascontiguousarray(x), *options, precision="double").evaluate(fun)
 
     many = evaluate(points)
-    for count in (1, 255, 2049, 16385):
+    for count in (1, 255, 2049, 8193, 16385):
         few = evaluate(points[:, :count])
         # the same terms summed in another grouping: about sqrt(1,920) roundings of terms that partly cancel
         assert np.linalg.norm(few - many[:, :count]) < 1e-13 * np.linalg.norm(many[:, :count])

@@ -71,6 +71,25 @@ def test_noalloc_matches_workspace_entry(op, kind, degree, precision_name):
         np.testing.assert_array_equal(out, ref)
 
 
+def _mixed_pairs(level, n_points):
+    return 20 * 4**level * 6 * n_points
+
+
+@pytest.mark.parametrize("op,kind,degree", [("helmholtz_single_layer", "P", 1), ("helmholtz_double_layer", "DP", 0)])
+def test_noalloc_matches_workspace_entry_mixed_scalar(op, kind, degree):
+    """As above, with so many (point, source) pairs that scalar potentials are not evaluated in FP64."""
+    import bempp_amd.api as bempp
+    from bempp_amd.core import hip_backend as hb
+
+    k = complex(2.0, 0.5) if op == "helmholtz_double_layer" else complex(2.5, 0.0)
+    for level, n_points, seed in [(4, 1100, 1), (3, 3400, 2)]:
+        assert _mixed_pairs(level, n_points) > 3 << 23
+        space = bempp.function_space(bempp.shapes.icosphere(level), kind, degree)
+        ref, out = _evaluate_both(op, space, k, hb.PRECISION_MIXED, n_points, seed)
+        assert np.all(np.isfinite(ref))
+        np.testing.assert_array_equal(out, ref)
+
+
 def test_noalloc_rejects_oversize_request():
     """A potential whose workspace exceeds the scratch buffer is refused before any device work."""
     import bempp_amd.api as bempp
