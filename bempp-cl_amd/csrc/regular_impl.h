@@ -1408,10 +1408,12 @@ __global__ __launch_bounds__(kRegThreads, (regular_waves<OP, MIXED, DUAL, SYM, K
             // Only LDS reads and global atomics: nothing waits for the atomics, which complete while
             // the next tile is computed. Device-scope atomics are executed behind the L2, one request
             // per 64-byte line and instruction, so the real and the imaginary part of an entry take
-            // neighbouring lanes and leave in one request. Bound by the rate of those requests (about
-            // 20 G/s) where a block's dofs are scattered over a row: 20,480 triangles with vertices
+            // neighbouring lanes and leave in one request. One request per part (about 20 G/s) had bound
+            // the pass where a block's dofs are scattered over a row: 20,480 triangles with vertices
             // numbered along x, single + double layer, mixed: 676 M -> 340 M requests, the step
-            // 35.4 -> 19.8 ms; numbered at random 50.5 -> 26.7 ms, along the elements 18.3 -> 18.6 ms.
+            // 35.4 -> 19.6 ms; numbered at random 50.5 -> 26.3 ms. Along the elements (130 M requests now)
+            // the step takes 18.2 ms (18.3 before): there as along x the vector unit is the bound, 9.0 G
+            // wave instructions, 14.6 ms at four cycles each on 1,024 SIMDs.
             auto add = [&](OutT *p, AccT v) {
                 if (v != (AccT)0) unsafeAtomicAdd(p, (OutT)v);
             };
