@@ -1169,7 +1169,29 @@ def main():
         result["cpu_baseline"] = cpu_baseline(grid, space, k, entries_per_step, args.cpu_seconds)
         log(f"cpu baseline {result['cpu_baseline']}")
     result["configs"] = config_summary(result)
-    print(json.dumps(result), flush=True)
+    # the whole record (20 KB) goes to stderr, the line of results to stdout
+    log("record " + json.dumps(result))
+    print(json.dumps(result_line(result)), flush=True)
+
+
+def result_line(result):
+    """The benchmark's line: the timed step, its errors and roofline, and a few figures per configuration."""
+
+    def brief(v):
+        if isinstance(v, dict):
+            if "frac" in v:  # a roofline record
+                return {k: v[k] for k in ("bound", "achieved", "peak", "unit", "frac", "traffic") if k in v}
+            if "kind" in v:  # a CPU baseline
+                return {k: v[k] for k in ("value", "unit", "cores", "kind") if k in v}
+            return {k: brief(x) for k, x in v.items()}
+        return v
+
+    keep = {k: v for k, v in result.items() if not isinstance(v, (dict, list))}
+    for k in ("config", "rel_err_vs_fp64", "roofline", "cpu_baseline", "configs"):
+        if k in result:
+            keep[k] = brief(result[k])
+    keep.get("configs", {}).pop("C2", None)  # the top level
+    return keep
 
 
 def config_summary(result):
