@@ -66,20 +66,23 @@ struct PotArgs {
     double *partial;  // [nchunk][kdim][npts][2]
     int nchunk, chunk_len;
     void *out;
-    EfieSeries ser;  // series of e^{i Re(k) delta} - 1 (EFIE potential)
+    EfieSeries ser;  // series of e^{i Re(k) delta} - 1 (mixed potentials)
+    bool groups;     // the prep kernel also forms the mixed scalar kernel's group data
 };
 
+// Mixed kernels: a (target, tile or group) pair whose reference distance r0 is below
+// kNearTileFactor times the radius R of the tile's sources around the reference takes the FP64
+// path: the FP32 offsets lose relative accuracy once the target comes within a fraction of R of
+// the sources (targets just off the surface), while targets beyond r0 >= 1.5 R stay within 1e-6
+// of FP64 (measured for the single, double layer and EFIE potentials on icosphere levels 2 and 4). Scalar
+// potentials: see potential_eval_mixed_scalar.
+constexpr double kNearTileFactor = 1.5;
+
+// Record of the source s.
 template <int OP>
-__global__ __launch_bounds__(256) void potential_prep_kernel(const PotArgs a) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= a.nsrc_pad) return;
+__device__ __forceinline__ void prepare_source(const PotArgs &a, int s) {
     double *src = a.src;
     const int P = a.nsrc_pad;
-    if (s >= a.nsrc) {  // padding sources contribute nothing
-        for (int k = 0; k < kSrcFields; ++k) src[k * P + s] = 0.0;
-        src[0 * P + s] = 1e30;  // far away: G ~ 0 and no division by zero
-        return;
-    }
     const int nq = a.rule.n;
     int ei = s / nq, q = s % nq;
     int e = a.sp.elements[ei];
@@ -128,6 +131,95 @@ __global__ __launch_bounds__(256) void potential_prep_kernel(const PotArgs a) {
         }
         src[6 * P + s] = cr;
         src[7 * P + s] = ci;
+    }
+}
+
+// Data of the mixed scalar kernel's groups and tiles, in the fields 8 and 9 that scalar sources leave free (field 8
+// from a group's first source on: the FP64 group sums over 4 pi, c n (6 values), c u.n (2), c (2), the radius
+// max |u| and (kNearTileFactor max |u|)^2; field 9 at a tile's first source: max |c_tile - y|^2). Once per source
+// here instead of once per 256 targets there, where the sums' shuffles took a tenth of the double layer (Laplace,
+// 20,480 triangles, 16,384 points: 1,255 -> 1,127 us).
+constexpr int kGroupSize = 32, kGroupField = 8, kTileField = 9, kGroupRadius = 10, kGroupNear2 = 11;
+
+__device__ __forceinline__ void prepare_groups(const PotArgs &a, int s) {
+    __shared__ double centre[3];
+    __shared__ float radius2[kPotThreads / 64];
+    const int P = a.nsrc_pad, j = threadIdx.x, gb = s - j % kGroupSize, tb = s - j;
+    const bool ok = s < a.nsrc;
+    double y[3], n[3] = {0.0, 0.0, 0.0}, w[10], cr = 0.0, ci = 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) y[d] = ok ? a.src[(int64_t)d * P + s] : 0.0;
+    if (ok) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) n[d] = a.src[(int64_t)(3 + d) * P + s];
+        cr = kInv4Pi * a.src[6 * (int64_t)P + s];
+        ci = kInv4Pi * a.src[7 * (int64_t)P + s];
+    }
+    // the middle source of the group (the last one of a short group), as in the kernel that uses the sums
+    const int mid = max(0, min(kGroupSize / 2, a.nsrc - 1 - gb));
+    double uu = 0.0, un = 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const double u = __shfl(y[d], mid, kGroupSize) - y[d];
+        uu += u * u;
+        un += u * n[d];
+        w[2 * d] = cr * n[d];
+        w[2 * d + 1] = ci * n[d];
+    }
+    w[6] = cr * un;
+    w[7] = ci * un;
+    w[8] = cr;
+    w[9] = ci;
+    if (!ok) uu = 0.0;
+#pragma unroll
+    for (int off = kGroupSize / 2; off >= 1; off >>= 1) {
+#pragma unroll
+        for (int k = 0; k < 10; ++k) w[k] += __shfl_xor(w[k], off, 64);
+        uu = fmax(uu, __shfl_xor(uu, off, 64));
+    }
+    double *out = a.src + (int64_t)kGroupField * P + gb;
+    if (s == gb) {
+#pragma unroll
+        for (int k = 0; k < 10; ++k) out[k] = w[k];
+        out[kGroupRadius] = sqrt(uu) * (1.0 + 1e-6);
+        out[kGroupNear2] = kNearTileFactor * kNearTileFactor * (1.0 + 1e-6) * uu;
+    }
+    // the tile's radius about its middle source
+    if (s == tb + max(0, min(kPotTile / 2, a.nsrc - 1 - tb))) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) centre[d] = y[d];
+    }
+    __syncthreads();
+    float t2 = 0.f;
+    if (ok) {
+        const double u0 = centre[0] - y[0], u1 = centre[1] - y[1], u2 = centre[2] - y[2];
+        t2 = (float)(u0 * u0 + u1 * u1 + u2 * u2);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) t2 = fmaxf(t2, __shfl_xor(t2, off, 64));
+    if ((j & 63) == 0) radius2[j >> 6] = t2;
+    __syncthreads();
+    if (j == 0) {
+#pragma unroll
+        for (int v = 1; v < kPotThreads / 64; ++v) t2 = fmaxf(t2, radius2[v]);
+        a.src[(int64_t)kTileField * P + tb] = t2;
+    }
+}
+
+template <int OP>
+__global__ __launch_bounds__(256) void potential_prep_kernel(const PotArgs a) {
+    // one workgroup per tile, its lanes in whole groups
+    const int s = blockIdx.x * kPotTile + threadIdx.x;
+    double *src = a.src;
+    const int P = a.nsrc_pad;
+    if (s >= a.nsrc) {  // padding sources contribute nothing
+        for (int k = 0; k < (OP == kMaxwellEFIE ? kSrcFields : kGroupField); ++k) src[k * P + s] = 0.0;
+        src[0 * P + s] = 1e30;  // far away: G ~ 0 and no division by zero
+    } else {
+        prepare_source<OP>(a, s);
+    }
+    if constexpr (OP != kMaxwellEFIE) {
+        if (a.groups) prepare_groups(a, s);
     }
 }
 
@@ -213,14 +305,6 @@ __device__ __forceinline__ void fp64_magnetic_source(F field, double x0, double 
     accr[2] += d0 * wr[1] - d1 * wr[0];
     acci[2] += d0 * wi[1] - d1 * wi[0];
 }
-
-// Mixed kernels: a (target, tile or group) pair whose reference distance r0 is below
-// kNearTileFactor times the radius R of the tile's sources around the reference takes the FP64
-// path: the FP32 offsets lose relative accuracy once the target comes within a fraction of R of
-// the sources (targets just off the surface), while targets beyond r0 >= 1.5 R stay within 1e-6
-// of FP64 (measured for the single, double layer and EFIE potentials on icosphere levels 2 and 4). Scalar
-// potentials: see potential_eval_mixed_scalar.
-constexpr double kNearTileFactor = 1.5;
 
 // The FP64 path of the mixed kernels for the sources [s_begin, s_end) of the workspace.
 template <int OP, int KD, int PH = 0>
@@ -590,13 +674,29 @@ __device__ __forceinline__ void scalar_em1(float delta, float kr, float kr_rev, 
     }
 }
 
+// e^{iy} - 1 of |y| <= 1 from the Taylor series through y^10 and y^9 (remainders 2e-9 and 3e-8)
+__device__ __forceinline__ void small_em1(float y, float &em1r, float &em1i) {
+    const float y2 = y * y;
+    float p = fmaf(y2, -1.f / 3628800.f, 1.f / 40320.f);
+    p = fmaf(y2, p, -1.f / 720.f);
+    p = fmaf(y2, p, 1.f / 24.f);
+    p = fmaf(y2, p, -0.5f);
+    em1r = y2 * p;
+    float q = fmaf(y2, 1.f / 362880.f, -1.f / 5040.f);
+    q = fmaf(y2, q, 1.f / 120.f);
+    q = fmaf(y2, q, -1.f / 6.f);
+    em1i = fmaf(y * y2, q, y);
+}
+
 // MIXED scalar potentials (Laplace and Helmholtz single and double layer), per (target, group of 32
 // neighbouring sources). With c the group's middle source, v = x - c, u = c - y (so x - y = v + u), r0 = |v|,
 // t = r^2 - r0^2 = 2 v.u + |u|^2, delta = r - r0 = t / (r + r0) and E = e^{ik delta}, the FP64 part forms r0 and
 // e^{ik r0}; the sources, staged per tile of 256 as FP32 records and read as LDS broadcasts, take one of three
 // paths, chosen per wave by the distance of its targets:
 //  * away from the whole tile (kNearTileFactor times its radius): E / r itself, with the hardware rsq, rcp, sin
-//    and cos, 17.5 instructions (single layer), error about 1e-7 of each term;
+//    and cos, 17.5 instructions (single layer), error about 1e-7 of each term; e^{ik r0} relative to the tile's
+//    middle source, where |k| times the tile's radius is at most 1 from an FP32 series, so that FP64 sines are
+//    taken once per tile;
 //  * closer to the tile, away from the group: the sums split into a group-centre term from FP64 group sums and
 //    a remainder of small differences in FP32 (as potential_eval_mixed_efie),
 //      single layer  sum_j c_j G        = e^{ik r0} / 4 pi [ sum_j c_j / r0 + sum_j f c_j ],  f = (E - 1) / r - q,
@@ -612,36 +712,35 @@ __device__ __forceinline__ void scalar_em1(float delta, float kr, float kr_rev, 
 // 15,680 triangles, up to the wavenumber of 8 elements a wavelength, against FP64: 2.5e-8 to 3.1e-8 where all
 // tiles are close (720 triangles; one reference per tile with FP64 near it 2.5e-8, E / r for all groups away from
 // 1.5 times their own radius 6e-8 to 1.1e-7), up to 1.5e-7 on large meshes (2.3e-7, 1.7e-7).
-// 20,480 triangles in rows, 16,384 points (whole call): 1.56 ms single layer (one reference per tile 7.5, E / r
-// for all groups 1.62), 2.2 ms double layer (9.1, 2.3). 15,680 triangles, 20,000 points, Helmholtz single layer,
-// kernel: points 10 to 20 from the centre 1.19 ms (1.01, 1.13), 1.02 to 1.3 2.6 ms (10.5, 3.4).
+// 20,480 triangles in rows, 16,384 points (whole call): 1.53 ms single layer (one reference per tile 7.5, E / r
+// for all groups 1.62), 2.1 ms double layer (9.1, 2.3). 15,680 triangles, 20,000 points, Helmholtz single layer,
+// kernel: points 10 to 20 from the centre 1.15 ms (1.01, 1.13), 1.02 to 1.3 2.4 ms (10.5, 3.4). 20,480 triangles
+// in compact order, 16,384 points at radius 2: 1.14 ms, error 1.3e-7 (1.02, 3.2e-7; 1.16, 1.2e-7).
 // DAMP: complex wavenumber, E = e^{-Im(k) delta} e^{i Re(k) delta}.
 template <int OP, bool DAMP>
 __global__ __launch_bounds__(kPotThreads, 4) void potential_eval_mixed_scalar(const PotArgs a) {
-    constexpr int GS = 32;
+    constexpr int GS = kGroupSize;
     constexpr int NG = kPotTile / GS;
     constexpr bool HELM = OP == kHelmholtzSL || OP == kHelmholtzDL;
     constexpr bool DL = OP == kLaplaceDL || OP == kHelmholtzDL;
     constexpr double kNearScalar = DL ? 2.5 : 1.5, kNearScalarPhase = 1.5;
-    constexpr int NW = DL ? 8 : 2;  // FP64 group sums: c (single layer); c n and c u.n (double layer), over 4 pi
+    // FP64 group sums (prepare_groups): c (single layer); c n and c u.n (double layer)
+    constexpr int NW = DL ? 8 : 2, kFirstSum = DL ? 0 : 8;
     static_assert(!DAMP || HELM, "only Helmholtz wavenumbers are complex");
-    __shared__ float4 shu[kPotTile];           // u, |u|^2
+    __shared__ float4 shu[kPotTile];           // 2 u, |u|^2
     __shared__ float4 shw[kPotTile];           // Re c / 4 pi, Im c / 4 pi, u.n_y, -
     __shared__ float4 shn[DL ? kPotTile : 1];  // n_y, -
     __shared__ double sc[NG][3];
     __shared__ double wsum[NG][NW];
     __shared__ float srad[NG];  // max |u| of the group's sources (bounds |delta|)
-    __shared__ float trad2[kPotThreads / 64];  // per wave: max |c_tile - y|^2 of the whole tile's sources
+    __shared__ double snear2[NG];              // (kNearTileFactor max |u|)^2
     const int m = blockIdx.x * kPotThreads + threadIdx.x;
     const int chunk = blockIdx.y;
     const int s0 = chunk * a.chunk_len;
     const int s1 = min(s0 + a.chunk_len, a.nsrc);
-    double x0 = 0, x1 = 0, x2 = 0;
-    if (m < a.npts) {
-        x0 = a.pts[3 * (int64_t)m];
-        x1 = a.pts[3 * (int64_t)m + 1];
-        x2 = a.pts[3 * (int64_t)m + 2];
-    }
+    // lanes beyond the targets repeat the last one
+    const double *x = a.pts + 3 * (int64_t)min(m, a.npts - 1);
+    const double x0 = x[0], x1 = x[1], x2 = x[2];
     double accr = 0.0, acci = 0.0;
     const float kr_f = (float)a.kr, ki_f = (float)a.ki;
     const float kr_rev = (float)(a.kr * 0.15915494309189533577);
@@ -649,80 +748,172 @@ __global__ __launch_bounds__(kPotThreads, 4) void potential_eval_mixed_scalar(co
     const float ki_log2e = (float)(a.ki * 1.4426950408889634), kmax = fmaxf(kabs, fabsf(ki_f));
     const EfieSeries &ser = a.ser;
     const int P = a.nsrc_pad;
+    // adds e^{ik r} (e^{-Im(k) r}) (cr + i ci)
+    auto add = [&](double cr, double ci, double r) {
+        if constexpr (HELM) {
+            double sn, cs;
+            sincos_fast(a.kr * r, &sn, &cs);
+            if constexpr (DAMP) {
+                const double damp = exp(-a.ki * r);
+                sn *= damp;
+                cs *= damp;
+            }
+            accr += cs * cr - sn * ci;
+            acci += cs * ci + sn * cr;
+        } else {
+            accr += cr;
+            acci += ci;
+        }
+    };
     for (int t0 = s0; t0 < s1; t0 += kPotTile) {
         const int nt = min(kPotTile, s1 - t0);
+        // targets close to a group's sources: the group in FP64 for the whole wave
+        auto near = [&](int j0, int j1, double r0sq, float rad) {
+            // every phase is at most |Re k| (r0 + R)
+            if (HELM && __all(fabs(a.kr) * (sqrt(r0sq) + (double)rad) < 0x1p25))
+                sources_fp64_near<OP, 1, kPhReduced | (DAMP ? 0 : kPhReal)>(a, t0 + j0, t0 + j1, x0, x1, x2, 0.0, 0.0, &accr,
+                                                                           &acci);
+            else
+                sources_fp64_near<OP, 1>(a, t0 + j0, t0 + j1, x0, x1, x2, 0.0, 0.0, &accr, &acci);
+        };
         // the whole tile that the staged sources are from (a chunk may be a part of one) and its middle source
-        const int tb = t0 - t0 % kPotTile, tn = min(kPotTile, a.nsrc - tb), tc = tb + min(kPotTile / 2, tn - 1);
+        const int tb = t0 - t0 % kPotTile, tc = min(tb + kPotTile / 2, a.nsrc - 1);
         const double tc0 = a.src[tc], tc1 = a.src[(int64_t)P + tc], tc2 = a.src[2 * (int64_t)P + tc];
         __syncthreads();
         {
             const int j = threadIdx.x, g = j / GS, s = t0 + j;
-            float t2 = 0.f;
-            if (j < tn) {
-                const double u0 = tc0 - a.src[tb + j], u1 = tc1 - a.src[(int64_t)P + tb + j], u2 = tc2 - a.src[2 * (int64_t)P + tb + j];
-                t2 = (float)(u0 * u0 + u1 * u1 + u2 * u2);
-            }
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) t2 = fmaxf(t2, __shfl_xor(t2, off, 64));
-            if ((j & 63) == 0) trad2[j >> 6] = t2;
+            if (j < NG * NW && t0 + j / NW * GS < s1)
+                wsum[j / NW][j % NW] = a.src[(int64_t)kGroupField * P + t0 + j / NW * GS + kFirstSum + j % NW];
             const int cidx = t0 + min(g * GS + GS / 2, nt - 1);
             double c[3];
             for (int d = 0; d < 3; ++d) c[d] = a.src[(int64_t)d * P + cidx];
-            if (j % GS == 0)
+            if (j % GS == 0 && s < s1) {
                 for (int d = 0; d < 3; ++d) sc[g][d] = c[d];
+                srad[g] = (float)a.src[(int64_t)kGroupField * P + s + kGroupRadius];
+                snear2[g] = a.src[(int64_t)kGroupField * P + s + kGroupNear2];
+            }
             float4 U = make_float4(0.f, 0.f, 0.f, 0.f), W = make_float4(0.f, 0.f, 0.f, 0.f);
             float4 N = make_float4(0.f, 0.f, 0.f, 0.f);
-            double uu = 0.0, w[NW];
-#pragma unroll
-            for (int k = 0; k < NW; ++k) w[k] = 0.0;
             if (j < nt) {
                 const double u0 = c[0] - a.src[s], u1 = c[1] - a.src[(int64_t)P + s], u2 = c[2] - a.src[2 * (int64_t)P + s];
-                uu = u0 * u0 + u1 * u1 + u2 * u2;
-                U = make_float4((float)u0, (float)u1, (float)u2, (float)uu);
-                const double cr = kInv4Pi * a.src[6 * (int64_t)P + s], ci = kInv4Pi * a.src[7 * (int64_t)P + s];
-                W.x = (float)cr;
-                W.y = (float)ci;
+                U = make_float4((float)(2.0 * u0), (float)(2.0 * u1), (float)(2.0 * u2), (float)(u0 * u0 + u1 * u1 + u2 * u2));
+                W.x = (float)(kInv4Pi * a.src[6 * (int64_t)P + s]);
+                W.y = (float)(kInv4Pi * a.src[7 * (int64_t)P + s]);
                 if constexpr (DL) {
-                    const double n[3] = {a.src[3 * (int64_t)P + s], a.src[4 * (int64_t)P + s], a.src[5 * (int64_t)P + s]};
-                    const double un = u0 * n[0] + u1 * n[1] + u2 * n[2];
-                    N = make_float4((float)n[0], (float)n[1], (float)n[2], 0.f);
-                    W.z = (float)un;
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) {
-                        w[2 * d] = cr * n[d];
-                        w[2 * d + 1] = ci * n[d];
-                    }
-                    w[6] = cr * un;
-                    w[7] = ci * un;
-                } else {
-                    w[0] = cr;
-                    w[1] = ci;
+                    const double n0 = a.src[3 * (int64_t)P + s], n1 = a.src[4 * (int64_t)P + s],
+                                 n2 = a.src[5 * (int64_t)P + s];
+                    N = make_float4((float)n0, (float)n1, (float)n2, 0.f);
+                    W.z = (float)(u0 * n0 + u1 * n1 + u2 * n2);
                 }
             }
             shu[j] = U;
             shw[j] = W;
             if constexpr (DL) shn[j] = N;
-#pragma unroll
-            for (int k = 0; k < NW; ++k) {
-#pragma unroll
-                for (int off = GS / 2; off >= 1; off >>= 1) w[k] += __shfl_xor(w[k], off, 64);
-            }
-#pragma unroll
-            for (int off = GS / 2; off >= 1; off >>= 1) uu = fmax(uu, __shfl_xor(uu, off, 64));
-            if (j % GS == 0) {
-#pragma unroll
-                for (int k = 0; k < NW; ++k) wsum[g][k] = w[k];
-                srad[g] = (float)(sqrt(uu) * (1.0 + 1e-6));
-            }
         }
         __syncthreads();
         // wave-uniform: every target is away from the tile
-        float R2 = trad2[0];
-#pragma unroll
-        for (int w = 1; w < kPotThreads / 64; ++w) R2 = fmaxf(R2, trad2[w]);
-        const double q0 = x0 - tc0, q1 = x1 - tc1, q2 = x2 - tc2;
-        const bool far = !__any(m < a.npts && q0 * q0 + q1 * q1 + q2 * q2 <
-                                                  kNearTileFactor * kNearTileFactor * (double)R2 * (1.0 + 1e-6));
+        const float R2 = (float)a.src[(int64_t)kTileField * P + tb];
+        const double q0 = x0 - tc0, q1 = x1 - tc1, q2 = x2 - tc2, rT2 = q0 * q0 + q1 * q1 + q2 * q2;
+        const bool far = !__any(rT2 < kNearTileFactor * kNearTileFactor * (double)R2 * (1.0 + 1e-6));
+        if (far) {
+            // e^{ik rT} of the tile's reference once; |r0 - rT| is at most the tile's radius
+            const double rT = rT2 * rsqrt_t(rT2);
+            const bool small = HELM && kmax * sqrtf(R2) <= 0.999f;
+            double tr = 0.0, ti = 0.0;
+            for (int g = 0; g < NG && g * GS < nt; ++g) {
+                const int j0 = g * GS, j1 = min(j0 + GS, nt);
+                const double v0d = x0 - sc[g][0], v1d = x1 - sc[g][1], v2d = x2 - sc[g][2];
+                const double r0sq_d = v0d * v0d + v1d * v1d + v2d * v2d;
+                if (__any(r0sq_d < snear2[g])) {
+                    near(j0, j1, r0sq_d, srad[g]);
+                    continue;
+                }
+                const double r0d = r0sq_d * rsqrt_t(r0sq_d);
+                const float v0 = (float)v0d, v1 = (float)v1d, v2 = (float)v2d;
+                const float r0sq = (float)r0sq_d, r0 = (float)r0d;
+                float Ar = 0.f, Ai = 0.f;
+                const float r0k = r0 * kinv;
+#pragma unroll 4
+                for (int j = j0; j < j1; ++j) {
+                    const float4 U = shu[j];
+                    const float4 W = shw[j];
+                    const float tt = fmaf(v0, U.x, fmaf(v1, U.y, fmaf(v2, U.z, U.w)));
+                    const float r2 = r0sq + tt;
+                    const float rinv = rsqrt_t(r2);
+                    float er = rinv, ei = 0.f;  // e^{ik(r - r0)} / r (Laplace: 1 / r)
+                    float r = 0.f;
+                    if constexpr (HELM) {
+                        r = r2 * rinv;
+                        float ph, amp = rinv;
+                        if constexpr (DAMP) {
+                            const float delta = tt * __builtin_amdgcn_rcpf(r + r0);
+                            ph = kr_rev * delta;
+                            amp *= __builtin_amdgcn_exp2f(-ki_log2e * delta);
+                        } else {
+                            ph = tt * __builtin_amdgcn_rcpf(r * kinv + r0k);
+                        }
+                        const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
+                        if constexpr (!DL) {
+                            // the weight times e^{ik(r - r0)} first, then one FMA by the amplitude
+                            Ar += amp * (cs * W.x - sn * W.y);
+                            Ai += amp * (cs * W.y + sn * W.x);
+                            continue;
+                        }
+                        er = cs * amp;
+                        ei = sn * amp;
+                    }
+                    if constexpr (DL) {
+                        // (1 - i k r) (x - y).n_y / r^2
+                        const float4 N = shn[j];
+                        const float f = (v0 * N.x + (v1 * N.y + (v2 * N.z + W.z))) * rinv * rinv;
+                        if constexpr (HELM) {
+                            const float ar = DAMP ? 1.f + ki_f * r : 1.f, ai = -kr_f * r;
+                            const float pr = (ar * er - ai * ei) * f, pi = (ar * ei + ai * er) * f;
+                            er = pr;
+                            ei = pi;
+                        } else {
+                            er *= f;
+                        }
+                    }
+                    Ar += er * W.x;
+                    Ai += er * W.y;
+                    if constexpr (HELM) {
+                        Ar -= ei * W.y;
+                        Ai += ei * W.x;
+                    }
+                }
+                if constexpr (HELM) {
+                    const double d0 = r0d - rT;
+                    if (small) {
+                        float er, ei;
+                        small_em1((float)(a.kr * d0), er, ei);
+                        float br = fmaf(er, Ar, fmaf(-ei, Ai, Ar)), bi = fmaf(er, Ai, fmaf(ei, Ar, Ai));
+                        if constexpr (DAMP) {
+                            const float damp = (float)exp_small(-a.ki * d0);
+                            br *= damp;
+                            bi *= damp;
+                        }
+                        tr += br;
+                        ti += bi;
+                    } else {
+                        double sn, cs;
+                        sincos_fast(a.kr * d0, &sn, &cs);
+                        if constexpr (DAMP) {
+                            const double damp = exp(-a.ki * d0);
+                            sn *= damp;
+                            cs *= damp;
+                        }
+                        tr += cs * Ar - sn * Ai;
+                        ti += cs * Ai + sn * Ar;
+                    }
+                } else {
+                    tr += Ar;
+                    ti += Ai;
+                }
+            }
+            add(tr, ti, rT);
+            continue;
+        }
         for (int g = 0; g < NG && g * GS < nt; ++g) {
             const int j0 = g * GS, j1 = min(j0 + GS, nt);
             // |Re(k) delta| <= |Re(k)| max |u| (wave-uniform)
@@ -730,20 +921,12 @@ __global__ __launch_bounds__(kPotThreads, 4) void potential_eval_mixed_scalar(co
             // per (target, group): FP64 reference distance and phase
             const double v0d = x0 - sc[g][0], v1d = x1 - sc[g][1], v2d = x2 - sc[g][2];
             const double r0sq_d = v0d * v0d + v1d * v1d + v2d * v2d;
-            // targets close to the group's sources: the group in FP64 for the whole wave
-            const double rn = (far ? kNearTileFactor : kNearScalar + kNearScalarPhase * (double)(kmax * srad[g])) * (double)srad[g];
-            if (__any(m < a.npts && r0sq_d < rn * rn)) {
-                // every phase is at most |Re k| (r0 + R)
-                const bool reduced = HELM && __all(fabs(a.kr) * (sqrt(r0sq_d) + (double)srad[g]) < 0x1p25);
-                if (reduced)
-                    sources_fp64_near<OP, 1, kPhReduced | (DAMP ? 0 : kPhReal)>(a, t0 + j0, t0 + j1, x0, x1, x2, 0.0, 0.0,
-                                                                               &accr, &acci);
-                else
-                    sources_fp64_near<OP, 1>(a, t0 + j0, t0 + j1, x0, x1, x2, 0.0, 0.0, &accr, &acci);
+            const double rn = (kNearScalar + kNearScalarPhase * (double)(kmax * srad[g])) * (double)srad[g];
+            if (__any(r0sq_d < rn * rn)) {
+                near(j0, j1, r0sq_d, srad[g]);
                 continue;
             }
             const double i0 = rsqrt_t(r0sq_d), i2 = i0 * i0, r0d = r0sq_d * i0;
-            const float tv0 = (float)(2.0 * v0d), tv1 = (float)(2.0 * v1d), tv2 = (float)(2.0 * v2d);
             const float v0 = (float)v0d, v1 = (float)v1d, v2 = (float)v2d;
             const float r0sq = (float)r0sq_d, r0 = (float)r0d, r0inv = (float)i0, r0inv2 = (float)i2;
             // h(r0) (double layer)
@@ -756,7 +939,7 @@ __global__ __launch_bounds__(kPotThreads, 4) void potential_eval_mixed_scalar(co
                 for (int j = j0; j < j1; ++j) {
                     const float4 U = shu[j];
                     const float4 W = shw[j];
-                    const float tt = fmaf(tv0, U.x, fmaf(tv1, U.y, fmaf(tv2, U.z, U.w)));  // r^2 - r0^2
+                    const float tt = fmaf(v0, U.x, fmaf(v1, U.y, fmaf(v2, U.z, U.w)));  // r^2 - r0^2
                     const float r2 = r0sq + tt;
                     const float rinv = rsqrt_t(r2);
                     const float delta = tt * __builtin_amdgcn_rcpf(fmaf(r2, rinv, r0));
@@ -813,59 +996,7 @@ __global__ __launch_bounds__(kPotThreads, 4) void potential_eval_mixed_scalar(co
             constexpr std::false_type series{};
             // the folded series need k^10 / 10! in FP32 range (|k| < 1000)
             const bool folded = kabs < 1000.f;
-            if (far) {
-                // the amplitude e^{ik delta} / r itself
-                const float r0k = r0 * kinv;
-#pragma unroll 4
-                for (int j = j0; j < j1; ++j) {
-                    const float4 U = shu[j];
-                    const float4 W = shw[j];
-                    const float tt = fmaf(tv0, U.x, fmaf(tv1, U.y, fmaf(tv2, U.z, U.w)));
-                    const float r2 = r0sq + tt;
-                    const float rinv = rsqrt_t(r2);
-                    float er = rinv, ei = 0.f;  // e^{ik(r - r0)} / r (Laplace: 1 / r)
-                    float r = 0.f;
-                    if constexpr (HELM) {
-                        r = r2 * rinv;
-                        float ph, amp = rinv;
-                        if constexpr (DAMP) {
-                            const float delta = tt * __builtin_amdgcn_rcpf(r + r0);
-                            ph = kr_rev * delta;
-                            amp *= __builtin_amdgcn_exp2f(-ki_log2e * delta);
-                        } else {
-                            ph = tt * __builtin_amdgcn_rcpf(r * kinv + r0k);
-                        }
-                        const float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
-                        if constexpr (!DL) {
-                            // the weight times e^{ik(r - r0)} first, then one FMA by the amplitude
-                            Ar += amp * (cs * W.x - sn * W.y);
-                            Ai += amp * (cs * W.y + sn * W.x);
-                            continue;
-                        }
-                        er = cs * amp;
-                        ei = sn * amp;
-                    }
-                    if constexpr (DL) {
-                        // (1 - i k r) (x - y).n_y / r^2
-                        const float4 N = shn[j];
-                        const float f = (v0 * N.x + (v1 * N.y + (v2 * N.z + W.z))) * rinv * rinv;
-                        if constexpr (HELM) {
-                            const float ar = DAMP ? 1.f + ki_f * r : 1.f, ai = -kr_f * r;
-                            const float pr = (ar * er - ai * ei) * f, pi = (ar * ei + ai * er) * f;
-                            er = pr;
-                            ei = pi;
-                        } else {
-                            er *= f;
-                        }
-                    }
-                    Ar += er * W.x;
-                    Ai += er * W.y;
-                    if constexpr (HELM) {
-                        Ar -= ei * W.y;
-                        Ai += ei * W.x;
-                    }
-                }
-            } else if constexpr (!HELM) {
+            if constexpr (!HELM) {
                 sources(integral_constant<int, 0>{}, series);
             } else if (DAMP && fabsf(ki_f) * srad[g] > 0.24f) {
                 if (ymax <= 1.96f)
@@ -883,30 +1014,18 @@ __global__ __launch_bounds__(kPotThreads, 4) void potential_eval_mixed_scalar(co
             } else {
                 sources(integral_constant<int, 4>{}, series);
             }
-            // the group-centre term, plus the remainder, times e^{i k r0} (e^{-Im(k) r0}) in FP64
+            // the group-centre term, plus the remainder
             double cr = Ar, ci = Ai;
-            if (!far) {
-                if constexpr (DL) {
-                    const double nr = v0d * wsum[g][0] + v1d * wsum[g][2] + v2d * wsum[g][4] + wsum[g][6];
-                    const double ni = v0d * wsum[g][1] + v1d * wsum[g][3] + v2d * wsum[g][5] + wsum[g][7];
-                    cr += h0rd * nr - (HELM ? h0id * ni : 0.0);
-                    ci += h0rd * ni + (HELM ? h0id * nr : 0.0);
-                } else {
-                    cr += i0 * wsum[g][0];
-                    ci += i0 * wsum[g][1];
-                }
-            }
-            if constexpr (HELM) {
-                double sn, cs;
-                sincos_fast(a.kr * r0d, &sn, &cs);
-                const double damp0 = DAMP ? exp(-a.ki * r0d) : 1.0;
-                const double pr = cs * damp0, pi = sn * damp0;
-                accr += pr * cr - pi * ci;
-                acci += pr * ci + pi * cr;
+            if constexpr (DL) {
+                const double nr = v0d * wsum[g][0] + v1d * wsum[g][2] + v2d * wsum[g][4] + wsum[g][6];
+                const double ni = v0d * wsum[g][1] + v1d * wsum[g][3] + v2d * wsum[g][5] + wsum[g][7];
+                cr += h0rd * nr - (HELM ? h0id * ni : 0.0);
+                ci += h0rd * ni + (HELM ? h0id * nr : 0.0);
             } else {
-                accr += cr;
-                acci += ci;
+                cr += i0 * wsum[g][0];
+                ci += i0 * wsum[g][1];
             }
+            add(cr, ci, r0d);
         }
     }
     if (m < a.npts) {
@@ -1353,7 +1472,7 @@ static int run_potential(PotArgs &a, int precision, int out_dtype, hipStream_t s
     int rc;
     // an empty space has no sources: only the reduction runs (it writes zeros)
     if (a.nsrc > 0) {
-        hipLaunchKernelGGL((potential_prep_kernel<OP>), dim3((a.nsrc_pad + 255) / 256), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((potential_prep_kernel<OP>), dim3(a.nsrc_pad / kPotTile), dim3(kPotTile), 0, s, a);
         if ((rc = check_launch("potential_prep_kernel"))) return rc;
         dim3 grid((a.npts + kPotThreads - 1) / kPotThreads, a.nchunk);
         if constexpr (FF >= 0) {
@@ -1475,6 +1594,7 @@ static int potential_evaluate(int op, const bem_space_t *space, const void *coef
     a.partial = a.src + (size_t)kSrcFields * a.nsrc_pad;
     a.out = out;
     a.ser = efie_series(a.kr);
+    a.groups = precision == BEM_PRECISION_MIXED && !is_vector_potential_op(op) && !is_far_field_op(op);
     switch (op) {
     case BEM_LAPLACE_SINGLE_LAYER: return run_potential<kLaplaceSL>(a, precision, out_dtype, s);
     case BEM_LAPLACE_DOUBLE_LAYER: return run_potential<kLaplaceDL>(a, precision, out_dtype, s);
