@@ -1175,22 +1175,30 @@ def main():
 
 
 def result_line(result):
-    """The benchmark's line: the timed step, its errors and roofline, and a few figures per configuration."""
+    """The benchmark's line, less than 2,000 characters: the timed step, its errors and roofline, and per
+    configuration its rate, error and roofline fraction."""
 
-    def brief(v):
-        if isinstance(v, dict):
-            if "frac" in v:  # a roofline record
-                return {k: v[k] for k in ("bound", "achieved", "peak", "unit", "frac", "traffic") if k in v}
-            if "kind" in v:  # a CPU baseline
-                return {k: v[k] for k in ("value", "unit", "cores", "kind") if k in v}
-            return {k: brief(x) for k, x in v.items()}
-        return v
+    def short(v):
+        return float(f"{v:.4g}") if isinstance(v, float) else v
 
-    keep = {k: v for k, v in result.items() if not isinstance(v, (dict, list))}
-    for k in ("config", "rel_err_vs_fp64", "roofline", "cpu_baseline", "configs"):
+    keep = {k: v for k, v in result.items()
+            if not isinstance(v, (dict, list)) and not k.startswith(("fp64_", "speedup_"))}
+    keep["speedup_vs_fp64"] = short(result.get("speedup_vs_fp64"))
+    for k, fields in (("config", ("workload", "triangles", "dofs", "wavenumber")),
+                      ("roofline", ("bound", "achieved", "peak", "unit", "frac", "traffic")),
+                      ("cpu_baseline", ("value", "unit", "cores", "kind")),
+                      ("rel_err_vs_fp64", ("helmholtz_single_layer", "helmholtz_double_layer"))):
         if k in result:
-            keep[k] = brief(result[k])
-    keep.get("configs", {}).pop("C2", None)  # the top level
+            keep[k] = {f: short(result[k][f]) for f in fields if f in result[k]}
+    keep["configs"] = {}
+    for name, c in result.get("configs", {}).items():
+        if name == "C2":  # the line's own value
+            continue
+        brief = {k: short(v) for k, v in c.items() if not isinstance(v, dict)}
+        for k in ("roofline", "roofline_backward"):
+            if k in c:
+                brief[k.replace("roofline", "frac")] = short(c[k]["frac"])
+        keep["configs"][name] = brief
     return keep
 
 
