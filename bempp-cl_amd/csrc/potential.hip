@@ -712,10 +712,14 @@ __device__ __forceinline__ void small_em1(float y, float &em1r, float &em1i) {
 // 15,680 triangles, up to the wavenumber of 8 elements a wavelength, against FP64: 2.5e-8 to 3.1e-8 where all
 // tiles are close (720 triangles; one reference per tile with FP64 near it 2.5e-8, E / r for all groups away from
 // 1.5 times their own radius 6e-8 to 1.1e-7), up to 1.5e-7 on large meshes (2.3e-7, 1.7e-7).
-// 20,480 triangles in rows, 16,384 points (whole call): 1.53 ms single layer (one reference per tile 7.5, E / r
+// 20,480 triangles in rows, 16,384 points (whole call): 1.50 ms single layer (one reference per tile 7.1, E / r
 // for all groups 1.62), 2.1 ms double layer (9.1, 2.3). 15,680 triangles, 20,000 points, Helmholtz single layer,
 // kernel: points 10 to 20 from the centre 1.15 ms (1.01, 1.13), 1.02 to 1.3 2.4 ms (10.5, 3.4). 20,480 triangles
 // in compact order, 16,384 points at radius 2: 1.14 ms, error 1.3e-7 (1.02, 3.2e-7; 1.16, 1.2e-7).
+// Bound by issue (29 instructions per evaluation, 95 % of the kernel's time, in rows). Four waves per SIMD: 128
+// registers and 6 to 45 spilled; Helmholtz single layer in rows / in compact order 1,531 / 1,139 us, at two or
+// three waves (152 to 167 registers) 1,604 / 1,195, at five 1,599 / 1,177; double layer 2,100 / 1,589, at two
+// 2,138 / 1,631, at five 2,226 / 1,615.
 // DAMP: complex wavenumber, E = e^{-Im(k) delta} e^{i Re(k) delta}.
 template <int OP, bool DAMP>
 __global__ __launch_bounds__(kPotThreads, 4) void potential_eval_mixed_scalar(const PotArgs a) {
